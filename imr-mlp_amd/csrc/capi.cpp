@@ -86,8 +86,10 @@ int upload_coeffs(mtpx_context *ctx)
     return MTPX_OK;
 }
 
-// Sizes and work-space offsets of the device view (no device pointers).
-void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm)
+// Sizes and work-space offsets of the device view (no device pointers) and
+// the moment tables of its kernel profile.
+void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm,
+                      std::vector<unsigned short> &mono)
 {
     dm.Z = M.Z;
     dm.M = M.M;
@@ -97,6 +99,7 @@ void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm)
     dm.T = M.T;
     dm.S = M.S;
     dm.nslots = P.nslots;
+    dm.nforce = (int)P.force_basic.size();
     dm.rmin = M.rmin;
     dm.rmax = M.rmax;
     dm.scaling = M.scaling;
@@ -133,6 +136,8 @@ void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm)
     dm.rb_general = M.general_basis() ? 1 : 0;
     dm.rb_table = nullptr;
     std::memcpy(dm.slot_base, P.slot_base, sizeof dm.slot_base);
+    moment_table(M, P, efs_profile_degree(dm), mono, dm.mono_groups);
+    dm.nmono = (int)mono.size();
     dm.fwd_nsteps = (int)(P.fwd_steps.size() / (2 * kWave));
     dm.bwd_nsteps = (int)(P.bwd_steps.size() / (2 * kWave));
 }
@@ -148,7 +153,8 @@ int install_model(mtpx_context *ctx, Model &&m)
     // Sizes first, in a local view: a model whose work space does not fit a
     // CU's LDS is refused before anything of the context changes.
     DevModel dm{};
-    fill_model_sizes(m, p, dm);
+    std::vector<unsigned short> mono;
+    fill_model_sizes(m, p, dm, mono);
     EfsLaunch probe;
     if (!efs_configure(dm, 1, 1, 0, ctx->lds_limit, probe))
         return set_error(ctx, MTPX_E_CAPACITY, "model needs more LDS than a CU provides");
@@ -166,7 +172,8 @@ int install_model(mtpx_context *ctx, Model &&m)
     hipStream_t s = ctx->stream;
     HIP_TRY(upload(ctx->map, M.map, s), "upload model");
     HIP_TRY(upload(ctx->slot_basic, P.slot_basic, s), "upload model");
-    HIP_TRY(upload(ctx->slot_abc, P.slot_abc, s), "upload model");
+    HIP_TRY(upload(ctx->force_basic, P.force_basic, s), "upload model");
+    HIP_TRY(upload(ctx->mono_tab, mono, s), "upload model");
     HIP_TRY(upload(ctx->dup, P.dup, s), "upload model");
     HIP_TRY(upload(ctx->fwd_level, P.fwd_level_step, s), "upload model");
     HIP_TRY(upload(ctx->fwd_steps, P.fwd_steps, s), "upload model");
@@ -216,7 +223,8 @@ int install_model(mtpx_context *ctx, Model &&m)
     }
     dm.map = ctx->map.as<int>();
     dm.slot_basic = ctx->slot_basic.as<int>();
-    dm.slot_abc = ctx->slot_abc.as<int>();
+    dm.force_basic = ctx->force_basic.as<int>();
+    dm.mono_tab = ctx->mono_tab.as<unsigned short>();
     dm.dup = ctx->dup.as<int>();
     dm.fwd_level_step = ctx->fwd_level.as<int>();
     dm.fwd_steps = ctx->fwd_steps.as<int2>();

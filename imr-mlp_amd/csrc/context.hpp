@@ -27,7 +27,7 @@ struct mtpx_context {
     Plan plan;
     DevModel dm{};
     // model buffers
-    DBuf radial, species, moment, map, seed, slot_basic, slot_abc, dup, fwd_level, fwd_steps,
+    DBuf radial, species, moment, map, seed, slot_basic, force_basic, mono_tab, dup, fwd_level, fwd_steps,
         fwd_lcomb, fwd_comb, bwd_level, bwd_steps, bwd_lcomb, bwd_comb, rb_table;
     // MTP-M head tables and the DevHead that points at them
     DBuf head_ids, head_proj, head_dsp, head_coef, head_params;
@@ -123,7 +123,7 @@ struct mtpx_context {
 
     ~mtpx_context()
     {
-        for (DBuf *b : {&radial, &species, &moment, &map, &seed, &slot_basic, &slot_abc, &dup,
+        for (DBuf *b : {&radial, &species, &moment, &map, &seed, &slot_basic, &force_basic, &mono_tab, &dup,
                         &fwd_level, &fwd_steps, &fwd_lcomb, &fwd_comb, &bwd_level, &bwd_steps,
                         &bwd_lcomb, &bwd_comb, &rb_table, &head_ids, &head_proj, &head_dsp,
                         &head_coef, &head_params, &offsets, &idx, &type, &x, &y, &z, &d,

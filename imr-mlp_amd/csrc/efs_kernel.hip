@@ -80,14 +80,10 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
 
         // ---- basic moments -------------------------------------------------
         for (int base = 0; base < n; base += kWave) {
-            FwdCtx cx{red, mom, L.slot_basic, lane, 0};
             Nbr<P::M> q;
             const bool valid = lane < n - base;
             load_neighbor<P>(m, nb, L.coef, ti, beg + base + lane, valid, q);
-            fwd_shells<0, P>(m, cx, q, nullptr);
-            const int rest = cx.slot % kChunk;
-            if (rest)
-                reduce_chunk(red, rest, cx.slot - rest, L.slot_basic, mom, lane);
+            add_moments<P>(m, red, L.mono, mom, q, n - base, lane);
         }
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
@@ -128,9 +124,9 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
             for (int k = 0; k < m.ndup; ++k)
                 A[m.dup[2 * k + 1]] += A[m.dup[2 * k]];
         wave_sync();
-        // slot-ordered adjoints
-        for (int s = lane; s < m.nslots; s += kWave) {
-            const int b = L.slot_basic[s];
+        // the force polynomials' coefficients
+        for (int s = lane; s < m.nforce; s += kWave) {
+            const int b = L.force_basic[s];
             As[s] = b >= 0 ? A[b] : 0.0;
         }
         wave_sync();
@@ -143,12 +139,8 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
             const int64_t p = beg + base + lane;
             Nbr<P::M> q;
             load_neighbor<P>(m, nb, L.coef, ti, p, valid, q);
-            BwdAcc acc{0, 0, 0, 0};
-            int slot = 0;
-            bwd_shells<0, P>(m, As, slot, q, nullptr, acc);
-            const double D0 = acc.s * q.ux + acc.gx * q.invd;
-            const double D1 = acc.s * q.uy + acc.gy * q.invd;
-            const double D2 = acc.s * q.uz + acc.gz * q.invd;
+            double D0, D1, D2;
+            force_of<P>(m, As, q, D0, D1, D2);
             const double r[3] = {q.x, q.y, q.z}, D[3] = {D0, D1, D2};
 #pragma unroll
             for (int a = 0; a < 3; ++a)
@@ -460,6 +452,17 @@ int efs_variant(const DevModel &m, int R)
     if (m.M <= 4 && m.numax_all <= 6 && R <= 8)
         return 3;
     return 4;
+}
+
+int efs_profile_degree(const DevModel &m)
+{
+    switch (efs_variant(m, m.R)) {
+    case 0: return ProfLevel16::NUMAX;
+    case 1: return ProfLevel20::NUMAX;
+    case 2: return ProfLevel10::NUMAX;
+    case 3: return ProfSmall::NUMAX;
+    default: return ProfGeneric::NUMAX;
+    }
 }
 
 hipError_t launch_efs(const DevModel &m, const DevNeighbors &nb, const EfsOut &out,

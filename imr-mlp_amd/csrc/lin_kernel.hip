@@ -80,6 +80,24 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
+// The monomials of degree NU from those of degree NU - 1.
+template <int NU, int MMAX>
+__device__ __forceinline__ void next_shell(const double *prev, double *cur, const Nbr<MMAX> &q)
+{
+#pragma unroll
+    for (int a = NU; a >= 0; --a)
+#pragma unroll
+        for (int b = NU - a; b >= 0; --b) {
+            const int i = shell_index(NU, a, b);
+            if (a > 0)
+                cur[i] = prev[shell_index(NU - 1, a - 1, b)] * q.ux;
+            else if (b > 0)
+                cur[i] = prev[shell_index(NU - 1, 0, b - 1)] * q.uy;
+            else
+                cur[i] = prev[shell_index(NU - 1, 0, 0)] * q.uz;
+        }
+}
+
 // Inverse of shell_index: the (a, b) of the i-th monomial of shell nu.
 constexpr int shell_a(int nu, int i)
 {
@@ -365,13 +383,9 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void lin_jac_kernel(DevModel m, D
             mom[k] = 0.0;
         wave_sync();
         for (int base = 0; base < n; base += kWave) {
-            FwdCtx cx{red, mom, Ls.slot_basic, lane, 0};
             Nbr<P::M> q;
             load_neighbor<P>(m, nb, Ls.coef, ti, beg + base + lane, lane < n - base, q);
-            fwd_shells<0, P>(m, cx, q, nullptr);
-            const int rest = cx.slot % kChunk;
-            if (rest)
-                reduce_chunk(red, rest, cx.slot - rest, Ls.slot_basic, mom, lane);
+            add_moments<P>(m, red, Ls.mono, mom, q, n - base, lane);
         }
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)

@@ -915,6 +915,14 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
                 }
         }
     p.nslots = (int)p.slot_basic.size();
+    for (int mu = 0; mu < m.M; ++mu) {
+        for (int a = p.numax[mu]; a >= 0; --a)
+            for (int b = p.numax[mu] - a; b >= 0; --b)
+                for (int c = p.numax[mu] - a - b; c >= 0; --c)
+                    p.force_basic.push_back(first[key(mu, a, b, c)]);
+        if (p.force_basic.size() & 1)
+            p.force_basic.push_back(-1);
+    }
     for (int k = 0; k < (kMaxNu + 1) * kMaxMu; ++k)
         p.slot_base[k] = -1;
     {
@@ -985,17 +993,18 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     // The moment reduction's transpose buffer lies over the adjoint block
     // (unused until the seeds are written; the zero slot and the partial sums
     // under it are cleared again after the neighbour pass) and the force
-    // pass's slot-ordered adjoints over the moments (not read after the
+    // pass's adjoints over the moments (not read after the
     // reverse rules), where they fit; then the wave's energy/virial sums.
     const int RB = kChunk * kRedStride;
+    const int F4 = ((int)p.force_basic.size() + 3) & ~3;
     int end;
-    if (N4 <= p.K4) {
+    if (F4 <= p.K4) {
         p.efs_red = p.K4;
         p.efs_stage = 0;
         end = std::max(p.red0, p.K4 + RB);
     } else {
         p.efs_red = p.efs_stage = p.red0;
-        end = p.red0 + std::max(RB, N4);
+        end = p.red0 + std::max(RB, F4);
     }
     p.efs_acc = (end + 3) & ~3;
     p.priv_doubles = p.efs_acc + 12;  // energy, virial[9], padding
@@ -1060,6 +1069,47 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     }
     p.tr_priv = end;
     return true;
+}
+
+void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
+                  unsigned &groups)
+{
+    tab.clear();
+    groups = 0;
+    std::vector<std::array<int, 3>> mono;
+    for (int c = 0; c <= nu; ++c)
+        for (int b = 0; b <= nu - c; ++b)
+            for (int a = 0; a <= nu - c - b; ++a)
+                mono.push_back({a, b, c});
+    for (size_t ch = 0; ch * kChunk < mono.size(); ++ch)
+        for (int g = 0; 4 * g < m.M; ++g) {
+            std::vector<unsigned short> t(kWave, 0xffff);
+            bool any = false;
+            for (int l = 0; l < kWave; ++l) {
+                const int mu = 4 * g + l / kChunk;
+                const size_t e = ch * kChunk + l % kChunk;
+                if (mu >= m.M || e >= mono.size())
+                    continue;
+                const int a = mono[e][0], b = mono[e][1], c = mono[e][2], n = a + b + c;
+                if (n > p.numax[mu])
+                    continue;
+                // position in the slot order: a = n..0, b = n-a..0
+                int pos = 0;
+                for (int ap = n; ap > a; --ap)
+                    pos += n - ap + 1;
+                const int basic = p.slot_basic[p.slot_base[n * kMaxMu + mu] + pos + (n - a - b)];
+                if (basic >= 0) {
+                    t[l] = (unsigned short)basic;
+                    any = true;
+                }
+            }
+            // (the first group's tables are all there: the compile-time
+            // profiles take every chunk for it)
+            if (any || g == 0) {
+                groups |= 1u << (2 * ch + g);
+                tab.insert(tab.end(), t.begin(), t.end());
+            }
+        }
 }
 
 namespace {

@@ -594,125 +594,307 @@ __device__ __forceinline__ void load_neighbor(const DevModel &m, const DevNeighb
     }
 }
 
-template <int NU, int MMAX>
-__device__ __forceinline__ void next_shell(const double *prev, double *cur, const Nbr<MMAX> &q)
+// ---- basic moments -----------------------------------------------------------
+// Every basic moment is sum_j f_mu(d_j) Y_abc(u_j) over the neighbours j: the
+// product of the M x n matrix of radial functions with the n x N matrix of
+// monomials.  The matrix cores form it with v_mfma_f64_4x4x4 (four blocks of
+// 4 x 4 x 4: four radial functions by sixteen monomials, four neighbours a
+// step), so the sum over the lanes needs no adds and lane swaps of its own,
+// and a monomial is written to the transpose buffer once, not once per radial
+// function.  Operand layouts: A (radial functions) row lane & 3, neighbour
+// lane >> 4; B (monomials) column lane & 15, neighbour lane >> 4; the result
+// column lane & 15, row lane >> 4.
+//
+// Monomials are numbered by c, b, a (a fastest, a + b + c <= NUMAX of the
+// kernel's profile): each is the one before times u_x, so the pass holds
+// three running products instead of two whole shells.
+constexpr int mono_count(int nu) { return (nu + 1) * (nu + 2) * (nu + 3) / 6; }
+constexpr int mono_chunks(int nu) { return (mono_count(nu) + kChunk - 1) / kChunk; }
+
+// Bit g: the chunk holds a moment of radial functions 4 g .. 4 g + 3.  The
+// run-time profiles read the masks of the table (Plan::mono_groups); a
+// compile-time profile's radial functions past the fourth reach degree 0
+// only, the first monomial.
+template <class P>
+__device__ __forceinline__ unsigned mono_groups(const DevModel &m, int ch)
 {
-#pragma unroll
-    for (int a = NU; a >= 0; --a)
-#pragma unroll
-        for (int b = NU - a; b >= 0; --b) {
-            const int i = shell_index(NU, a, b);
-            if (a > 0)
-                cur[i] = prev[shell_index(NU - 1, a - 1, b)] * q.ux;
-            else if (b > 0)
-                cur[i] = prev[shell_index(NU - 1, 0, b - 1)] * q.uy;
-            else
-                cur[i] = prev[shell_index(NU - 1, 0, 0)] * q.uz;
-        }
+    if constexpr (P::exact) {
+        static_assert(P::M <= 4 || P::nm[4] == 0, "second group: degree 0");
+        return P::M > 4 && ch == 0 ? 3u : 1u;
+    } else {
+        return (m.mono_groups >> (2 * ch)) & 3u;
+    }
 }
 
-// Sum `nrows` slots of the transpose buffer over the neighbour columns and
-// add the sums to the moment array.  Rows hold 64 columns; columns of lanes
-// without a neighbour hold zeros.  Lanes 0 .. nrows-1 hold the row sums.
-__device__ __forceinline__ void reduce_chunk(const double *red, int nrows, int slot0,
-                                             const int *slot_basic, double *mom, int lane)
+// One 8-byte LDS read; volatile keeps the compiler from pairing reads into
+// ds_read2_b64, which moves 16 bytes a lane in 8.3 cycles of the LDS pipe
+// (two ds_read_b64: 5.4).
+__device__ __forceinline__ double lds_read(const double *p)
+{
+    return *(const volatile __attribute__((address_space(3))) double *)p;
+}
+__device__ __forceinline__ void lds_write(double *p, double v)
+{
+    *(volatile __attribute__((address_space(3))) double *)p = v;
+}
+
+// The chunk of kChunk monomials in the transpose buffer, against the radial
+// functions of group G (rows 4 G .. 4 G + 3): the sums go to the moments of
+// the chunk's table entries (0xffff: no such moment).  Columns past the
+// batch's neighbours hold zero radial functions, so whole groups of sixteen
+// neighbours past the end are left out.
+template <int G>
+__device__ __forceinline__ void moment_chunk(const double *red, const double (&af)[G][kWave / 4],
+                                             unsigned groups, const unsigned short *tab, int cnt,
+                                             double *mom, int lane)
 {
     wave_sync();
-    const double acc = chunk_row_sum(red, lane);
-    if (lane < nrows) {
-        const int b = slot_basic[slot0 + lane];
-        if (b >= 0)
-            mom[b] += acc;
-    }
-    wave_sync();
-}
-
-struct FwdCtx {
-    double *red, *mom;
-    const int *slot_basic;
-    int lane, slot;  // slots written so far; rows are packed across (nu, mu) blocks
-};
-
-template <int NU, class P>
-__device__ __forceinline__ void fwd_shells(const DevModel &m, FwdCtx &cx, const Nbr<P::M> &q,
-                                           const double *prev)
-{
-    double cur[shell_size(NU)];
-    if constexpr (NU == 0)
-        cur[0] = 1.0;
-    else
-        next_shell<NU, P::M>(prev, cur, q);
+    const double *b = red + (lane & (kChunk - 1)) * kRedStride + (lane >> 4);
+    double s0[G], s1[G];
 #pragma unroll
-    for (int mu = 0; mu < P::M; ++mu) {
-        if (P::active(m, mu, NU)) {
-            __builtin_amdgcn_sched_barrier(0);
+    for (int g = 0; g < G; ++g)
+        s0[g] = s1[g] = 0.0;
+    double v[kWave / 4];
 #pragma unroll
-            for (int i = 0; i < shell_size(NU); ++i) {
-                cx.red[(cx.slot % kChunk) * kRedStride + cx.lane] = q.f[mu] * cur[i];
-                ++cx.slot;
-                if (cx.slot % kChunk == 0)
-                    reduce_chunk(cx.red, kChunk, cx.slot - kChunk, cx.slot_basic, cx.mom,
-                                 cx.lane);
-            }
-        }
-    }
-    if constexpr (NU < P::NUMAX) {
-        if (P::deeper(m, NU))
-            fwd_shells<NU + 1, P>(m, cx, q, cur);
-    }
-}
-
-struct BwdAcc {
-    double s, gx, gy, gz;
-};
-
-// Force pass over the slots: u = sum A Y, G = sum (a A, b A, c A) . Y_{-1}
-// with the slot-ordered adjoints A (an 8-byte LDS broadcast per slot; the
-// integer factors are applied in registers).
-template <int NU, class P>
-__device__ __forceinline__ void bwd_shells(const DevModel &m, const double *As, int &slot,
-                                           const Nbr<P::M> &q, const double *prev, BwdAcc &acc)
-{
-    double cur[shell_size(NU)];
-    if constexpr (NU == 0)
-        cur[0] = 1.0;
-    else
-        next_shell<NU, P::M>(prev, cur, q);
+    for (int q = 0; q < kWave / 4; ++q)
+        v[q] = lds_read(b + 4 * q);
 #pragma unroll
-    for (int mu = 0; mu < P::M; ++mu) {
-        if (P::active(m, mu, NU)) {
-            // keep the adjoint loads of one (nu, mu) block from being hoisted
-            // into the previous one: bounds the live registers
-            __builtin_amdgcn_sched_barrier(0);
-            double u = 0, Gx = 0, Gy = 0, Gz = 0;
+    for (int k = 0; k < kWave / 4; k += 4)
+        if (4 * k < cnt) {
 #pragma unroll
-            for (int a = NU; a >= 0; --a)
+            for (int g = 0; g < G; ++g)
+                if (groups >> g & 1) {
 #pragma unroll
-                for (int b = NU - a; b >= 0; --b) {
-                    const int i = shell_index(NU, a, b);
-                    const double w = As[slot + i];  // LDS broadcast
-                    u += w * cur[i];
-                    if constexpr (NU > 0) {
-                        if (a > 0)
-                            Gx += (w * a) * prev[shell_index(NU - 1, a - 1, b)];
-                        if (b > 0)
-                            Gy += (w * b) * prev[shell_index(NU - 1, a, b - 1)];
-                        if (NU - a - b > 0)
-                            Gz += (w * (NU - a - b)) * prev[shell_index(NU - 1, a, b)];
+                    for (int q = k; q < k + 4; q += 2) {
+                        s0[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(af[g][q], v[q], s0[g], 0, 0, 0);
+                        s1[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(af[g][q + 1], v[q + 1], s1[g],
+                                                                   0, 0, 0);
                     }
                 }
-            const double h = q.fd[mu] - NU * q.f[mu] * q.invd;
-            acc.s += h * u;
-            acc.gx += q.f[mu] * Gx;
-            acc.gy += q.f[mu] * Gy;
-            acc.gz += q.f[mu] * Gz;
-            slot += shell_size(NU);
+        }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+        if (groups >> g & 1) {
+            const int t = tab[lane];
+            tab += kWave;
+            if (t != 0xffff)
+                mom[t] += s0[g] + s1[g];
+        }
+    wave_sync();
+}
+
+// Adds one batch of neighbours (cnt <= 64, lane j holds neighbour j) to the
+// basic moments.  red: 16 rows of kRedStride doubles; tab: m.mono_tab.
+template <class P>
+__device__ __forceinline__ void add_moments(const DevModel &m, double *red,
+                                            const unsigned short *tab, double *mom,
+                                            const Nbr<P::M> &q, int cnt, int lane)
+{
+    constexpr int G = (P::M + 3) / 4;
+    // the radial functions through the transpose buffer into the A operands
+#pragma unroll
+    for (int mu = 0; mu < P::M; ++mu)
+        lds_write(red + mu * kRedStride + lane, q.f[mu]);
+    wave_sync();
+    double af[G][kWave / 4];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        // (rows past the last radial function repeat it; their sums have no
+        // table entry)
+        const double *a = red + min(4 * g + (lane & 3), P::M - 1) * kRedStride + (lane >> 4);
+#pragma unroll
+        for (int s = 0; s < kWave / 4; ++s)
+            af[g][s] = lds_read(a + 4 * s);
+    }
+    wave_sync();
+    double zc = 1.0;
+    int e = 0;
+#pragma unroll
+    for (int c = 0; c <= P::NUMAX; ++c) {
+        double yz = zc;
+#pragma unroll
+        for (int b = 0; b <= P::NUMAX - c; ++b) {
+            double v = yz;
+#pragma unroll
+            for (int a = 0; a <= P::NUMAX - c - b; ++a) {
+                lds_write(red + (e % kChunk) * kRedStride + lane, v);
+                ++e;
+                if (e % kChunk == 0 || e == mono_count(P::NUMAX)) {
+                    const int ch = (e - 1) / kChunk;
+                    const unsigned groups = mono_groups<P>(m, ch);
+                    moment_chunk<G>(red, af, groups, tab, cnt, mom, lane);
+                    tab += kWave * __builtin_popcount(groups);
+                }
+                v *= q.ux;
+            }
+            yz *= q.uy;
+        }
+        zc *= q.uz;
+    }
+}
+
+// ---- force polynomials ---------------------------------------------------
+// The force pass needs, per radial function mu and neighbour, the value and
+// the gradient of the polynomial p_mu(u) = sum_abc A_(mu,abc) ux^a uy^b uz^c
+// (all degrees of mu together, A the adjoints of its basic moments): with
+// t = grad p - u (u . grad p),
+//   sum_abc A grad_r[f Y_abc] = f' p u + (f / d) t,
+// because u . grad Y = nu Y for a monomial of degree nu.  A nested Horner
+// scheme gives both with two multiply-adds per coefficient and holds a dozen
+// values, where a sum over monomials and their derivatives took seven and
+// two whole shells.  Coefficients lie in the order they are used (a, b, c
+// descending, Plan::force_basic), read 16 bytes at a time as LDS broadcasts.
+
+// Coefficients of mu's polynomial, padded to an even count (16-byte pairs).
+constexpr int force_size(int nu) { return nu < 0 ? 0 : ((nu + 1) * (nu + 2) * (nu + 3) / 6 + 1) & ~1; }
+
+struct PolyGrad {
+    double p, x, y, z;
+};
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) const v2d *lds_v2d;
+__device__ __forceinline__ unsigned lds_address(const double *p)
+{
+    return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const double *)p;
+}
+
+// Coefficients of one polynomial, streamed from LDS in blocks of eight
+// (16-byte broadcast reads: 4.5 cycles of the LDS pipe for two, against 8.3
+// for the ds_read2_b64 the compiler forms from 8-byte reads), one block ahead
+// of its use.  The asm ties a block's reads to the running sums, so the
+// compiler cannot move all reads to the front and spill.
+template <int kCount>
+struct CoefStream {
+    unsigned at;
+    v2d buf[2][4];
+    __device__ __forceinline__ void load(int block)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (8 * block + 2 * k < kCount)
+                buf[block & 1][k] = ((lds_v2d)(uintptr_t)at)[4 * block + k];
+    }
+    // tie: a sum that is complete before the first read
+    __device__ __forceinline__ CoefStream(const double *A, double &tie) : at(lds_address(A))
+    {
+        asm volatile("" : "+v"(at), "+v"(tie));
+        load(0);
+    }
+    // coefficient e (asked for in order); v and w: the sums they go into
+    __device__ __forceinline__ double next(int e, double &v, double &w)
+    {
+        if (e % 8 == 0 && e + 8 < kCount) {
+            asm volatile("" : "+v"(at), "+v"(v), "+v"(w));
+            load(e / 8 + 1);
+        }
+        const v2d c = buf[(e / 8) & 1][(e % 8) / 2];
+        return e & 1 ? c.y : c.x;
+    }
+};
+template <int N>
+__device__ __forceinline__ PolyGrad poly_grad(const double *A, double x, double y, double z,
+                                              double &tie)
+{
+    CoefStream<force_size(N)> c(A, tie);
+    PolyGrad g{0, 0, 0, 0};
+    int e = 0;
+#pragma unroll
+    for (int a = N; a >= 0; --a) {
+        double q = 0, qy = 0, qz = 0;
+#pragma unroll
+        for (int b = N - a; b >= 0; --b) {
+            double r = a < N && b == N - a ? c.next(e, g.p, g.x) : c.next(e, q, qz), rz = 0;
+            ++e;
+#pragma unroll
+            for (int k = N - a - b - 1; k >= 0; --k) {
+                const double v = c.next(e, r, rz);
+                ++e;
+                rz = k == N - a - b - 1 ? r : fma(rz, z, r);
+                r = fma(r, z, v);
+            }
+            if (b == N - a) {
+                q = r;
+                qz = rz;
+            } else {
+                qy = b == N - a - 1 ? q : fma(qy, y, q);
+                qz = fma(qz, y, rz);
+                q = fma(q, y, r);
+            }
+            // rows are summed in order (asm statements keep theirs): rows
+            // left open side by side would hold their sums in registers
+            asm volatile("" : "+v"(q), "+v"(qy), "+v"(qz));
+        }
+        if (a == N) {
+            g = PolyGrad{q, 0, qy, qz};
+        } else {
+            g.x = a == N - 1 ? g.p : fma(g.x, x, g.p);
+            g.y = fma(g.y, x, qy);
+            g.z = fma(g.z, x, qz);
+            g.p = fma(g.p, x, q);
+        }
+        asm volatile("" : "+v"(g.p), "+v"(g.x), "+v"(g.y), "+v"(g.z));
+    }
+    return g;
+}
+
+// s = sum_mu f' p, (gx, gy, gz) = sum_mu f grad p
+struct ForceAcc {
+    double s, gx, gy, gz;
+    __device__ __forceinline__ void add(const PolyGrad &g, double f, double fd)
+    {
+        s = fma(fd, g.p, s);
+        gx = fma(f, g.x, gx);
+        gy = fma(f, g.y, gy);
+        gz = fma(f, g.z, gz);
+        asm volatile("" : "+v"(s), "+v"(gx), "+v"(gy), "+v"(gz));
+    }
+};
+template <class P, int MU = 0, int OFF = 0>
+__device__ __forceinline__ void force_exact(const double *As, const Nbr<P::M> &q, ForceAcc &acc)
+{
+    acc.add(poly_grad<P::nm[MU]>(As + OFF, q.ux, q.uy, q.uz, acc.s), q.f[MU], q.fd[MU]);
+    if constexpr (MU + 1 < P::M)
+        force_exact<P, MU + 1, OFF + force_size(P::nm[MU])>(As, q, acc);
+}
+template <int N, int NMAX>
+__device__ __forceinline__ PolyGrad poly_grad_of(int nu, const double *A, double x, double y,
+                                                 double z, double &tie)
+{
+    if constexpr (N < NMAX)
+        if (nu > N)
+            return poly_grad_of<N + 1, NMAX>(nu, A, x, y, z, tie);
+    return poly_grad<N>(A, x, y, z, tie);
+}
+// dE/dr of one neighbour from the staged adjoints.
+template <class P>
+__device__ __forceinline__ void force_of(const DevModel &m, const double *As,
+                                         const Nbr<P::M> &q, double &D0, double &D1, double &D2)
+{
+    ForceAcc acc{0, 0, 0, 0};
+    if constexpr (P::exact) {
+        force_exact<P>(As, q, acc);
+    } else {
+        const double *A = As;
+#pragma unroll 1
+        for (int mu = 0; mu < m.M; ++mu) {
+            const int nu = m.numax[mu];
+            if (nu < 0)
+                continue;
+            double f = q.f[0], fd = q.fd[0];
+#pragma unroll
+            for (int k = 1; k < P::M; ++k) {
+                f = mu == k ? q.f[k] : f;
+                fd = mu == k ? q.fd[k] : fd;
+            }
+            acc.add(poly_grad_of<0, P::NUMAX>(nu, A, q.ux, q.uy, q.uz, acc.s), f, fd);
+            A += force_size(nu);
         }
     }
-    if constexpr (NU < P::NUMAX) {
-        if (P::deeper(m, NU))
-            bwd_shells<NU + 1, P>(m, As, slot, q, cur, acc);
-    }
+    const double ug = fma(q.ux, acc.gx, fma(q.uy, acc.gy, q.uz * acc.gz)) * q.invd;
+    const double s = acc.s - ug;
+    D0 = fma(s, q.ux, acc.gx * q.invd);
+    D1 = fma(s, q.uy, acc.gy * q.invd);
+    D2 = fma(s, q.uz, acc.gz * q.invd);
 }
 
 // One group of up to four steps of a level (cnt of them applied).
@@ -853,7 +1035,8 @@ __device__ __forceinline__ void run_rules(const int2 *tab, const int *level_step
 // optional step tables; every part a multiple of 32 bytes).
 struct Shared {
     double *coef, *seed, *moment;
-    int *map, *slot_basic, *slot_abc;
+    int *map, *slot_basic, *force_basic;
+    unsigned short *mono;
     int2 *fwd_steps, *bwd_steps;
 };
 
@@ -864,8 +1047,8 @@ __device__ __host__ __forceinline__ size_t shared_doubles(const DevModel &m, boo
                                                           bool seeds = true)
 {
     const size_t r4c = ((size_t)m.Z * m.Z * m.M * m.R + 3) & ~size_t(3);
-    const size_t S4 = (m.S + 3) & ~3, N4 = (m.nslots + 3) & ~3;
-    size_t d = r4c + (seeds ? m.K4 : 0) + S4 + (S4 + 2 * N4) / 2;
+    const size_t S4 = (m.S + 3) & ~3, N4 = (m.nslots + 3) & ~3, F4 = (m.nforce + 3) & ~3;
+    size_t d = r4c + (seeds ? m.K4 : 0) + S4 + (S4 + N4 + F4) / 2 + m.nmono / 4;
     if (tables)
         d += (size_t)(m.fwd_nsteps + m.bwd_nsteps) * kWave;
     return (d + 3) & ~size_t(3);
@@ -875,15 +1058,16 @@ __device__ __forceinline__ Shared shared_layout(const DevModel &m, double *base,
                                                 bool seeds = true)
 {
     const int r4c = (m.Z * m.Z * m.M * m.R + 3) & ~3;
-    const int S4 = (m.S + 3) & ~3, N4 = (m.nslots + 3) & ~3;
+    const int S4 = (m.S + 3) & ~3, N4 = (m.nslots + 3) & ~3, F4 = (m.nforce + 3) & ~3;
     Shared L;
     L.coef = base;
     L.seed = seeds ? L.coef + r4c : nullptr;
     L.moment = L.coef + r4c + (seeds ? m.K4 : 0);
     L.map = reinterpret_cast<int *>(L.moment + S4);
     L.slot_basic = L.map + S4;
-    L.slot_abc = L.slot_basic + N4;
-    L.fwd_steps = reinterpret_cast<int2 *>(L.slot_abc + N4);
+    L.force_basic = L.slot_basic + N4;
+    L.mono = reinterpret_cast<unsigned short *>(L.force_basic + F4);
+    L.fwd_steps = reinterpret_cast<int2 *>(L.mono + m.nmono);
     L.bwd_steps = L.fwd_steps + (size_t)m.fwd_nsteps * kWave;
     return L;
 }
@@ -902,10 +1086,12 @@ __device__ __forceinline__ void stage_shared(const DevModel &m, const Shared &L,
         L.moment[k] = m.moment[k];
         L.map[k] = m.map[k];
     }
-    for (int k = tid; k < m.nslots; k += nthreads) {
+    for (int k = tid; k < m.nslots; k += nthreads)
         L.slot_basic[k] = m.slot_basic[k];
-        L.slot_abc[k] = m.slot_abc[k];
-    }
+    for (int k = tid; k < m.nforce; k += nthreads)
+        L.force_basic[k] = m.force_basic[k];
+    for (int k = tid; k < m.nmono; k += nthreads)
+        L.mono[k] = m.mono_tab[k];
     if (tables) {
         for (int k = tid; k < m.fwd_nsteps * kWave; k += nthreads)
             L.fwd_steps[k] = m.fwd_steps[k];

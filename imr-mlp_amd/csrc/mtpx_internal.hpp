@@ -260,6 +260,10 @@ struct Plan {
     int nslots = 0;           // canonical (nu, mu, alpha) slots
     std::vector<int> slot_basic;   // [nslots] basic index or -1 (padding)
     std::vector<int> slot_abc;     // [nslots] a | b << 8 | c << 16
+    // [nforce] basic index (or -1) of each coefficient of the force
+    // polynomials: per mu, a, b, c descending over all degrees up to
+    // numax[mu], padded to an even count
+    std::vector<int> force_basic;
     std::vector<int> dup;          // [ndup][2] {duplicate basic, source basic}
     // Each wave owns a private LDS work space (indices in doubles):
     //   [0, K4) moments | [K4, 2 K4) adjoints | dummy (a zero slot) |
@@ -306,6 +310,10 @@ struct Plan {
     int max_level = 0;
 };
 bool build_plan(const Model &m, Plan &p, std::string &err);
+// The moment tables of a kernel profile whose monomials reach degree nu
+// (numbered by c, b, a, a fastest): see DevModel::mono_tab.
+void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
+                  unsigned &groups);
 
 // Linear-fit plan (sparse Jacobian of the scalar moments w.r.t. the basic
 // moments, see build_lin_plan).  Work space per wave (doubles): the E/F/S
@@ -351,7 +359,7 @@ struct DevHead {
 
 // Device view passed to the kernels by value.
 struct DevModel {
-    int Z, M, R, K, B, T, S, nslots;
+    int Z, M, R, K, B, T, S, nslots, nforce;
     double rmin, rmax, scaling, mult, su, pu;
     // general radial bases (split, or another kind than RBChebyshev): per
     // ordered pair kRbStride doubles (RadialBasis); 0 and nullptr for the
@@ -368,7 +376,14 @@ struct DevModel {
     const int *map;         // [S]
     const double *seed;     // [K] sum of moment coefficients mapped to each moment
     const int *slot_basic;  // [nslots]
-    const int *slot_abc;    // [nslots] a | b << 8 | c << 16
+    const int *force_basic; // [nforce]
+    // moment tables of the kernel's profile (moment_table): per chunk of
+    // kChunk monomials and group of four radial functions with a moment in
+    // it, the basic of lane l (function 4 g + (l >> 4), monomial l & 15) or
+    // 0xffff; two mask bits (groups) per chunk
+    int nmono;
+    unsigned mono_groups;
+    const unsigned short *mono_tab;  // [nmono]
     const int *dup;         // [ndup][2]
     int max_partials;
     int K4, dummy, part0, red0, priv_doubles;  // per-wave work space (Plan)
@@ -428,6 +443,8 @@ struct EfsLaunch {
 bool efs_configure(const DevModel &m, int n, int num_cus, int max_waves, size_t lds_limit,
                    EfsLaunch &cfg, int table_pref = -1);
 int efs_variant(const DevModel &m, int R);
+// Highest degree of the variant's profile.
+int efs_profile_degree(const DevModel &m);
 // launch_efs flags: ordered force assembly (per-entry derivatives, no
 // atomics); site energies and energy only; with the ordered assembly, each
 // atom's own force stored by the kernel (the gather over the mirror entries
