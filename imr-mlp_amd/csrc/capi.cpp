@@ -113,10 +113,8 @@ void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm,
     dm.ndup = (int)P.dup.size() / 2;
     dm.nfwd = (int)P.fwd_level_step.size() - 1;
     dm.nbwd = (int)P.bwd_level_step.size() - 1;
-    dm.max_partials = P.max_partials;
     dm.K4 = P.K4;
     dm.dummy = P.dummy;
-    dm.part0 = P.part0;
     dm.red0 = P.red0;
     dm.priv_doubles = P.priv_doubles;
     dm.efs_red = P.efs_red;
@@ -176,13 +174,13 @@ int install_model(mtpx_context *ctx, Model &&m)
     HIP_TRY(upload(ctx->mono_tab, mono, s), "upload model");
     HIP_TRY(upload(ctx->dup, P.dup, s), "upload model");
     HIP_TRY(upload(ctx->fwd_level, P.fwd_level_step, s), "upload model");
-    HIP_TRY(upload(ctx->fwd_steps, P.fwd_steps, s), "upload model");
+    HIP_TRY(upload(ctx->fwd_steps,
+                   device_steps(P.fwd_steps, P.fwd_level_step, P.fwd_comb, P.fwd_level_comb), s),
+            "upload model");
     HIP_TRY(upload(ctx->bwd_level, P.bwd_level_step, s), "upload model");
-    HIP_TRY(upload(ctx->bwd_steps, P.bwd_steps, s), "upload model");
-    HIP_TRY(upload(ctx->fwd_lcomb, P.fwd_level_comb, s), "upload model");
-    HIP_TRY(upload(ctx->fwd_comb, P.fwd_comb, s), "upload model");
-    HIP_TRY(upload(ctx->bwd_lcomb, P.bwd_level_comb, s), "upload model");
-    HIP_TRY(upload(ctx->bwd_comb, P.bwd_comb, s), "upload model");
+    HIP_TRY(upload(ctx->bwd_steps,
+                   device_steps(P.bwd_steps, P.bwd_level_step, P.bwd_comb, P.bwd_level_comb), s),
+            "upload model");
     if (dm.rb_general) {
         // per ordered pair: kind, min, max, scaling and the setup constants
         // of the basis (basis/basis.cpp setup(): mult, su, pu, pi / max,
@@ -230,18 +228,14 @@ int install_model(mtpx_context *ctx, Model &&m)
     dm.fwd_steps = ctx->fwd_steps.as<int2>();
     dm.bwd_level_step = ctx->bwd_level.as<int>();
     dm.bwd_steps = ctx->bwd_steps.as<int2>();
-    dm.fwd_level_comb = ctx->fwd_lcomb.as<int>();
-    dm.fwd_comb = ctx->fwd_comb.as<int4>();
-    dm.bwd_level_comb = ctx->bwd_lcomb.as<int>();
-    dm.bwd_comb = ctx->bwd_comb.as<int4>();
     // linear-fit plan: optional (the linear entry points report its error)
     const bool lin_ok = build_lin_plan(M, P, ctx->lin, ctx->lin_err);
     if (lin_ok) {
         const LinPlan &lp = ctx->lin;
         HIP_TRY(upload(ctx->lin_level, lp.level_step, s), "upload model");
-        HIP_TRY(upload(ctx->lin_steps, lp.steps, s), "upload model");
-        HIP_TRY(upload(ctx->lin_lcomb, lp.level_comb, s), "upload model");
-        HIP_TRY(upload(ctx->lin_comb, lp.comb, s), "upload model");
+        HIP_TRY(upload(ctx->lin_steps,
+                       device_steps(lp.steps, lp.level_step, lp.comb, lp.level_comb), s),
+                "upload model");
         HIP_TRY(upload(ctx->lin_ent, lp.slot_L, s), "upload model");
         HIP_TRY(upload(ctx->lin_estart, lp.slot_mask, s), "upload model");
         HIP_TRY(upload(ctx->lin_chunk, lp.chunk_s0, s), "upload model");
@@ -251,17 +245,15 @@ int install_model(mtpx_context *ctx, Model &&m)
         HIP_TRY(upload(ctx->lin_walk, lp.walk, s), "upload model");
         HIP_TRY(upload(ctx->lin_walk_off, lp.walk_off, s), "upload model");
         HIP_TRY(upload(ctx->lin_flevel, lp.fwd_level_step, s), "upload model");
-        HIP_TRY(upload(ctx->lin_fsteps, lp.fwd_steps, s), "upload model");
-        HIP_TRY(upload(ctx->lin_flcomb, lp.fwd_level_comb, s), "upload model");
-        HIP_TRY(upload(ctx->lin_fcomb, lp.fwd_comb, s), "upload model");
+        HIP_TRY(upload(ctx->lin_fsteps,
+                       device_steps(lp.fwd_steps, lp.fwd_level_step, lp.fwd_comb, lp.fwd_level_comb), s),
+                "upload model");
         DevLin &L = ctx->dl;
         L.dummy = lp.dummy;
         L.red0 = lp.red0;
         L.nfwd = (int)lp.fwd_level_step.size() - 1;
         L.fwd_level_step = ctx->lin_flevel.as<int>();
-        L.fwd_level_comb = ctx->lin_flcomb.as<int>();
         L.fwd_steps = ctx->lin_fsteps.as<int2>();
-        L.fwd_comb = ctx->lin_fcomb.as<int4>();
         L.nL = lp.nL;
         L.one = lp.one;
         L.L0 = lp.L0;
@@ -272,9 +264,7 @@ int install_model(mtpx_context *ctx, Model &&m)
         L.nchunks = lp.nchunks;
         L.nlev = (int)lp.level_step.size() - 1;
         L.level_step = ctx->lin_level.as<int>();
-        L.level_comb = ctx->lin_lcomb.as<int>();
         L.steps = ctx->lin_steps.as<int2>();
-        L.comb = ctx->lin_comb.as<int4>();
         L.slot_L = ctx->lin_ent.as<int>();
         L.slot_mask = ctx->lin_estart.as<int>();
         L.chunk_s0 = ctx->lin_chunk.as<int>();

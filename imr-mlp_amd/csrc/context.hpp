@@ -28,7 +28,7 @@ struct mtpx_context {
     DevModel dm{};
     // model buffers
     DBuf radial, species, moment, map, seed, slot_basic, force_basic, mono_tab, dup, fwd_level, fwd_steps,
-        fwd_lcomb, fwd_comb, bwd_level, bwd_steps, bwd_lcomb, bwd_comb, rb_table;
+        bwd_level, bwd_steps, rb_table;
     // MTP-M head tables and the DevHead that points at them
     DBuf head_ids, head_proj, head_dsp, head_coef, head_params;
 
@@ -72,8 +72,8 @@ struct mtpx_context {
     std::string lin_err;
     LinPlan lin;
     DevLin dl{};
-    DBuf lin_level, lin_steps, lin_lcomb, lin_comb, lin_ent, lin_estart, lin_chunk, lin_maskw,
-        lin_clist, lin_flevel, lin_fsteps, lin_flcomb, lin_fcomb, lin_walk, lin_walk_off, lin_cscal;
+    DBuf lin_level, lin_steps, lin_ent, lin_estart, lin_chunk, lin_maskw,
+        lin_clist, lin_flevel, lin_fsteps, lin_walk, lin_walk_off, lin_cscal;
     DBuf comp, row_src, row_sw, row_y, rowsA, rowsY, gram_part, gram_out, lin_pair, lin_site;
     // tile path: walk-order Jacobian values per site, structure lists per size class
     DBuf lin_lw, lin_tiles;
@@ -124,8 +124,7 @@ struct mtpx_context {
     ~mtpx_context()
     {
         for (DBuf *b : {&radial, &species, &moment, &map, &seed, &slot_basic, &force_basic, &mono_tab, &dup,
-                        &fwd_level, &fwd_steps, &fwd_lcomb, &fwd_comb, &bwd_level, &bwd_steps,
-                        &bwd_lcomb, &bwd_comb, &rb_table, &head_ids, &head_proj, &head_dsp,
+                        &fwd_level, &fwd_steps, &bwd_level, &bwd_steps, &rb_table, &head_ids, &head_proj, &head_dsp,
                         &head_coef, &head_params, &offsets, &idx, &type, &x, &y, &z, &d,
                         &center_type, &rev_offsets, &rev_pairs, &forces, &site_energy, &partial,
                         &pair_ders, &out10, &soff, &center_structure, &site_virial, &benergy,
@@ -133,12 +132,10 @@ struct mtpx_context {
                         &metric_rows, &metrics, &grad_rows, &grad, &nbh_tmp.offsets,
                         &nbh_tmp.idx, &nbh_tmp.type, &nbh_tmp.x, &nbh_tmp.y, &nbh_tmp.z,
                         &nbh_tmp.d, &nbh_tmp.center_type, &nbh.mirror, &nbh_tmp.mirror,
-                        &lin_level, &lin_steps, &lin_lcomb,
-                        &lin_comb, &lin_ent, &lin_estart, &lin_chunk, &lin_maskw, &lin_clist,
+                        &lin_level, &lin_steps, &lin_ent, &lin_estart, &lin_chunk, &lin_maskw, &lin_clist,
                         &lin_walk, &lin_walk_off, &lin_cscal,
                         &comp, &row_src, &row_sw, &row_y, &rowsA, &rowsY, &gram_part, &gram_out,
-                        &lin_pair, &lin_site, &lin_flevel, &lin_fsteps, &lin_flcomb,
-                        &lin_fcomb, &lin_lw, &lin_tiles})
+                        &lin_pair, &lin_site, &lin_flevel, &lin_fsteps, &lin_lw, &lin_tiles})
             b->release();
         scratch.release_all();
         sites.release();

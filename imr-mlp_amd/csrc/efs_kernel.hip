@@ -14,16 +14,21 @@
 //   1. lanes over neighbours: Chebyshev basis Q_k(d), radial functions
 //      f_mu = sum_k c[ti,tj,mu,k] Q_k (coefficients staged in LDS), unit
 //      vector u = r/d.  Every basic moment (mu, a, b, c) equals
-//      sum_j f_mu(d_j) * Y_abc(u_j) with Y_abc = ux^a uy^b uz^c, so the basics
-//      are produced shell by shell (degree nu = a+b+c, compile-time unrolled)
-//      in registers and summed over neighbours through a padded LDS
-//      transpose, 16 slots at a time.
+//      sum_j f_mu(d_j) * Y_abc(u_j) with Y_abc = ux^a uy^b uz^c: the product
+//      of radial functions and monomials, formed on the fp64 matrix cores
+//      from 16 monomials at a time in a transpose buffer (add_moments).
 //   2. the product rules run lane-parallel from lane-major step tables of
 //      8-byte entries, one dependency level at a time (forward values, then
-//      reverse adjoints).
-//   3. lanes over neighbours again: dE_i/dr_j from the closed form
-//      grad_r[f Y] = (f' - nu f/d) Y u + (f/d) grad_u Y, with the basic
-//      adjoints read as LDS broadcasts.
+//      reverse adjoints; run_rules).
+//   3. lanes over neighbours again: dE_i/dr_j from the value and gradient of
+//      one polynomial in u per radial function, by nested Horner over the
+//      basic adjoints read as LDS broadcasts (force_of).
+//   Measured (32,000 atoms, level 16; 256,000 atoms, level 20): slots summed
+//   through the buffer, per-slot force sums and rules with predicated
+//   read-modify-writes 294 us and 6.0 ms; the matrix-core moments and Horner
+//   forces 246 us and 4.9 ms; rules in seven instructions a step 207 us and
+//   4.3 ms.  It is bound by the LDS pipe (rule gathers, transposes) and the
+//   vector unit in about equal parts.
 //   4. F_i += sum_j D_j, F_idx(j) -= D_j, S_ab -= D_ja r_jb.  Fast mode uses
 //      fp64 atomics for the neighbour reactions; deterministic mode stores D
 //      per pair for an ordered gather.  Each atom's energy and virial are
@@ -58,15 +63,12 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
 
     // model tables the per-atom phases index, staged once per workgroup
     stage_shared(m, L, kTabLds, tid, blockDim.x);
-    // the dummy slot and the partial sums start at zero; the rule phases
-    // leave them zero
-    for (int k = m.dummy + lane; k < m.red0; k += kWave)
-        ws[k] = 0.0;
     if (lane < 10)
         sums[lane] = 0.0;
     __syncthreads();
-    const int2 *fwd_tab = kTabLds ? L.fwd_steps : m.fwd_steps;
-    const int2 *bwd_tab = kTabLds ? L.bwd_steps : m.bwd_steps;
+    using Steps = std::conditional_t<kTabLds, LdsSteps, GlobalSteps>;
+    const Steps fwd_tab(kTabLds ? L.fwd_steps : m.fwd_steps, lane);
+    const Steps bwd_tab(kTabLds ? L.bwd_steps : m.bwd_steps, lane);
 
     const int row = blockIdx.x * nwaves + wave;
     for (int i = row; i < nb.n; i += gridDim.x * nwaves) {
@@ -88,12 +90,12 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
                 mom[m.dup[2 * k]] = mom[m.dup[2 * k + 1]];
-        // the zero slot and the partial sums may lie under the transpose buffer
-        for (int k = m.dummy + lane; k < m.red0; k += kWave)
-            ws[k] = 0.0;
+        // the zero slot may lie under the transpose buffer
+        if (lane == 0)
+            ws[m.dummy] = 0.0;
         wave_sync();
 
-        run_rules<false, false>(fwd_tab, m.fwd_level_step, m.fwd_level_comb, m.fwd_comb, m.nfwd, ws, lane);
+        run_rules<false>(fwd_tab, m.fwd_level_step, m.nfwd, ws);
 
         // ---- site energy (potential_mtp.cpp:2966-2970) and adjoint seed ----
         // (an MTP-M head: the head of the descriptors, its seeds per atom)
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
                 A[k] = L.seed[k];
         wave_sync();
 
-        run_rules<false, true>(bwd_tab, m.bwd_level_step, m.bwd_level_comb, m.bwd_comb, m.nbwd, ws, lane);
+        run_rules<false>(bwd_tab, m.bwd_level_step, m.nbwd, ws);
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
                 A[m.dup[2 * k + 1]] += A[m.dup[2 * k]];

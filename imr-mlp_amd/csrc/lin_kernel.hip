@@ -361,8 +361,8 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void lin_jac_kernel(DevModel m, D
     double *mom = ws, *red = ws + L.red0;
 
     stage_shared(m, Ls, false, tid, blockDim.x);
-    for (int k = L.dummy + lane; k < L.red0; k += kWave)
-        ws[k] = 0.0;
+    if (lane == 0)
+        ws[L.dummy] = 0.0;
     // the walk order's work-space indices, the same for every site: held in
     // lane registers where they fit (entry lane + 64 k in register k)
     constexpr int kWalkRegs = 16;
@@ -391,15 +391,14 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void lin_jac_kernel(DevModel m, D
             for (int k = 0; k < m.ndup; ++k)
                 mom[m.dup[2 * k]] = mom[m.dup[2 * k + 1]];
         wave_sync();
-        run_rules<false, false>(L.fwd_steps, L.fwd_level_step, L.fwd_level_comb, L.fwd_comb,
-                                L.nfwd, ws, lane);
+        run_rules<false>(GlobalSteps(L.fwd_steps, lane), L.fwd_level_step, L.nfwd, ws);
         double *srow = g.site + (size_t)(i - g.a0) * m.S;
         for (int s = lane; s < m.S; s += kWave)
             srow[s] = mom[Ls.map[s]];
         for (int k = L.one + lane; k < L.L0 + L.nL; k += kWave)
             ws[k] = k == L.one ? 1.0 : 0.0;
         wave_sync();
-        run_rules<false, false>(L.steps, L.level_step, L.level_comb, L.comb, L.nlev, ws, lane);
+        run_rules<false>(GlobalSteps(L.steps, lane), L.level_step, L.nlev, ws);
         double *lw = g.lw + (size_t)(i - g.a0) * L.nwalk;
         if (walk_regs) {
 #pragma unroll

@@ -1071,6 +1071,34 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     return true;
 }
 
+std::vector<int> device_steps(const std::vector<int> &steps, const std::vector<int> &level_step,
+                              const std::vector<int> &comb, const std::vector<int> &level_comb)
+{
+    std::vector<int> out(steps);
+    size_t i = 0;
+    for (size_t L = 0; L < level_step.size(); ++L) {
+        // the targets of the level's partial sums (numbered anew per level);
+        // the padding after the last level has none
+        std::map<int, int> target;
+        const bool level = L + 1 < level_step.size();
+        if (level)
+            for (int c = 4 * level_comb[L]; c < 4 * level_comb[L + 1]; c += 4)
+                for (int k = 0; k < comb[c + 2]; ++k)
+                    target[comb[c + 1] + k] = comb[c];
+        const size_t end = level ? (size_t)level_step[L + 1] * kWave : steps.size() / 2;
+        for (; i < end; ++i) {
+            const int y = steps[2 * i + 1], last = (y >> 17) & 1, c = y >> 18;
+            int w = y & 0xffff;
+            const auto t = target.find(w);
+            if (last && t != target.end())
+                w = t->second;
+            out[2 * i + 1] =
+                (int)((unsigned)w | ((unsigned)c & 0x3fffu) << 17 | (unsigned)last << 31);
+        }
+    }
+    return out;
+}
+
 void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
                   unsigned &groups)
 {

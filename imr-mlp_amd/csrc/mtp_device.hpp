@@ -5,6 +5,7 @@
 #include "mtpx_internal.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mtpx {
 namespace {
@@ -897,57 +898,101 @@ __device__ __forceinline__ void force_of(const DevModel &m, const double *As,
     D2 = fma(s, q.uz, acc.gz * q.invd);
 }
 
-// One group of up to four steps of a level (cnt of them applied).
-template <bool kInit>
-__device__ __forceinline__ void rule_group(const int2 (&e)[4], int cnt, double *ws, double &acc)
+// ---- product rules -------------------------------------------------------------
+// base + kScale * (the low / high 16 bits of x): the LDS address of a table
+// entry's operand in one instruction
+template <int kScale>
+__device__ __forceinline__ unsigned lo16_address(unsigned x, unsigned base)
 {
+    unsigned a;
+    asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(a) : "v"(x), "n"(kScale), "v"(base));
+    return a;
+}
+template <int kScale>
+__device__ __forceinline__ unsigned hi16_address(unsigned x, unsigned base)
+{
+    unsigned a;
+    asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]"
+        : "=v"(a)
+        : "v"(x), "n"(kScale), "v"(base));
+    return a;
+}
+__device__ __forceinline__ void lds_add(unsigned at, double v)
+{
+    __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double *)(uintptr_t)at,
+                                        v);
+}
+
+// A lane's column of a step table: in LDS (8-byte reads, not paired: see
+// lds_read) or in global memory.
+struct LdsSteps {
+    unsigned at;
+    __device__ __forceinline__ LdsSteps(const int2 *tab, int lane)
+        : at(lds_address(reinterpret_cast<const double *>(tab)) + 8u * lane)
+    {
+    }
+    __device__ __forceinline__ int2 operator[](int s) const
+    {
+        const long long v = *(const volatile __attribute__((address_space(3))) long long *)(
+            uintptr_t)(at + (unsigned)s * (8u * kWave));
+        int y = (int)(v >> 32);
+        asm("" : "+v"(y));  // (a test of y's sign stays a 32-bit compare)
+        return int2{(int)v, y};
+    }
+};
+struct GlobalSteps {
+    const int2 *tab;
+    __device__ __forceinline__ GlobalSteps(const int2 *t, int lane) : tab(t + lane) {}
+    __device__ __forceinline__ int2 operator[](int s) const { return tab[(size_t)s * kWave]; }
+};
+
+// The first cnt of four steps of a level.  A task's sum starts from zero and
+// is added to its target on the task's last entry (the sign bit of y): an
+// LDS add, so no lane waits for the target's old value, and the pieces of a
+// split task add to one target in program order.
+__device__ __forceinline__ double step_factor(int y) { return (double)((int)((unsigned)y << 1) >> 18); }
+__device__ __forceinline__ void rule_group(const int2 (&e)[4], int cnt, unsigned base, double &acc,
+                                           double &)
+{
+    typedef __attribute__((address_space(3))) const double *ptr;
     double ml[4], mr[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int l = e[k].x & 0xffff, r = (unsigned)e[k].x >> 16;
-        ml[k] = ws[l];
-        mr[k] = ws[r];
+        ml[k] = *(ptr)(uintptr_t)lo16_address<8>(e[k].x, base);
+        mr[k] = *(ptr)(uintptr_t)hi16_address<8>(e[k].x, base);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k >= cnt)
             break;
-        const double c = (double)(e[k].y >> 18);
-        acc = fma(c * ml[k], mr[k], acc);
-        if (e[k].y & 0x20000) {
-            const int w = e[k].y & 0xffff;
-            ws[w] = kInit ? ws[w] + acc : acc;
+        acc = fma(step_factor(e[k].y) * ml[k], mr[k], acc);
+        if (e[k].y < 0) {
+            lds_add(lo16_address<8>(e[k].y, base), acc);
             acc = 0.0;
         }
     }
 }
-
 // The same over {value, dual} pairs.
-template <bool kInit>
-__device__ __forceinline__ void rule_group_dual(const int2 (&e)[4], int cnt, double2 *wp,
+__device__ __forceinline__ void rule_group_dual(const int2 (&e)[4], int cnt, unsigned base,
                                                 double &acc, double &acd)
 {
-    double2 vl[4], vr[4];
+    v2d vl[4], vr[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        vl[k] = wp[e[k].x & 0xffff];
-        vr[k] = wp[(unsigned)e[k].x >> 16];
+        vl[k] = *(lds_v2d)(uintptr_t)lo16_address<16>(e[k].x, base);
+        vr[k] = *(lds_v2d)(uintptr_t)hi16_address<16>(e[k].x, base);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k >= cnt)
             break;
-        const double c = (double)(e[k].y >> 18);
-        acc = fma(c * vl[k].x, vr[k].x, acc);
-        acd = fma(c * vl[k].x, vr[k].y, fma(c * vl[k].y, vr[k].x, acd));
-        if (e[k].y & 0x20000) {
-            const int w = e[k].y & 0xffff;
-            if (kInit) {
-                const double2 o = wp[w];
-                wp[w] = double2{o.x + acc, o.y + acd};
-            } else {
-                wp[w] = double2{acc, acd};
-            }
+        const double c = step_factor(e[k].y), l = c * vl[k].x;
+        acc = fma(l, vr[k].x, acc);
+        acd = fma(l, vr[k].y, fma(c * vl[k].y, vr[k].x, acd));
+        if (e[k].y < 0) {
+            const unsigned w = lo16_address<16>(e[k].y, base);
+            lds_add(w, acc);
+            lds_add(w + 8, acd);
             acc = 0.0;
             acd = 0.0;
         }
@@ -956,77 +1001,75 @@ __device__ __forceinline__ void rule_group_dual(const int2 (&e)[4], int cnt, dou
 
 // Product rules from a lane-major step table (forward: potential_mtp.cpp:
 // 2918-2924; reverse: backpropagate_moments, :3292-3305), one dependency
-// level at a time.  Steps are taken in groups of four: the entries of the
-// next group are loaded while the current one runs, and every operand of a
-// group is read before any of its results is written (a level never reads
-// what it writes).  A level's last group holds its last one to four steps;
-// the entries it loads past the level (the next level's, or the padding
-// after the last level) are read but not applied.  A task's sum starts
-// from zero and is stored on the task's last entry: added to its target
-// (kInit: adjoints, which start from their seeds) or written over it
-// (outputs and partial sums, which start at zero).  No task reads or writes
-// another task's target within a level.
+// level at a time.  An entry is x = l | r << 16 (operands, work-space
+// indices), y = w | c << 17 | last << 31 (target, factor, a task's last
+// entry): x_w += c x_l x_r, with targets that start from zero (outputs) or
+// from their seeds (adjoints).  Steps are taken in groups of four: the
+// entries of the next group (of the next level, at a level's end) are loaded
+// while the current one runs, and every operand of a group is read before
+// any of its results is written (a level never reads what it writes).  A
+// level's last group holds its last one to four steps; the entries it loads
+// past the level are read but not applied.  No task reads another task's
+// target within a level.
+//
+// The LDS pipe bounds the phase (two gathers of 6.6 cycles a step, against
+// 2.7 for a linear read) with the vector unit close behind: a step takes
+// seven instructions (two addresses, factor, product, sum, end test) where
+// separate shifts and masks, a predicated read-modify-write of the target
+// and partial sums combined afterwards took 17 and a wait per task.
 //
 // kDual carries a dual value beside every element: the work space holds
 // pairs {x, x'} (element x's value in double 2x, its dual in 2x + 1; the
-// tables' indices count pairs), read and written 16 bytes at a time, and
-// for a step  x_w += c x_l x_r  it adds  c (x'_l x_r + x_l x'_r)  to x'_w.
+// tables' indices count pairs), read 16 bytes at a time, and for a step
+// x_w += c x_l x_r  it adds  c (x'_l x_r + x_l x'_r)  to x'_w.
 // Forward entries then propagate tangents (Q_o += c (Q_l m_r + m_l Q_r));
 // reverse entries, whose l is an adjoint and r a moment, propagate the
 // adjoint of the tangent computation (G_x += c (G_o m_r + A_o Q_r)).
-template <bool kDual, bool kInit>
-__device__ __forceinline__ void run_rules(const int2 *tab, const int *level_step,
-                                          const int *level_comb, const int4 *comb, int nlev,
-                                          double *ws, int lane)
+template <bool kDual, class Steps>
+__device__ __forceinline__ void run_rules(const Steps tab, const int *level_step, int nlev,
+                                          double *ws)
 {
-    double2 *wp = reinterpret_cast<double2 *>(ws);
-    for (int L = 0; L < nlev; ++L) {
-        const int s0 = level_step[L], s1 = level_step[L + 1];
-        double acc = 0.0, acd = 0.0;
-        auto group = [&](const int2(&e)[4], int cnt) {
-            if constexpr (kDual)
-                rule_group_dual<kInit>(e, cnt, wp, acc, acd);
-            else
-                rule_group<kInit>(e, cnt, ws, acc);
-        };
-        if (s1 > s0) {
-            const int2 *t = tab + (size_t)s0 * kWave + lane;
-            int2 e[4] = {t[0], t[kWave], t[2 * kWave], t[3 * kWave]};
-            int st = s0;
-            for (; st + 4 < s1; st += 4) {
-                const int2 *u = t + (size_t)(st + 4 - s0) * kWave;
-                const int2 nx[4] = {u[0], u[kWave], u[2 * kWave], u[3 * kWave]};
-                group(e, 4);
+    const unsigned base = lds_address(ws);
+    // uniform reads: scalar loads
+    const auto *level = (const __attribute__((address_space(4))) int *)(uintptr_t)level_step;
+    auto load = [&](int2(&e)[4], int s) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    e[k] = nx[k];
-            }
-            group(e, s1 - st);
+        for (int k = 0; k < 4; ++k)
+            e[k] = tab[s + k];
+    };
+    auto group = [&](const int2(&e)[4], int cnt, double &acc, double &acd) {
+        if constexpr (kDual)
+            rule_group_dual(e, cnt, base, acc, acd);
+        else
+            rule_group(e, cnt, base, acc, acd);
+    };
+    int2 A[4], B[4];
+    load(A, 0);
+    int st = 0;
+    for (int L = 0; L < nlev; ++L) {
+        const int end = __builtin_amdgcn_readfirstlane(level[L + 1]);
+        double acc = 0.0, acd = 0.0;
+        for (; st + 8 < end; st += 8) {
+            load(B, st + 4);
+            group(A, 4, acc, acd);
+            load(A, st + 8);
+            group(B, 4, acc, acd);
         }
-        const int c0 = level_comb[L], c1 = level_comb[L + 1];
-        if (c1 > c0) {
-            wave_sync();
-            for (int c = c0 + lane; c < c1; c += kWave) {
-                const int4 q = comb[c];
-                if constexpr (kDual) {
-                    double2 sum = wp[q.x];
-                    for (int k = 0; k < q.z; ++k) {
-                        const double2 v = wp[q.y + k];
-                        sum.x += v.x;
-                        sum.y += v.y;
-                        wp[q.y + k] = double2{0.0, 0.0};
-                    }
-                    wp[q.x] = sum;
-                } else {
-                    double sum = ws[q.x];
-                    for (int k = 0; k < q.z; ++k) {
-                        sum += ws[q.y + k];
-                        ws[q.y + k] = 0.0;
-                    }
-                    ws[q.x] = sum;
-                }
-            }
+        // the level's last one or two groups; the last loads the next
+        // level's first
+        if (st + 4 < end) {
+            load(B, st + 4);
+            group(A, 4, acc, acd);
+            load(A, end);
+            group(B, end - st - 4, acc, acd);
+        } else if (st < end) {
+            load(B, end);
+            group(A, end - st, acc, acd);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                A[k] = B[k];
         }
+        st = end;
         wave_sync();
     }
 }

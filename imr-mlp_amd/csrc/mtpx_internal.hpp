@@ -19,11 +19,11 @@ constexpr int kWave = 64;       // CDNA wavefront
 constexpr int kChunk = 16;      // slots per LDS reduction chunk
 constexpr int kRedStride = 66;  // row stride of the reduction buffer (16-byte rows, no bank conflicts)
 // Product-rule step tables: the shortest piece a task is split into, and
-// the padding steps after the last level (the kernels read the steps in
-// groups of four, so a group that starts in a level's last steps reads at
-// most three steps past it).
+// the padding steps after the last level (the kernels load the steps in
+// groups of four, one group ahead, so the last level's last group loads four
+// steps past it).
 constexpr int kMinPiece = 2;
-constexpr int kRulePad = 3;
+constexpr int kRulePad = 4;
 
 // Growable device allocation owned by a context.
 struct DBuf {
@@ -301,7 +301,8 @@ struct Plan {
     // reverse entries of one destination) longer than the level's fair share
     // (entries / 64) is split into pieces that write zeroed partial sums; the
     // level's combine list {target, first partial, count, 0} then adds them
-    // in order to the target and clears them.  Padding steps have c = 0 and
+    // in order to the target (the kernels add the pieces to the target as
+    // they end: device_steps).  Padding steps have c = 0 and
     // read the dummy slot and write nothing.  Tasks and pieces are spread over the
     // lanes by longest-processing-time assignment.
     std::vector<int> fwd_level_step, fwd_steps, fwd_level_comb, fwd_comb;
@@ -310,6 +311,12 @@ struct Plan {
     int max_level = 0;
 };
 bool build_plan(const Model &m, Plan &p, std::string &err);
+// A step table as the kernels read it (run_rules): x as in the plan,
+// y = w | c << 17 | last << 31, and an entry that ends a piece of a split
+// task names the task's target (the kernels add the pieces there; the
+// combine list is not needed).
+std::vector<int> device_steps(const std::vector<int> &steps, const std::vector<int> &level_step,
+                              const std::vector<int> &comb, const std::vector<int> &level_comb);
 // The moment tables of a kernel profile whose monomials reach degree nu
 // (numbered by c, b, a, a fastest): see DevModel::mono_tab.
 void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
@@ -385,8 +392,7 @@ struct DevModel {
     unsigned mono_groups;
     const unsigned short *mono_tab;  // [nmono]
     const int *dup;         // [ndup][2]
-    int max_partials;
-    int K4, dummy, part0, red0, priv_doubles;  // per-wave work space (Plan)
+    int K4, dummy, red0, priv_doubles;  // per-wave work space (Plan)
     int tr_red1, tr_red4, tr_stage, tr_grad, tr_ctype, tr_priv;
     int efs_red, efs_stage, efs_acc;
     // MTP-M head (kHeadNone: the linear MTP of species, moment and seed),
@@ -397,13 +403,9 @@ struct DevModel {
     int slot_base[(kMaxNu + 1) * kMaxMu];
     int fwd_nsteps, bwd_nsteps;  // steps per lane, all levels and the padding
     const int *fwd_level_step;  // [nfwd+1]
-    const int2 *fwd_steps;
-    const int *fwd_level_comb;  // [nfwd+1]
-    const int4 *fwd_comb;
+    const int2 *fwd_steps;      // device_steps
     const int *bwd_level_step;  // [nbwd+1]
     const int2 *bwd_steps;
-    const int *bwd_level_comb;  // [nbwd+1]
-    const int4 *bwd_comb;
 };
 
 // Neighbour lists resident on the device (SoA).
@@ -460,12 +462,10 @@ struct DevLin {
     int nL, one, L0, part0, acc, priv, CH, nchunks, nlev;
     int lane_walk;
     int compiled_walk;  // the plan equals the compiled level-16 walk (lin_walk_compiled)
-    const int *fwd_level_step, *fwd_level_comb;  // [nfwd + 1]
-    const int2 *fwd_steps;
-    const int4 *fwd_comb;
-    const int *level_step, *level_comb;  // [nlev + 1]
-    const int2 *steps;
-    const int4 *comb;
+    const int *fwd_level_step;  // [nfwd + 1]
+    const int2 *fwd_steps;      // device_steps
+    const int *level_step;      // [nlev + 1]
+    const int2 *steps;          // device_steps
     const int *chunk_s0;    // [nchunks + 1] into chunk_scalar
     const int *chunk_scalar;  // [S] the scalars of chunk after chunk
     const int *slot_mask;   // [nchunks][nslots]

@@ -408,15 +408,14 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
     int *ctype = reinterpret_cast<int *>(ws + m.tr_ctype);
 
     stage_shared(m, L, kTabLds, tid, blockDim.x);
-    for (int k = m.dummy + lane; k < m.red0; k += kWave)
-        wp[k] = double2{0.0, 0.0};
     for (int k = lane; k < m.nradial; k += kWave)
         grad[k] = 0.0;
     for (int k = m.nradial + lane; k < m.ncoef; k += kWave)
         grow[k] = 0.0;
     __syncthreads();
-    const int2 *fwd_tab = kTabLds ? L.fwd_steps : m.fwd_steps;
-    const int2 *bwd_tab = kTabLds ? L.bwd_steps : m.bwd_steps;
+    using Steps = std::conditional_t<kTabLds, LdsSteps, GlobalSteps>;
+    const Steps fwd_tab(kTabLds ? L.fwd_steps : m.fwd_steps, lane);
+    const Steps bwd_tab(kTabLds ? L.bwd_steps : m.bwd_steps, lane);
     const int MR = P::exact ? P::M * P::RMAX : m.M * m.R;
 
     for (int i = rowid; i < nb.n; i += gridDim.x * nwaves) {
@@ -458,14 +457,13 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
                 wp[m.dup[2 * k]] = wp[m.dup[2 * k + 1]];
-        // the zero slots and partial sums may lie under a transpose buffer
-        for (int k = m.dummy + lane; k < m.red0; k += kWave)
-            wp[k] = double2{0.0, 0.0};
+        // the zero slot may lie under a transpose buffer
+        if (lane == 0)
+            wp[m.dummy] = double2{0.0, 0.0};
         wave_sync();
 
         // ---- 2. rules forward with tangents; moment and species gradient ----
-        run_rules<true, false>(fwd_tab, m.fwd_level_step, m.fwd_level_comb, m.fwd_comb, m.nfwd, ws,
-                               lane);
+        run_rules<true>(fwd_tab, m.fwd_level_step, m.nfwd, ws);
         for (int s = lane; s < m.S; s += kWave) {
             const double2 x = wp[L.map[s]];
             grow[m.nradial + m.Z + s] += se * x.x + x.y;
@@ -479,8 +477,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
             wp[m.K4 + k] = double2{sd, se * sd};
         }
         wave_sync();
-        run_rules<true, true>(bwd_tab, m.bwd_level_step, m.bwd_level_comb, m.bwd_comb, m.nbwd, ws,
-                              lane);
+        run_rules<true>(bwd_tab, m.bwd_level_step, m.nbwd, ws);
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k) {
                 const double2 v = wp[m.K4 + m.dup[2 * k]];
