@@ -21,17 +21,19 @@ int upload_coeffs(mtpx_context *ctx)
 {
     const Model &m = ctx->model;
     const size_t sp = (size_t)m.nradial(), mo = sp + (size_t)m.nspecies();
-    std::vector<double> radial(m.coef.begin(), m.coef.begin() + sp);
     std::vector<double> species(m.coef.begin() + sp, m.coef.begin() + sp + m.Z);
-    std::vector<double> moment(m.coef.begin() + mo, m.coef.begin() + mo + m.S);
-    std::vector<double> seed((size_t)m.K, 0.0);
+    // the coefficient part of the packed tables
+    const SharedOffsets o(ctx->dm);
+    std::vector<double> packed(o.map, 0.0);
+    std::copy(m.coef.begin(), m.coef.begin() + sp, packed.begin());
+    std::copy(m.coef.begin() + mo, m.coef.begin() + mo + m.S, packed.begin() + o.moment);
     if (m.linear())
         for (int s = 0; s < m.S; ++s)
-            seed[m.map[s]] += moment[s];
-    HIP_TRY(upload(ctx->radial, radial, ctx->stream), "upload radial coefficients");
+            packed[o.seed + m.map[s]] += m.coef[mo + s];
     HIP_TRY(upload(ctx->species, species, ctx->stream), "upload species coefficients");
-    HIP_TRY(upload(ctx->moment, moment, ctx->stream), "upload moment coefficients");
-    HIP_TRY(upload(ctx->seed, seed, ctx->stream), "upload adjoint seeds");
+    HIP_TRY(hipMemcpyAsync(ctx->shared.p, packed.data(), sizeof(double) * packed.size(),
+                           hipMemcpyHostToDevice, ctx->stream),
+            "upload coefficients");
     ctx->dm.hd = nullptr;
     if (!m.linear()) {
         const int P = m.head.P;
@@ -79,10 +81,7 @@ int upload_coeffs(mtpx_context *ctx)
         ctx->dm.hd = static_cast<const DevHead *>(ctx->head_params.p);
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream), "upload coefficients");
-    ctx->dm.radial = ctx->radial.as<double>();
     ctx->dm.species = ctx->species.as<double>();
-    ctx->dm.moment = ctx->moment.as<double>();
-    ctx->dm.seed = ctx->seed.as<double>();
     return MTPX_OK;
 }
 
@@ -168,19 +167,22 @@ int install_model(mtpx_context *ctx, Model &&m)
     const Model &M = ctx->model;
     const Plan &P = ctx->plan;
     hipStream_t s = ctx->stream;
-    HIP_TRY(upload(ctx->map, M.map, s), "upload model");
-    HIP_TRY(upload(ctx->slot_basic, P.slot_basic, s), "upload model");
-    HIP_TRY(upload(ctx->force_basic, P.force_basic, s), "upload model");
-    HIP_TRY(upload(ctx->mono_tab, mono, s), "upload model");
+    // the packed tables (the coefficients follow in upload_coeffs)
+    const SharedOffsets o(dm);
+    std::vector<double> packed(o.end, 0.0);
+    auto pack = [&packed](size_t at, const auto &v) {
+        std::memcpy(packed.data() + at, v.data(), v.size() * sizeof v[0]);
+    };
+    pack(o.map, M.map);
+    pack(o.slot, P.slot_basic);
+    pack(o.force, P.force_basic);
+    pack(o.mono, mono);
+    pack(o.fwd, device_steps(P.fwd_steps, P.fwd_level_step, P.fwd_comb, P.fwd_level_comb));
+    pack(o.bwd, device_steps(P.bwd_steps, P.bwd_level_step, P.bwd_comb, P.bwd_level_comb));
+    HIP_TRY(upload(ctx->shared, packed, s), "upload model");
     HIP_TRY(upload(ctx->dup, P.dup, s), "upload model");
     HIP_TRY(upload(ctx->fwd_level, P.fwd_level_step, s), "upload model");
-    HIP_TRY(upload(ctx->fwd_steps,
-                   device_steps(P.fwd_steps, P.fwd_level_step, P.fwd_comb, P.fwd_level_comb), s),
-            "upload model");
     HIP_TRY(upload(ctx->bwd_level, P.bwd_level_step, s), "upload model");
-    HIP_TRY(upload(ctx->bwd_steps,
-                   device_steps(P.bwd_steps, P.bwd_level_step, P.bwd_comb, P.bwd_level_comb), s),
-            "upload model");
     if (dm.rb_general) {
         // per ordered pair: kind, min, max, scaling and the setup constants
         // of the basis (basis/basis.cpp setup(): mult, su, pu, pi / max,
@@ -219,15 +221,19 @@ int install_model(mtpx_context *ctx, Model &&m)
         HIP_TRY(upload(ctx->rb_table, t, s), "upload model");
         dm.rb_table = ctx->rb_table.as<double>();
     }
-    dm.map = ctx->map.as<int>();
-    dm.slot_basic = ctx->slot_basic.as<int>();
-    dm.force_basic = ctx->force_basic.as<int>();
-    dm.mono_tab = ctx->mono_tab.as<unsigned short>();
+    double *const base = ctx->shared.as<double>();
+    dm.shared = dm.radial = base;
+    dm.seed = base + o.seed;
+    dm.moment = base + o.moment;
+    dm.map = reinterpret_cast<int *>(base + o.map);
+    dm.slot_basic = reinterpret_cast<int *>(base + o.slot);
+    dm.force_basic = reinterpret_cast<int *>(base + o.force);
+    dm.mono_tab = reinterpret_cast<unsigned short *>(base + o.mono);
+    dm.fwd_steps = reinterpret_cast<int2 *>(base + o.fwd);
+    dm.bwd_steps = reinterpret_cast<int2 *>(base + o.bwd);
     dm.dup = ctx->dup.as<int>();
     dm.fwd_level_step = ctx->fwd_level.as<int>();
-    dm.fwd_steps = ctx->fwd_steps.as<int2>();
     dm.bwd_level_step = ctx->bwd_level.as<int>();
-    dm.bwd_steps = ctx->bwd_steps.as<int2>();
     // linear-fit plan: optional (the linear entry points report its error)
     const bool lin_ok = build_lin_plan(M, P, ctx->lin, ctx->lin_err);
     if (lin_ok) {

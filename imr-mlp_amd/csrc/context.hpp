@@ -27,8 +27,7 @@ struct mtpx_context {
     Plan plan;
     DevModel dm{};
     // model buffers
-    DBuf radial, species, moment, map, seed, slot_basic, force_basic, mono_tab, dup, fwd_level, fwd_steps,
-        bwd_level, bwd_steps, rb_table;
+    DBuf shared, species, dup, fwd_level, bwd_level, rb_table;
     // MTP-M head tables and the DevHead that points at them
     DBuf head_ids, head_proj, head_dsp, head_coef, head_params;
 
@@ -123,9 +122,8 @@ struct mtpx_context {
 
     ~mtpx_context()
     {
-        for (DBuf *b : {&radial, &species, &moment, &map, &seed, &slot_basic, &force_basic, &mono_tab, &dup,
-                        &fwd_level, &fwd_steps, &bwd_level, &bwd_steps, &rb_table, &head_ids, &head_proj, &head_dsp,
-                        &head_coef, &head_params, &offsets, &idx, &type, &x, &y, &z, &d,
+        for (DBuf *b : {&shared, &species, &dup, &fwd_level, &bwd_level, &rb_table,
+                        &head_ids, &head_proj, &head_dsp, &head_coef, &head_params, &offsets, &idx, &type, &x, &y, &z, &d,
                         &center_type, &rev_offsets, &rev_pairs, &forces, &site_energy, &partial,
                         &pair_ders, &out10, &soff, &center_structure, &site_virial, &benergy,
                         &bstress, &active, &tE, &wE, &tF, &wF, &tS, &wS, &dLdE, &dLdF, &dLdS,

@@ -1074,8 +1074,9 @@ __device__ __forceinline__ void run_rules(const Steps tab, const int *level_step
     }
 }
 
-// Block-shared LDS tables, in this order (doubles, then ints, then the
-// optional step tables; every part a multiple of 32 bytes).
+// The block-shared model tables in LDS, laid out as the device's packed copy
+// m.shared (SharedOffsets), the adjoint seeds and the step tables left out
+// where a kernel does not take them.
 struct Shared {
     double *coef, *seed, *moment;
     int *map, *slot_basic, *force_basic;
@@ -1083,63 +1084,57 @@ struct Shared {
     int2 *fwd_steps, *bwd_steps;
 };
 
-// The block-shared model tables in LDS: radial coefficients, the adjoint
-// seeds (kernels that run the reverse rules from LDS), moment coefficients,
-// map, slot tables and optionally the rule step tables.
 __device__ __host__ __forceinline__ size_t shared_doubles(const DevModel &m, bool tables,
                                                           bool seeds = true)
 {
-    const size_t r4c = ((size_t)m.Z * m.Z * m.M * m.R + 3) & ~size_t(3);
-    const size_t S4 = (m.S + 3) & ~3, N4 = (m.nslots + 3) & ~3, F4 = (m.nforce + 3) & ~3;
-    size_t d = r4c + (seeds ? m.K4 : 0) + S4 + (S4 + N4 + F4) / 2 + m.nmono / 4;
-    if (tables)
-        d += (size_t)(m.fwd_nsteps + m.bwd_nsteps) * kWave;
-    return (d + 3) & ~size_t(3);
+    const SharedOffsets o(m);
+    return ((tables ? o.end : o.fwd) - (seeds ? 0 : o.moment - o.seed) + 3) & ~size_t(3);
 }
 
 __device__ __forceinline__ Shared shared_layout(const DevModel &m, double *base,
                                                 bool seeds = true)
 {
-    const int r4c = (m.Z * m.Z * m.M * m.R + 3) & ~3;
-    const int S4 = (m.S + 3) & ~3, N4 = (m.nslots + 3) & ~3, F4 = (m.nforce + 3) & ~3;
+    const SharedOffsets o(m);
+    double *rest = seeds ? base : base - (o.moment - o.seed);  // the parts after the seeds
     Shared L;
     L.coef = base;
-    L.seed = seeds ? L.coef + r4c : nullptr;
-    L.moment = L.coef + r4c + (seeds ? m.K4 : 0);
-    L.map = reinterpret_cast<int *>(L.moment + S4);
-    L.slot_basic = L.map + S4;
-    L.force_basic = L.slot_basic + N4;
-    L.mono = reinterpret_cast<unsigned short *>(L.force_basic + F4);
-    L.fwd_steps = reinterpret_cast<int2 *>(L.mono + m.nmono);
-    L.bwd_steps = L.fwd_steps + (size_t)m.fwd_nsteps * kWave;
+    L.seed = seeds ? base + o.seed : nullptr;
+    L.moment = rest + o.moment;
+    L.map = reinterpret_cast<int *>(rest + o.map);
+    L.slot_basic = reinterpret_cast<int *>(rest + o.slot);
+    L.force_basic = reinterpret_cast<int *>(rest + o.force);
+    L.mono = reinterpret_cast<unsigned short *>(rest + o.mono);
+    L.fwd_steps = reinterpret_cast<int2 *>(rest + o.fwd);
+    L.bwd_steps = reinterpret_cast<int2 *>(rest + o.bwd);
     return L;
 }
 
-// Model tables every workgroup stages into its shared LDS region.
+// Copies the model tables into a workgroup's shared LDS region: 16 bytes a
+// lane, eight in flight, so the 27 KB of level 16 arrive in one round trip
+// even to four waves (table by table, each of eight loops waited for its own
+// loads; a level-10 launch of 108 atoms took 15.6 us and takes 12.2).
 __device__ __forceinline__ void stage_shared(const DevModel &m, const Shared &L, bool tables,
                                              int tid, int nthreads)
 {
-    const int ncoef_r = m.Z * m.Z * m.M * m.R;
-    for (int k = tid; k < ncoef_r; k += nthreads)
-        L.coef[k] = m.radial[k];
-    if (L.seed)
-        for (int k = tid; k < m.K; k += nthreads)
-            L.seed[k] = m.seed[k];
-    for (int k = tid; k < m.S; k += nthreads) {
-        L.moment[k] = m.moment[k];
-        L.map[k] = m.map[k];
-    }
-    for (int k = tid; k < m.nslots; k += nthreads)
-        L.slot_basic[k] = m.slot_basic[k];
-    for (int k = tid; k < m.nforce; k += nthreads)
-        L.force_basic[k] = m.force_basic[k];
-    for (int k = tid; k < m.nmono; k += nthreads)
-        L.mono[k] = m.mono_tab[k];
-    if (tables) {
-        for (int k = tid; k < m.fwd_nsteps * kWave; k += nthreads)
-            L.fwd_steps[k] = m.fwd_steps[k];
-        for (int k = tid; k < m.bwd_nsteps * kWave; k += nthreads)
-            L.bwd_steps[k] = m.bwd_steps[k];
+    const SharedOffsets o(m);
+    const v2d *src = reinterpret_cast<const v2d *>(m.shared);
+    v2d *dst = reinterpret_cast<v2d *>(L.coef);
+    const int skip = L.seed ? 0 : (int)(o.moment - o.seed) / 2, cut = (int)o.seed / 2;
+    const int n = (int)(tables ? o.end : o.fwd) / 2 - skip;
+    for (int k0 = tid; k0 < n; k0 += 8 * nthreads) {
+        v2d v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = k0 + u * nthreads;
+            if (k < n)
+                v[u] = src[k < cut ? k : k + skip];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = k0 + u * nthreads;
+            if (k < n)
+                dst[k] = v[u];
+        }
     }
 }
 
@@ -1356,6 +1351,17 @@ inline bool configure_launch(const DevModel &m, int n, int num_cus, int wcap, si
         return false;
     cfg.lds_tables = table_pref < 0 ? wt > 0 && wt >= wg : table_pref == 1 && wt > 0;
     cfg.waves = cfg.lds_tables ? wt : wg;
+    // Few atoms: as many waves per workgroup as give every CU one workgroup
+    // and every wave the same number of atoms (a wave alone on its SIMD is
+    // faster than three sharing one), at least one wave per SIMD: a
+    // workgroup's table copy then stays one round trip (one wave at least
+    // measured the same at 40 to 10,000 atoms).  E/F/S, level 16, full
+    // workgroups -> this rule with the packed table copy: 997 atoms 29.3 ->
+    // 18.2 us, 4,000 atoms with a head 58 -> 49 us; from 3,072 atoms times a
+    // few on the two shapes are the same.
+    const int rounds = (std::max(n, 1) + num_cus * cfg.waves - 1) / (num_cus * cfg.waves);
+    const int even = (std::max(n, 1) + num_cus * rounds - 1) / (num_cus * rounds);
+    cfg.waves = std::min(cfg.waves, std::max(4, even));
     cfg.lds_bytes = shared_doubles(m, cfg.lds_tables, seeds) * sizeof(double) + cfg.waves * priv;
     const int per_cu = std::max<int>(1, (int)(lds_limit / cfg.lds_bytes));
     const int need = (std::max(n, 1) + cfg.waves - 1) / cfg.waves;

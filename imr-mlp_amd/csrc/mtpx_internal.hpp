@@ -377,6 +377,7 @@ struct DevModel {
     int numax_all;
     int ndup;
     int nfwd, nbwd;  // levels
+    const double *shared;   // the packed tables below (SharedOffsets)
     const double *radial;   // [Z*Z*M*R]
     const double *species;  // [Z]
     const double *moment;   // [S]
@@ -406,6 +407,29 @@ struct DevModel {
     const int2 *fwd_steps;      // device_steps
     const int *bwd_level_step;  // [nbwd+1]
     const int2 *bwd_steps;
+};
+
+// The block-shared model tables (offsets in doubles, every part a multiple of
+// 16 bytes): radial coefficients | adjoint seeds | moment coefficients | map |
+// slot_basic | force_basic | mono_tab | forward | reverse step tables.  The
+// device keeps them packed in this order (DevModel::shared), so a workgroup
+// copies them into LDS as one block.
+struct SharedOffsets {
+    size_t coef, seed, moment, map, slot, force, mono, fwd, bwd, end;
+    __host__ __device__ explicit SharedOffsets(const DevModel &m)
+    {
+        auto four = [](int n) { return ((size_t)n + 3) & ~size_t(3); };
+        coef = 0;
+        seed = four(m.Z * m.Z * m.M * m.R);
+        moment = seed + m.K4;
+        map = moment + four(m.S);
+        slot = map + four(m.S) / 2;
+        force = slot + four(m.nslots) / 2;
+        mono = force + four(m.nforce) / 2;
+        fwd = mono + (size_t)m.nmono / 4;
+        bwd = fwd + (size_t)m.fwd_nsteps * kWave;
+        end = bwd + (size_t)m.bwd_nsteps * kWave;
+    }
 };
 
 // Neighbour lists resident on the device (SoA).
