@@ -88,7 +88,7 @@ int upload_coeffs(mtpx_context *ctx)
 // Sizes and work-space offsets of the device view (no device pointers) and
 // the moment tables of its kernel profile.
 void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm,
-                      std::vector<unsigned short> &mono)
+                      std::vector<unsigned short> &mono, std::vector<unsigned> &shift)
 {
     dm.Z = M.Z;
     dm.M = M.M;
@@ -133,7 +133,7 @@ void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm,
     dm.rb_general = M.general_basis() ? 1 : 0;
     dm.rb_table = nullptr;
     std::memcpy(dm.slot_base, P.slot_base, sizeof dm.slot_base);
-    moment_table(M, P, efs_profile_degree(dm), mono, dm.mono_groups);
+    moment_table(M, P, efs_profile_degree(dm), mono, shift, dm.mono_groups);
     dm.nmono = (int)mono.size();
     dm.fwd_nsteps = (int)(P.fwd_steps.size() / (2 * kWave));
     dm.bwd_nsteps = (int)(P.bwd_steps.size() / (2 * kWave));
@@ -151,7 +151,8 @@ int install_model(mtpx_context *ctx, Model &&m)
     // CU's LDS is refused before anything of the context changes.
     DevModel dm{};
     std::vector<unsigned short> mono;
-    fill_model_sizes(m, p, dm, mono);
+    std::vector<unsigned> shift;
+    fill_model_sizes(m, p, dm, mono, shift);
     EfsLaunch probe;
     if (!efs_configure(dm, 1, 1, 0, ctx->lds_limit, probe))
         return set_error(ctx, MTPX_E_CAPACITY, "model needs more LDS than a CU provides");
@@ -180,6 +181,7 @@ int install_model(mtpx_context *ctx, Model &&m)
     pack(o.fwd, device_steps(P.fwd_steps, P.fwd_level_step, P.fwd_comb, P.fwd_level_comb));
     pack(o.bwd, device_steps(P.bwd_steps, P.bwd_level_step, P.bwd_comb, P.bwd_level_comb));
     HIP_TRY(upload(ctx->shared, packed, s), "upload model");
+    HIP_TRY(upload(ctx->mono_shift, shift, s), "upload model");
     HIP_TRY(upload(ctx->dup, P.dup, s), "upload model");
     HIP_TRY(upload(ctx->fwd_level, P.fwd_level_step, s), "upload model");
     HIP_TRY(upload(ctx->bwd_level, P.bwd_level_step, s), "upload model");
@@ -231,6 +233,7 @@ int install_model(mtpx_context *ctx, Model &&m)
     dm.mono_tab = reinterpret_cast<unsigned short *>(base + o.mono);
     dm.fwd_steps = reinterpret_cast<int2 *>(base + o.fwd);
     dm.bwd_steps = reinterpret_cast<int2 *>(base + o.bwd);
+    dm.mono_shift = ctx->mono_shift.as<unsigned>();
     dm.dup = ctx->dup.as<int>();
     dm.fwd_level_step = ctx->fwd_level.as<int>();
     dm.bwd_level_step = ctx->bwd_level.as<int>();

@@ -27,7 +27,7 @@ struct mtpx_context {
     Plan plan;
     DevModel dm{};
     // model buffers
-    DBuf shared, species, dup, fwd_level, bwd_level, rb_table;
+    DBuf shared, species, mono_shift, dup, fwd_level, bwd_level, rb_table;
     // MTP-M head tables and the DevHead that points at them
     DBuf head_ids, head_proj, head_dsp, head_coef, head_params;
 
@@ -122,7 +122,7 @@ struct mtpx_context {
 
     ~mtpx_context()
     {
-        for (DBuf *b : {&shared, &species, &dup, &fwd_level, &bwd_level, &rb_table,
+        for (DBuf *b : {&shared, &species, &mono_shift, &dup, &fwd_level, &bwd_level, &rb_table,
                         &head_ids, &head_proj, &head_dsp, &head_coef, &head_params, &offsets, &idx, &type, &x, &y, &z, &d,
                         &center_type, &rev_offsets, &rev_pairs, &forces, &site_energy, &partial,
                         &pair_ders, &out10, &soff, &center_structure, &site_virial, &benergy,

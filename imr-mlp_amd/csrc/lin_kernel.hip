@@ -70,16 +70,6 @@ __device__ __forceinline__ double readlane_d(double v, int l)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// Compile-time loop: f(integral_constant<int, I>) for I in [B, E).
-template <int B, int E, class F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
-
 // The monomials of degree NU from those of degree NU - 1.
 template <int NU, int MMAX>
 __device__ __forceinline__ void next_shell(const double *prev, double *cur, const Nbr<MMAX> &q)

@@ -1061,11 +1061,11 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     const bool over_adjoints = 2 * (p.red0 - K4) >= RB;
     p.tr_red1 = over_adjoints ? 2 * K4 : red_region();
     p.tr_red4 = over_adjoints ? 2 * K4 : red_region();
-    if (N4 <= K4) {
+    if (F4 <= K4) {
         p.tr_stage = 0;
     } else {
         p.tr_stage = end;
-        end += 2 * N4;
+        end += 2 * F4;
     }
     p.tr_priv = end;
     return true;
@@ -1100,42 +1100,53 @@ std::vector<int> device_steps(const std::vector<int> &steps, const std::vector<i
 }
 
 void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
-                  unsigned &groups)
+                  std::vector<unsigned> &shift, unsigned &groups)
 {
     tab.clear();
+    shift.clear();
     groups = 0;
     std::vector<std::array<int, 3>> mono;
     for (int c = 0; c <= nu; ++c)
         for (int b = 0; b <= nu - c; ++b)
             for (int a = 0; a <= nu - c - b; ++a)
                 mono.push_back({a, b, c});
+    // the basic (mu, a, b, c), 0xffff where there is none
+    auto basic = [&](int mu, int a, int b, int c) -> unsigned {
+        const int n = a + b + c;
+        if (mu >= m.M || n > p.numax[mu])
+            return 0xffff;
+        // position in the slot order: a = n..0, b = n-a..0
+        int pos = 0;
+        for (int ap = n; ap > a; --ap)
+            pos += n - ap + 1;
+        const int i = p.slot_basic[p.slot_base[n * kMaxMu + mu] + pos + (n - a - b)];
+        return i < 0 ? 0xffff : (unsigned)i;
+    };
     for (size_t ch = 0; ch * kChunk < mono.size(); ++ch)
         for (int g = 0; 4 * g < m.M; ++g) {
             std::vector<unsigned short> t(kWave, 0xffff);
+            std::vector<unsigned> s(3 * kWave, 0xffff);
             bool any = false;
             for (int l = 0; l < kWave; ++l) {
                 const int mu = 4 * g + l / kChunk;
                 const size_t e = ch * kChunk + l % kChunk;
-                if (mu >= m.M || e >= mono.size())
+                if (e >= mono.size())
                     continue;
-                const int a = mono[e][0], b = mono[e][1], c = mono[e][2], n = a + b + c;
-                if (n > p.numax[mu])
-                    continue;
-                // position in the slot order: a = n..0, b = n-a..0
-                int pos = 0;
-                for (int ap = n; ap > a; --ap)
-                    pos += n - ap + 1;
-                const int basic = p.slot_basic[p.slot_base[n * kMaxMu + mu] + pos + (n - a - b)];
-                if (basic >= 0) {
-                    t[l] = (unsigned short)basic;
-                    any = true;
-                }
+                const int a = mono[e][0], b = mono[e][1], c = mono[e][2];
+                t[l] = (unsigned short)basic(mu, a, b, c);
+                s[l] = basic(mu, a + 1, b, c) | (unsigned)(a + 1) << 16;
+                s[kWave + l] = basic(mu, a, b + 1, c) | (unsigned)(b + 1) << 16;
+                s[2 * kWave + l] = basic(mu, a, b, c + 1) | (unsigned)(c + 1) << 16;
+                // (a moment structure may lack a basic below one it has)
+                any = any || t[l] != 0xffff || (s[l] & 0xffff) != 0xffff ||
+                      (s[kWave + l] & 0xffff) != 0xffff || (s[2 * kWave + l] & 0xffff) != 0xffff;
             }
             // (the first group's tables are all there: the compile-time
             // profiles take every chunk for it)
             if (any || g == 0) {
                 groups |= 1u << (2 * ch + g);
                 tab.insert(tab.end(), t.begin(), t.end());
+                shift.insert(shift.end(), s.begin(), s.end());
             }
         }
 }

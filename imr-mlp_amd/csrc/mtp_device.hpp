@@ -10,6 +10,16 @@
 namespace mtpx {
 namespace {
 
+// Compile-time loop: f(integral_constant<int, I>) for I in [B, E).
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
+}
+
 constexpr int shell_size(int nu) { return (nu + 1) * (nu + 2) / 2; }
 
 // Position of (a, b, c = nu-a-b) in the shell enumeration a = nu..0, b = nu-a..0.
@@ -612,6 +622,46 @@ __device__ __forceinline__ void load_neighbor(const DevModel &m, const DevNeighb
 constexpr int mono_count(int nu) { return (nu + 1) * (nu + 2) * (nu + 3) / 6; }
 constexpr int mono_chunks(int nu) { return (mono_count(nu) + kChunk - 1) / kChunk; }
 
+// The exponents of monomial e.
+struct MonoPowers {
+    int a, b, c;
+};
+constexpr MonoPowers mono_powers(int nu, int e)
+{
+    for (int c = 0; c <= nu; ++c)
+        for (int b = 0; b <= nu - c; ++b) {
+            const int n = nu - c - b + 1;
+            if (e < n)
+                return {e, b, c};
+            e -= n;
+        }
+    return {0, 0, 0};
+}
+// f(integral_constant e, value) for every monomial of degree <= NU, in order.
+template <int NU, class F>
+__device__ __forceinline__ void for_monomials(double x, double y, double z, F f)
+{
+    double zc = 1.0, yz = 1.0, v = 1.0;
+    static_for<0, mono_count(NU)>([&](auto E) __attribute__((always_inline)) {
+        constexpr int e = decltype(E)::value;
+        constexpr MonoPowers p = mono_powers(NU, e);
+        if constexpr (e > 0) {
+            if constexpr (p.a > 0) {
+                v *= x;
+            } else {
+                if constexpr (p.b > 0) {
+                    yz *= y;
+                } else {
+                    zc *= z;
+                    yz = zc;
+                }
+                v = yz;
+            }
+        }
+        f(E, v);
+    });
+}
+
 // Bit g: the chunk holds a moment of radial functions 4 g .. 4 g + 3.  The
 // run-time profiles read the masks of the table (Plan::mono_groups); a
 // compile-time profile's radial functions past the fourth reach degree 0
@@ -625,6 +675,18 @@ __device__ __forceinline__ unsigned mono_groups(const DevModel &m, int ch)
     } else {
         return (m.mono_groups >> (2 * ch)) & 3u;
     }
+}
+
+// Position of the chunk's table of group g (chunk after chunk, its groups in
+// order).
+template <class P>
+__device__ __forceinline__ int mono_entry(const DevModel &m, int ch, int g)
+{
+    if constexpr (P::exact)
+        return ch + (P::M > 4 && ch > 0 ? 1 : 0) + g;
+    else
+        return __builtin_popcount(m.mono_groups & ((1u << (2 * ch)) - 1u)) +
+               (g ? (int)(m.mono_groups >> (2 * ch) & 1u) : 0);
 }
 
 // One 8-byte LDS read; volatile keeps the compiler from pairing reads into
@@ -708,30 +770,15 @@ __device__ __forceinline__ void add_moments(const DevModel &m, double *red,
             af[g][s] = lds_read(a + 4 * s);
     }
     wave_sync();
-    double zc = 1.0;
-    int e = 0;
-#pragma unroll
-    for (int c = 0; c <= P::NUMAX; ++c) {
-        double yz = zc;
-#pragma unroll
-        for (int b = 0; b <= P::NUMAX - c; ++b) {
-            double v = yz;
-#pragma unroll
-            for (int a = 0; a <= P::NUMAX - c - b; ++a) {
-                lds_write(red + (e % kChunk) * kRedStride + lane, v);
-                ++e;
-                if (e % kChunk == 0 || e == mono_count(P::NUMAX)) {
-                    const int ch = (e - 1) / kChunk;
-                    const unsigned groups = mono_groups<P>(m, ch);
-                    moment_chunk<G>(red, af, groups, tab, cnt, mom, lane);
-                    tab += kWave * __builtin_popcount(groups);
-                }
-                v *= q.ux;
-            }
-            yz *= q.uy;
+    for_monomials<P::NUMAX>(q.ux, q.uy, q.uz, [&](auto E, double v) __attribute__((always_inline)) {
+        constexpr int e = decltype(E)::value, ch = e / kChunk;
+        lds_write(red + (e % kChunk) * kRedStride + lane, v);
+        if constexpr (e % kChunk == kChunk - 1 || e == mono_count(P::NUMAX) - 1) {
+            const unsigned groups = mono_groups<P>(m, ch);
+            moment_chunk<G>(red, af, groups, tab, cnt, mom, lane);
+            tab += kWave * __builtin_popcount(groups);
         }
-        zc *= q.uz;
-    }
+    });
 }
 
 // ---- force polynomials ---------------------------------------------------

@@ -318,9 +318,9 @@ bool build_plan(const Model &m, Plan &p, std::string &err);
 std::vector<int> device_steps(const std::vector<int> &steps, const std::vector<int> &level_step,
                               const std::vector<int> &comb, const std::vector<int> &level_comb);
 // The moment tables of a kernel profile whose monomials reach degree nu
-// (numbered by c, b, a, a fastest): see DevModel::mono_tab.
+// (numbered by c, b, a, a fastest): see DevModel::mono_tab, mono_shift.
 void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
-                  unsigned &groups);
+                  std::vector<unsigned> &shift, unsigned &groups);
 
 // Linear-fit plan (sparse Jacobian of the scalar moments w.r.t. the basic
 // moments, see build_lin_plan).  Work space per wave (doubles): the E/F/S
@@ -392,6 +392,9 @@ struct DevModel {
     int nmono;
     unsigned mono_groups;
     const unsigned short *mono_tab;  // [nmono]
+    // per table entry, for x, y and z: the basic whose monomial has one power
+    // more (0xffff: none) | that power << 16 (training)
+    const unsigned *mono_shift;      // [nmono / 64][3][64]
     const int *dup;         // [ndup][2]
     int K4, dummy, red0, priv_doubles;  // per-wave work space (Plan)
     int tr_red1, tr_red4, tr_stage, tr_grad, tr_ctype, tr_priv;

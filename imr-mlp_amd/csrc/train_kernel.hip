@@ -17,8 +17,8 @@
 // The gradient kernel runs one wave per atom, like the E/F/S kernel, in
 // directional form instead of forming the reference's per-pair Jacobians:
 //   1. lanes over neighbours: basic moments m_b = sum_j f Y and their
-//      tangents along W, q_b = sum_j W_j . grad_r(f Y), reduced together
-//      through the transpose buffer;
+//      tangents along W, q_b = sum_j W_j . grad_r(f Y), summed on the matrix
+//      cores (add_dual_moments);
 //   2. the product rules carry (m, Q) forward: Q_o += c (Q_l m_r + m_l Q_r);
 //      then dG/dxi_s = dLdE m_map(s) + Q_map(s);
 //   3. reverse rules carry (A, Gb) with seeds (xi, dLdE xi):
@@ -29,8 +29,9 @@
 //      function mu,
 //        dG/dc[ti,tj,mu,k] += alpha Q_k + beta Q'_k,
 //        alpha = H - (w_u/d) V + Wg/d,  beta = w_u U,  w_u = W . u,
-//      summed over the neighbours of species tj by a typed transpose
-//      reduction into the wave's gradient accumulator.
+//      from the value and gradient of two polynomials per radial function by
+//      nested Horner, summed over the neighbours of each species on the
+//      matrix cores into the wave's gradient accumulator.
 // Each wave accumulates over its atoms in LDS and writes one gradient row;
 // the rows are summed in a fixed order, so the gradient is repeatable bit
 // for bit for a given launch shape.
@@ -172,77 +173,6 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const double *rows, in
 
 // ---- gradient kernel ---------------------------------------------------
 
-// First slot of the (nu, mu) block in the canonical slot order.
-template <class P>
-__device__ __forceinline__ int slot_base(const DevModel &m, int nu, int mu)
-{
-    if constexpr (P::exact) {
-        int s = 0;
-        for (int n = 0; n < nu; ++n)
-            for (int q = 0; q < P::M; ++q)
-                if (P::nm[q] >= n)
-                    s += shell_size(n);
-        for (int q = 0; q < mu; ++q)
-            if (P::nm[q] >= nu)
-                s += shell_size(nu);
-        return s;
-    } else {
-        return m.slot_base[nu * kMaxMu + mu];
-    }
-}
-
-// Transpose-buffer reduction of `nrows` rows; tgt(row, sum) for each row.
-template <class Tgt>
-__device__ __forceinline__ void reduce_rows(const double *red, int nrows, int row0, int lane,
-                                            Tgt tgt)
-{
-    wave_sync();
-    const double acc = chunk_row_sum(red, lane);
-    if (lane < nrows)
-        tgt(row0 + lane, acc);
-    wave_sync();
-}
-
-// As reduce_rows, with one sum per neighbour species: column j counts for
-// species ctype[j] (-1: no neighbour).
-template <class Tgt>
-__device__ __forceinline__ void reduce_rows_typed(const double *red, int nrows, int row0,
-                                                  int lane, const int *ctype, int Z, Tgt tgt)
-{
-    wave_sync();
-    const double2 *row = reinterpret_cast<const double2 *>(red + (lane & (kChunk - 1)) * kRedStride +
-                                                           (lane >> 4) * 16);
-    const int4 *ty = reinterpret_cast<const int4 *>(ctype + (lane >> 4) * 16);
-    double v[16];
-    int t[16];
-#pragma unroll
-    for (int jj = 0; jj < 8; ++jj) {
-        const double2 x = row[jj];
-        v[2 * jj] = x.x;
-        v[2 * jj + 1] = x.y;
-    }
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-        const int4 x = ty[jj];
-        t[4 * jj] = x.x;
-        t[4 * jj + 1] = x.y;
-        t[4 * jj + 2] = x.z;
-        t[4 * jj + 3] = x.w;
-    }
-    for (int tj = 0; tj < Z; ++tj) {
-        double a0 = 0.0, a1 = 0.0;
-#pragma unroll
-        for (int jj = 0; jj < 16; jj += 2) {
-            a0 += t[jj] == tj ? v[jj] : 0.0;
-            a1 += t[jj + 1] == tj ? v[jj + 1] : 0.0;
-        }
-        const double acc = xor16_sum(xor32_sum(a0 + a1));
-        if (lane < nrows)
-            tgt(row0 + lane, tj, acc);
-    }
-    wave_sync();
-}
-
 struct GradNbr {
     double wx, wy, wz, wu;  // W_ij and W_ij . u
 };
@@ -272,120 +202,314 @@ __device__ __forceinline__ GradNbr pair_weight(const DevNeighbors &nb, const Tra
     return g;
 }
 
-// Rows of the first pass alternate m and q of one slot; the sums go to the
-// pair of the slot's basic moment (m at 2b, q at 2b + 1).
-struct DualCtx {
-    double *red, *ws;
-    const int *slot_basic;
-    int lane, row;
+// Step 1.  With h = f' w_u and t = (f / d) (W - w_u u), the tangent of a basic
+// moment is
+//   q_abc = sum_j [h Y_abc + t . grad_u Y_abc]
+//         = H_abc + a X_(a-1)bc + b Y_a(b-1)c + c Z_ab(c-1)
+// with H, X, Y, Z the sums of h, t_x, t_y, t_z times the monomials: five
+// products of neighbour values and monomials (f gives the moments), formed
+// on the matrix cores as in add_moments from one transpose of the monomials,
+// and the factors a, b, c applied once per atom instead of once per
+// neighbour.  Sums go to the pairs {m, q} with LDS adds: tab as add_moments,
+// shift (m.mono_shift, from global memory) the basic moment and factor that a
+// gradient sum adds to.
+template <class P>
+__device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red,
+                                                 const unsigned short *tab, unsigned base,
+                                                 const Nbr<P::M> &q, const GradNbr &g, int cnt,
+                                                 int lane)
+{
+    constexpr int G = (P::M + 3) / 4, S = kWave / 4;
+    const double tx = (g.wx - g.wu * q.ux) * q.invd, ty = (g.wy - g.wu * q.uy) * q.invd,
+                 tz = (g.wz - g.wu * q.uz) * q.invd;
+#pragma unroll
+    for (int grp = 0; grp < G; ++grp) {
+        // neighbour values of four radial functions: f, h, t_x, t_y, t_z
+        constexpr int T = 5;
+        double af[T][S];
+        auto take = [&](int t0, int n) {
+            wave_sync();
+#pragma unroll
+            for (int t = t0; t < t0 + n; ++t) {
+                const double *a = red + (4 * (t - t0) + (lane & 3)) * kRedStride + (lane >> 4);
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    af[t][s] = lds_read(a + 4 * s);
+            }
+            wave_sync();
+        };
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int mu = 4 * grp + k < P::M ? 4 * grp + k : P::M - 1;
+            lds_write(red + k * kRedStride + lane, q.f[mu]);
+            lds_write(red + (4 + k) * kRedStride + lane, q.fd[mu] * g.wu);
+            lds_write(red + (8 + k) * kRedStride + lane, q.f[mu] * tx);
+            lds_write(red + (12 + k) * kRedStride + lane, q.f[mu] * ty);
+        }
+        take(0, 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int mu = 4 * grp + k < P::M ? 4 * grp + k : P::M - 1;
+            lds_write(red + k * kRedStride + lane, q.f[mu] * tz);
+        }
+        take(4, 1);
+        // (functions of degree 0 have no gradient sums)
+        bool grads = true;
+        if constexpr (P::exact)
+            grads = P::nm[4 * grp] > 0;
+        auto chunk = [&](int entry) __attribute__((always_inline)) {
+            wave_sync();
+            unsigned sh[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                sh[t] = m.mono_shift[(3 * entry + t) * kWave + lane];
+            const double *b = red + (lane & (kChunk - 1)) * kRedStride + (lane >> 4);
+            double v[S], s0[T], s1[T];
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                v[s] = lds_read(b + 4 * s);
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                s0[t] = s1[t] = 0.0;
+#pragma unroll
+            for (int k = 0; k < S; k += 4)
+                if (4 * k < cnt) {
+#pragma unroll
+                    for (int s = k; s < k + 4; s += 2)
+#pragma unroll
+                        for (int t = 0; t < T; ++t)
+                            if (t < 2 || grads) {
+                                s0[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(af[t][s], v[s], s0[t],
+                                                                           0, 0, 0);
+                                s1[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(
+                                    af[t][s + 1], v[s + 1], s1[t], 0, 0, 0);
+                            }
+                }
+            const unsigned w = tab[entry * kWave + lane];
+            if (w != 0xffffu) {
+                lds_add(base + 16 * w, s0[0] + s1[0]);
+                lds_add(base + 16 * w + 8, s0[1] + s1[1]);
+            }
+            if (grads)
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    const unsigned w2 = sh[t] & 0xffffu;
+                    if (w2 != 0xffffu)
+                        lds_add(base + 16 * w2 + 8,
+                                (double)(int)(sh[t] >> 16) * (s0[2 + t] + s1[2 + t]));
+                }
+            wave_sync();
+        };
+        for_monomials<P::NUMAX>(
+            q.ux, q.uy, q.uz, [&](auto E, double v) __attribute__((always_inline)) {
+                constexpr int e = decltype(E)::value;
+                if (mono_groups<P>(m, e / kChunk) >> grp & 1) {
+                    lds_write(red + (e % kChunk) * kRedStride + lane, v);
+                    if constexpr (e % kChunk == kChunk - 1 || e == mono_count(P::NUMAX) - 1)
+                        chunk(mono_entry<P>(m, e / kChunk, grp));
+                }
+            });
+    }
+}
+
+// Step 4: the force polynomials' scheme (poly_grad) over the staged pairs
+// {A, G}: value and gradient of the A polynomial and value of the G one.
+struct PolyPair {
+    PolyGrad a;
+    double g;
 };
-
-// Powers u_x^k, u_y^k, u_z^k for k = 0 .. N: every monomial of every shell
-// is a product of three of them, so the passes below hold 3 (N + 1) values
-// per lane instead of two whole shells (at level 20, 27 doubles against 81),
-// which lets the kernel run two waves per SIMD.
-template <int N, int MMAX>
-__device__ __forceinline__ void unit_powers(const Nbr<MMAX> &q, double *px, double *py, double *pz)
-{
-    px[0] = py[0] = pz[0] = 1.0;
+template <int kCount>
+struct PairStream {
+    unsigned at;
+    v2d buf[2][4];
+    __device__ __forceinline__ void load(int block)
+    {
 #pragma unroll
-    for (int k = 1; k <= N; ++k) {
-        px[k] = px[k - 1] * q.ux;
-        py[k] = py[k - 1] * q.uy;
-        pz[k] = pz[k - 1] * q.uz;
+        for (int k = 0; k < 4; ++k)
+            if (4 * block + k < kCount)
+                buf[block & 1][k] = ((lds_v2d)(uintptr_t)at)[4 * block + k];
     }
+    __device__ __forceinline__ PairStream(const double2 *AG, double &tie)
+        : at(lds_address(reinterpret_cast<const double *>(AG)))
+    {
+        asm volatile("" : "+v"(at), "+v"(tie));
+        load(0);
+    }
+    __device__ __forceinline__ v2d next(int e, double &v, double &w)
+    {
+        if (e % 4 == 0 && e + 4 < kCount) {
+            asm volatile("" : "+v"(at), "+v"(v), "+v"(w));
+            load(e / 4 + 1);
+        }
+        return buf[(e / 4) & 1][e % 4];
+    }
+};
+template <int N>
+__device__ __forceinline__ PolyPair poly_pair(const double2 *AG, double x, double y, double z,
+                                              double &tie)
+{
+    PairStream<mono_count(N)> c(AG, tie);
+    PolyGrad g{0, 0, 0, 0};
+    double h = 0;
+    int e = 0;
+#pragma unroll
+    for (int a = N; a >= 0; --a) {
+        double q = 0, qy = 0, qz = 0, qh = 0;
+#pragma unroll
+        for (int b = N - a; b >= 0; --b) {
+            const v2d first = a < N && b == N - a ? c.next(e, g.p, h) : c.next(e, q, qh);
+            double r = first.x, rz = 0, rh = first.y;
+            ++e;
+#pragma unroll
+            for (int k = N - a - b - 1; k >= 0; --k) {
+                const v2d v = c.next(e, r, rh);
+                ++e;
+                rz = k == N - a - b - 1 ? r : fma(rz, z, r);
+                r = fma(r, z, v.x);
+                rh = fma(rh, z, v.y);
+            }
+            if (b == N - a) {
+                q = r;
+                qz = rz;
+                qh = rh;
+            } else {
+                qy = b == N - a - 1 ? q : fma(qy, y, q);
+                qz = fma(qz, y, rz);
+                q = fma(q, y, r);
+                qh = fma(qh, y, rh);
+            }
+            asm volatile("" : "+v"(q), "+v"(qy), "+v"(qz), "+v"(qh));
+        }
+        if (a == N) {
+            g = PolyGrad{q, 0, qy, qz};
+            h = qh;
+        } else {
+            g.x = a == N - 1 ? g.p : fma(g.x, x, g.p);
+            g.y = fma(g.y, x, qy);
+            g.z = fma(g.z, x, qz);
+            g.p = fma(g.p, x, q);
+            h = fma(h, x, qh);
+        }
+        asm volatile("" : "+v"(g.p), "+v"(g.x), "+v"(g.y), "+v"(g.z), "+v"(h));
+    }
+    return PolyPair{g, h};
+}
+template <int N, int NMAX>
+__device__ __forceinline__ PolyPair poly_pair_of(int nu, const double2 *AG, double x, double y,
+                                                 double z, double &tie)
+{
+    if constexpr (N < NMAX)
+        if (nu > N)
+            return poly_pair_of<N + 1, NMAX>(nu, AG, x, y, z, tie);
+    return poly_pair<N>(AG, x, y, z, tie);
 }
 
-// W . grad_u Y_abc = a W_x Y_(a-1)bc + b W_y Y_a(b-1)c + c W_z Y_ab(c-1),
-// with the weights (wx, wy, wz) as given
-template <int NU>
-__device__ __forceinline__ double grad_u_dot(int a, int b, const double *px, const double *py,
-                                             const double *pz, double wx, double wy, double wz)
+// alpha_mu and beta_mu of one neighbour into rows mu and kMaxMu + mu of the
+// transpose buffer:
+//   alpha = p_G + (1 / d) (W - w_u u) . grad p_A,  beta = w_u p_A
+struct RadialRows {
+    double *red;
+    int lane;
+    double tx, ty, tz, wu, win, tie;
+    __device__ __forceinline__ void put(int mu, const PolyPair &p)
+    {
+        const double al = fma(tx, p.a.x, fma(ty, p.a.y, fma(tz, p.a.z, p.g)));
+        lds_write(red + mu * kRedStride + lane, al * win);
+        lds_write(red + (kMaxMu + mu) * kRedStride + lane, wu * p.a.p * win);
+    }
+};
+template <class P, int MU = 0, int OFF = 0>
+__device__ __forceinline__ void radial_rows_exact(const double2 *AG, const Nbr<P::M> &q,
+                                                  RadialRows &r)
 {
-    const int c = NU - a - b;
-    double gy = 0.0;
-    if (a > 0)
-        gy = fma(a * wx, px[a - 1] * (py[b] * pz[c]), gy);
-    if (b > 0)
-        gy = fma(b * wy, px[a] * (py[b - 1] * pz[c]), gy);
-    if (c > 0)
-        gy = fma(c * wz, px[a] * (py[b] * pz[c - 1]), gy);
-    return gy;
+    r.put(MU, poly_pair<P::nm[MU]>(AG + OFF, q.ux, q.uy, q.uz, r.tie));
+    if constexpr (MU + 1 < P::M)
+        radial_rows_exact<P, MU + 1, OFF + force_size(P::nm[MU])>(AG, q, r);
 }
 
-// Step 1: per (nu, mu) block, rows m = f Y and q = W . grad_r(f Y)
-//   = Y (f' - nu f/d) w_u + (f/d) W . grad_u Y.
-template <int NU, class P>
-__device__ __forceinline__ void fwd_dual_shells(const DevModel &m, DualCtx &cx,
-                                                const Nbr<P::M> &q, const GradNbr &g,
-                                                const double *px, const double *py,
-                                                const double *pz)
+// Step 4 of one batch: the radial gradient
+//   grad[tj][mu][k] += sum_j [t_j = tj] (alpha_mu Q_k + beta_mu Q'_k),
+// per mu the product of four species' masked alphas (betas) with the basis
+// functions on the matrix cores (rows species, columns k).
+template <class P>
+__device__ __forceinline__ void add_radial_gradient(const DevModel &m, double *red, int *ctype,
+                                                    const double2 *AG, double *grad, int MR,
+                                                    int ti, int tj, double win,
+                                                    const Nbr<P::M> &q, const GradNbr &g, int cnt,
+                                                    int lane)
 {
-    auto flush = [&]() {
-        reduce_rows(cx.red, kChunk, cx.row - kChunk, cx.lane, [&](int r, double acc) {
-            const int b = cx.slot_basic[r >> 1];
-            if (b >= 0)
-                cx.ws[2 * b + (r & 1)] += acc;
-        });
-    };
+    constexpr int S = kWave / 4;
+    const int R = P::exact ? P::RMAX : m.R;
+    double bq[2][S];
+    {
+        double Q[2][P::RMAX];
+        radial_basis<P>(m, ti, tj, q.d, Q[0], Q[1]);
+        ctype[lane] = tj;
+        // (columns past the basis size hold what the buffer held: their sums
+        // are not used)
+        const double *b = red + (lane & (kChunk - 1)) * kRedStride + (lane >> 4);
 #pragma unroll
-    for (int mu = 0; mu < P::M; ++mu) {
-        if (P::active(m, mu, NU)) {
-            __builtin_amdgcn_sched_barrier(0);
-            const double hw = (q.fd[mu] - NU * q.f[mu] * q.invd) * g.wu;
-            const double fd = q.f[mu] * q.invd;
+        for (int t = 0; t < 2; ++t) {
 #pragma unroll
-            for (int a = NU; a >= 0; --a)
+            for (int k = 0; k < P::RMAX; ++k)
+                lds_write(red + k * kRedStride + lane, Q[t][k]);
+            wave_sync();
 #pragma unroll
-                for (int b = NU - a; b >= 0; --b) {
-                    const double y = px[a] * (py[b] * pz[NU - a - b]);
-                    const double gy = grad_u_dot<NU>(a, b, px, py, pz, g.wx, g.wy, g.wz);
-                    cx.red[(cx.row % kChunk) * kRedStride + cx.lane] = q.f[mu] * y;
-                    ++cx.row;
-                    cx.red[(cx.row % kChunk) * kRedStride + cx.lane] = hw * y + fd * gy;
-                    ++cx.row;
-                    if (cx.row % kChunk == 0)
-                        flush();
-                }
+            for (int s = 0; s < S; ++s)
+                bq[t][s] = lds_read(b + 4 * s);
+            wave_sync();
         }
     }
-    if constexpr (NU < P::NUMAX) {
-        if (P::deeper(m, NU))
-            fwd_dual_shells<NU + 1, P>(m, cx, q, g, px, py, pz);
-    }
-}
-
-// Step 4, all radial functions at once, monomial by monomial with the
-// radial functions innermost: per mu, alpha_mu (without its beta-like
-// term) and U_mu,
-//   alpha += G Y + A (W/d . grad_u Y - nu (w_u/d) Y),  U += A Y.
-template <int NU, class P>
-__device__ __forceinline__ void rad_shells(const DevModel &m, const double2 *AG,
-                                           const double *px, const double *py, const double *pz,
-                                           const GradNbr &g, double invd, double *alpha,
-                                           double *U)
-{
-    const double ncw = -NU * g.wu * invd;
-    const double wxd = g.wx * invd, wyd = g.wy * invd, wzd = g.wz * invd;
+    int ty[S];
 #pragma unroll
-    for (int a = NU; a >= 0; --a)
-#pragma unroll
-        for (int b = NU - a; b >= 0; --b) {
-            const int i = shell_index(NU, a, b);
-            const double y = px[a] * (py[b] * pz[NU - a - b]);
-            const double t = fma(ncw, y, grad_u_dot<NU>(a, b, px, py, pz, wxd, wyd, wzd));
-#pragma unroll
-            for (int mu = 0; mu < P::M; ++mu)
-                if (P::active(m, mu, NU)) {
-                    const double2 w = AG[slot_base<P>(m, NU, mu) + i];  // {A, G}, LDS broadcast
-                    U[mu] = fma(w.x, y, U[mu]);
-                    alpha[mu] = fma(w.y, y, fma(w.x, t, alpha[mu]));
-                }
+    for (int s = 0; s < S; ++s)
+        ty[s] = ctype[4 * s + (lane >> 4)];
+    RadialRows r{red, lane, (g.wx - g.wu * q.ux) * q.invd, (g.wy - g.wu * q.uy) * q.invd,
+                 (g.wz - g.wu * q.uz) * q.invd, g.wu, win, 0.0};
+    if constexpr (P::exact) {
+        radial_rows_exact<P>(AG, q, r);
+    } else {
+#pragma unroll 1
+        for (int mu = 0; mu < m.M; ++mu) {
+            const int nu = m.numax[mu];
+            if (nu < 0) {
+                r.put(mu, PolyPair{{0, 0, 0, 0}, 0});
+                continue;
+            }
+            r.put(mu, poly_pair_of<0, P::NUMAX>(nu, AG, q.ux, q.uy, q.uz, r.tie));
+            AG += force_size(nu);
         }
-    if constexpr (NU < P::NUMAX) {
-        if (P::deeper(m, NU))
-            rad_shells<NU + 1, P>(m, AG, px, py, pz, g, invd, alpha, U);
     }
+    wave_sync();
+#pragma unroll 1
+    for (int mu = 0; mu < (P::exact ? P::M : m.M); ++mu) {
+        const double *a = red + mu * kRedStride + (lane >> 4);
+        double va[2][S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            va[0][s] = lds_read(a + 4 * s);
+            va[1][s] = lds_read(a + kMaxMu * kRedStride + 4 * s);
+        }
+        for (int z0 = 0; z0 < m.Z; z0 += 4) {
+            const int sp = z0 + (lane & 3);
+            double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+            for (int k = 0; k < S; k += 4)
+                if (4 * k < cnt) {
+#pragma unroll
+                    for (int s = k; s < k + 4; ++s) {
+                        s0 = __builtin_amdgcn_mfma_f64_4x4x4f64(ty[s] == sp ? va[0][s] : 0.0,
+                                                                bq[0][s], s0, 0, 0, 0);
+                        s1 = __builtin_amdgcn_mfma_f64_4x4x4f64(ty[s] == sp ? va[1][s] : 0.0,
+                                                                bq[1][s], s1, 0, 0, 0);
+                    }
+                }
+            const int so = z0 + (lane >> 4), k = lane & (kChunk - 1);
+            if (so < m.Z && k < R)
+                grad[(ti * m.Z + so) * MR + mu * R + k] += s0 + s1;
+        }
+    }
+    wave_sync();
 }
 
 template <class P, bool kTabLds, int kMaxWaves>
@@ -437,23 +561,14 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
 
         // ---- 1. basic moments and their tangents ----------------------------
         for (int base = 0; base < n; base += kWave) {
-            DualCtx cx{red1, ws, L.slot_basic, lane, 0};
             Nbr<P::M> q;
             const bool valid = lane < n - base;
             const int64_t p = beg + base + lane;
             load_neighbor<P>(m, nb, L.coef, ti, p, valid, q);
             const GradNbr g = pair_weight<P>(nb, t, fi, S, p, valid, q);
-            double px[P::NUMAX + 1], py[P::NUMAX + 1], pz[P::NUMAX + 1];
-            unit_powers<P::NUMAX>(q, px, py, pz);
-            fwd_dual_shells<0, P>(m, cx, q, g, px, py, pz);
-            const int rest = cx.row % kChunk;
-            if (rest)
-                reduce_rows(red1, rest, cx.row - rest, lane, [&](int r, double acc) {
-                    const int b = L.slot_basic[r >> 1];
-                    if (b >= 0)
-                        ws[2 * b + (r & 1)] += acc;
-                });
+            add_dual_moments<P>(m, red1, L.mono, lds_address(ws), q, g, n - base, lane);
         }
+        wave_sync();
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
                 wp[m.dup[2 * k]] = wp[m.dup[2 * k + 1]];
@@ -485,16 +600,15 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
                 t = double2{t.x + v.x, t.y + v.y};
             }
         wave_sync();
-        // slot-ordered {A, G} (the stage may lie over the moment pairs, which
-        // are no longer read; the adjoint pairs are not under it)
-        for (int s = lane; s < m.nslots; s += kWave) {
-            const int b = L.slot_basic[s];
+        // {A, G} in the polynomials' order (the stage may lie over the moment
+        // pairs, which are no longer read; the adjoint pairs are not under it)
+        for (int s = lane; s < m.nforce; s += kWave) {
+            const int b = L.force_basic[s];
             AG[s] = b >= 0 ? wp[m.K4 + b] : double2{0.0, 0.0};
         }
         wave_sync();
 
         // ---- 4. radial coefficient gradient ---------------------------------
-        const int gbase = ti * m.Z * MR;
         for (int base = 0; base < n; base += kWave) {
             Nbr<P::M> q;
             int tj;
@@ -502,39 +616,8 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
             const int64_t p = beg + base + lane;
             const double win = load_geometry<P::M, !P::exact>(m, nb, p, valid, q, tj, ti);
             const GradNbr g = pair_weight<P>(nb, t, fi, S, p, valid, q);
-            ctype[lane] = win != 0.0 ? tj : -1;
-            double alpha[P::M], U[P::M];
-#pragma unroll
-            for (int mu = 0; mu < P::M; ++mu)
-                alpha[mu] = U[mu] = 0.0;
-            double px[P::NUMAX + 1], py[P::NUMAX + 1], pz[P::NUMAX + 1];
-            unit_powers<P::NUMAX>(q, px, py, pz);
-            rad_shells<0, P>(m, AG, px, py, pz, g, q.invd, alpha, U);
-            double Q[P::RMAX], dQ[P::RMAX];
-            radial_basis<P>(m, ti, tj, q.d, Q, dQ);
-            int row = 0;
-            auto flush = [&](int nrows) {
-                reduce_rows_typed(red4, nrows, row - nrows, lane, ctype, m.Z,
-                                  [&](int r, int tj2, double acc) {
-                                      grad[gbase + tj2 * MR + r] += acc;
-                                  });
-            };
-#pragma unroll
-            for (int mu = 0; mu < P::M; ++mu) {
-                if (P::exact || mu < m.M) {
-                    const double al = alpha[mu] * win, be = g.wu * U[mu] * win;
-#pragma unroll
-                    for (int k = 0; k < P::RMAX; ++k)
-                        if (P::exact || k < m.R) {
-                            red4[(row % kChunk) * kRedStride + lane] = al * Q[k] + be * dQ[k];
-                            ++row;
-                            if (row % kChunk == 0)
-                                flush(kChunk);
-                        }
-                }
-            }
-            if (row % kChunk)
-                flush(row % kChunk);
+            add_radial_gradient<P>(m, red4, ctype, AG, grad, MR, ti, tj, win, q, g, n - base,
+                                   lane);
         }
         wave_sync();
     }
