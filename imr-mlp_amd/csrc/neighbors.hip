@@ -83,6 +83,21 @@ __global__ void box_rank_kernel(const int *box, const int *box_start, const int 
     items[s + r] = i;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave: rows of 16 by DPP row
+// shifts (lanes without a source add 0), then each row adds the totals of
+// the rows before it (lane reads).
+__device__ __forceinline__ int wave_incl_scan(int x, int lane)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    const int t0 = __builtin_amdgcn_readlane(x, 15), t1 = __builtin_amdgcn_readlane(x, 31),
+              t2 = __builtin_amdgcn_readlane(x, 47);
+    const int r = lane >> 4;
+    return x + (r >= 1 ? t0 : 0) + (r >= 2 ? t1 : 0) + (r >= 3 ? t2 : 0);
+}
+
 // Rank every staged entry within its list by key and write it to its final
 // slot (SoA); a staged entry is its key and its two points (neighbour,
 // centre), from which the displacement and distance are formed again.  One
@@ -98,8 +113,12 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int l)
     return ((uint64_t)hi << 32) | lo;
 }
 
-__global__ __launch_bounds__(256) void list_rank_kernel(const int *offsets, int n, int cap,
-                                                        const int *overflow, const uint64_t *key,
+// With cnt (a small build) the offsets are not there yet: each workgroup sums
+// the counts before its four lists itself and writes their offsets (n <= kSmallAtoms
+// makes at most 12 loads a thread, against one more launch).
+__global__ __launch_bounds__(256) void list_rank_kernel(int *offsets, const int *cnt_of, int n,
+                                                        int cap, const int *overflow,
+                                                        const uint64_t *key,
                                                         const int *st_nbr, const int *st_ctr,
                                                         const double *pts, const int *orig,
                                                         const int *types, int *idx, int *type,
@@ -108,9 +127,35 @@ __global__ __launch_bounds__(256) void list_rank_kernel(const int *offsets, int 
 {
     const int lane = threadIdx.x & 63;
     const int l = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
+    int s = 0, cnt = 0;
+    if (cnt_of) {
+        __shared__ int wsum[4];
+        const int l0 = blockIdx.x * 4;
+        int before = 0;
+        for (int i = threadIdx.x; i < l0; i += 256)
+            before += min(cnt_of[i], cap);
+        const int sum = wave_incl_scan(before, lane);
+        if (lane == 63)
+            wsum[threadIdx.x / 64] = sum;
+        __syncthreads();
+        s = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+        for (int i = l0; i < l && i < n; ++i)
+            s += min(cnt_of[i], cap);
+        if (l < n) {
+            cnt = min(cnt_of[l], cap);
+            if (lane == 0) {
+                offsets[l] = s;
+                if (l == n - 1)
+                    offsets[n] = s + cnt;
+            }
+        }
+    }
     if (l >= n || (overflow && *overflow))
         return;  // uniform over the wave
-    const int s = offsets[l], cnt = offsets[l + 1] - s;
+    if (!cnt_of) {
+        s = offsets[l];
+        cnt = offsets[l + 1] - s;
+    }
     const int64_t sb = cap ? (int64_t)l * cap : s;  // the list's first staged entry
     for (int j0 = 0; j0 < cnt; j0 += 64) {
         const int j = j0 + lane;
@@ -145,12 +190,19 @@ __global__ __launch_bounds__(256) void list_rank_kernel(const int *offsets, int 
 }
 
 // mirror[final(q)] = final(mate(q)) for every staged entry q (the staging
-// as list_rank_kernel reads it; nothing when a bin overflowed).
+// as list_rank_kernel reads it; nothing when a bin overflowed).  With status
+// (pinned host memory) the overflow flag and the entry total go there, which
+// saves the copy before the final synchronisation.
 __global__ __launch_bounds__(256) void mirror_kernel(const int *offsets, int n, int cap,
                                                      const int *overflow, const int *mate,
-                                                     const int *st_final, int *mirror)
+                                                     const int *st_final, int *mirror,
+                                                     int *status)
 {
     const int lane = threadIdx.x & 63;
+    if (status && blockIdx.x == 0 && threadIdx.x == 0) {
+        status[0] = *overflow;
+        status[1] = offsets[n];
+    }
     const int l = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
     if (l >= n || (overflow && *overflow))
         return;  // uniform over the wave
@@ -281,21 +333,6 @@ __global__ __launch_bounds__(256) void sum64_kernel(const int *in, int64_t n,
     }
 }
 
-// Inclusive prefix sum over the 64 lanes of a wave: rows of 16 by DPP row
-// shifts (lanes without a source add 0), then each row adds the totals of
-// the rows before it (lane reads).
-__device__ __forceinline__ int wave_incl_scan(int x, int lane)
-{
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    const int t0 = __builtin_amdgcn_readlane(x, 15), t1 = __builtin_amdgcn_readlane(x, 31),
-              t2 = __builtin_amdgcn_readlane(x, 47);
-    const int r = lane >> 4;
-    return x + (r >= 1 ? t0 : 0) + (r >= 2 ? t1 : 0) + (r >= 3 ? t2 : 0);
-}
-
 // One-workgroup scans use 1,024 threads (16 waves).
 constexpr int kScan1Threads = 1024, kScan1Waves = kScan1Threads / 64;
 
@@ -407,30 +444,27 @@ inline unsigned blocks(int64_t n, int t) { return (unsigned)std::max<int64_t>(1,
 // visit the passing triples in the same order, so the appended images are
 // identical.  Translations use Eigen's Matrix3d * Vector3d order: rows 0, 1
 // summed left to right, row 2 as b0 + (b1 + b2).
-int image_candidates(const double cell[9], const int pbc[3], const double lo[3],
-                     const double hi[3], double cutoff, std::vector<double> &cand,
-                     std::string &err)
+//
+// The integer ranges come first: the periodic basis (columns in walk order),
+// its dimension, and |image index| <= rng[k] for points within ext of each
+// other.
+int image_ranges(const double cell[9], const int pbc[3], const double ext[3], double basis[9],
+                 int &dims, long rng[3], std::string &err)
 {
-    cand.clear();
-    if (!pbc[0] && !pbc[1] && !pbc[2])
-        return MTPX_OK;
     int axes[3] = {0, 1, 2};
     double nrm[3];
     for (int a = 0; a < 3; ++a)
         nrm[a] = cell[3 * a] * cell[3 * a] + cell[3 * a + 1] * cell[3 * a + 1] +
                  cell[3 * a + 2] * cell[3 * a + 2];
     std::stable_sort(axes, axes + 3, [&](int a, int b) { return nrm[a] < nrm[b]; });
-    double basis[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int dims = 0;
+    std::fill(basis, basis + 9, 0.0);
+    dims = 0;
     for (int q = 0; q < 3; ++q)
         if (pbc[axes[q]]) {
             for (int r = 0; r < 3; ++r)
                 basis[r * 3 + dims] = cell[axes[q] * 3 + r];
             dims++;
         }
-    double ext[3];
-    for (int d = 0; d < 3; ++d)
-        ext[d] = hi[d] - lo[d] + cutoff;
     // pseudo-inverse of the 3 x dims basis
     double g[9] = {0}, gi[9] = {0};
     for (int a = 0; a < dims; ++a)
@@ -456,7 +490,7 @@ int image_candidates(const double cell[9], const int pbc[3], const double lo[3],
         err = "singular periodic cell";
         return MTPX_E_INVALID;
     }
-    long rng[3] = {0, 0, 0};
+    rng[0] = rng[1] = rng[2] = 0;
     for (int k = 0; k < dims; ++k) {
         double bnd = 0;
         for (int r = 0; r < 3; ++r) {
@@ -471,6 +505,23 @@ int image_candidates(const double cell[9], const int pbc[3], const double lo[3],
         }
         rng[k] = (long)std::ceil(bnd) + 1;
     }
+    return MTPX_OK;
+}
+
+int image_candidates(const double cell[9], const int pbc[3], const double lo[3],
+                     const double hi[3], double cutoff, std::vector<double> &cand,
+                     std::string &err)
+{
+    cand.clear();
+    if (!pbc[0] && !pbc[1] && !pbc[2])
+        return MTPX_OK;
+    double ext[3], basis[9];
+    int dims;
+    long rng[3];
+    for (int d = 0; d < 3; ++d)
+        ext[d] = hi[d] - lo[d] + cutoff;
+    if (int rc = image_ranges(cell, pbc, ext, basis, dims, rng, err))
+        return rc;
     long img[3];
     for (img[2] = dims > 2 ? -rng[2] : 0; img[2] <= (dims > 2 ? rng[2] : 0); ++img[2])
         for (img[1] = dims > 1 ? -rng[1] : 0; img[1] <= (dims > 1 ? rng[1] : 0); ++img[1])
@@ -850,6 +901,24 @@ __global__ void points_kernel(Seg g, const double *wr, int ntot, long long nflag
 
 // Box index (neighborhoods_base.h:179-224): ceil(tp * (bl - 2) / xd), originals
 // clamped into [1, bl-2], images into [0, bl-1]; boxes numbered globally.
+__device__ __forceinline__ int box_of(const SegGeom &b, int d, double x, bool original)
+{
+    const double tp = x - b.lo[d];
+    int v = (int)ceil(tp * (b.bl[d] - 2) / b.xd[d]);
+    if (original) {
+        if (v == 0)
+            v = 1;
+        if (v == b.bl[d] - 1)
+            --v;
+    } else {
+        if (v < 0)
+            v = 0;
+        if (v >= b.bl[d])
+            v = b.bl[d] - 1;
+    }
+    return v;
+}
+
 __global__ void box_index_kernel(Seg g, const double *pts, int *box, int *box_count)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -861,22 +930,8 @@ __global__ void box_index_kernel(Seg g, const double *pts, int *box, int *box_co
     const SegGeom &b = g.geo[c];
     int ix[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const double tp = pts[3 * (size_t)p + d] - b.lo[d];
-        int v = (int)ceil(tp * (b.bl[d] - 2) / b.xd[d]);
-        if (original) {
-            if (v == 0)
-                v = 1;
-            if (v == b.bl[d] - 1)
-                --v;
-        } else {
-            if (v < 0)
-                v = 0;
-            if (v >= b.bl[d])
-                v = b.bl[d] - 1;
-        }
-        ix[d] = v;
-    }
+    for (int d = 0; d < 3; ++d)
+        ix[d] = box_of(b, d, pts[3 * (size_t)p + d], original);
     const int gb = g.box_off[c] + (ix[0] * b.bl[1] + ix[1]) * b.bl[2] + ix[2];
     box[p] = gb;
     atomicAdd(&box_count[gb], 1);
@@ -991,6 +1046,8 @@ __global__ __launch_bounds__(256) void construct_kernel(Seg g, Construct cb, int
     const int a = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
     if (a >= cb.ntot)
         return;  // uniform over the wave
+    if (MODE == 2 && *cb.overflow)
+        return;  // the build is redone (a small preparation's limit, or a full bin)
     const int c = seg_of(g.atom_off, g.nconf, a);
     const SegGeom &geo = g.geo[c];
     const int bl1 = geo.bl[1], bl2 = geo.bl[2], box0 = g.box_off[c];
@@ -1140,6 +1197,335 @@ __global__ __launch_bounds__(256) void construct_kernel(Seg g, Construct cb, int
 }
 
 
+// ---- small structures: the whole preparation in one workgroup -------------
+//
+// A fully periodic structure of at most kSmallAtoms atoms needs about a
+// microsecond of work in each of the eleven launches from the wrap to the
+// centre ranks, but every launch costs about five, and the host waits for the
+// AABB in between.  One workgroup of 16 waves does all of it with the
+// positions, image tests and box counters in LDS, and the host gives it only
+// the integer image ranges (from the cell: a wrapped point lies in it).  Both
+// ways produce the same points, boxes and ranks.  What does not fit the limits
+// below sets scal[10] and is built the general way.
+constexpr int kSmallAtoms = 3072;    // positions: 72 KB of LDS
+constexpr int kSmallPoints = 18432;  // 16-bit boxes of the points: 36 KB
+constexpr int kSmallTriples = 1024;  // image triples, one a thread
+constexpr int kSmallImages = 256;    // of which this many reach the box
+constexpr int kSmallUnits = 2048;    // (image, 64 atoms) tests
+constexpr int kSmallBoxes = 4096;    // four a thread
+constexpr size_t kSmallLds = sizeof(double) * 3 * (kSmallAtoms + kSmallImages) +
+                             sizeof(uint64_t) * kSmallUnits + sizeof(int) * kSmallBoxes +
+                             sizeof(uint16_t) * (kSmallUnits + kSmallPoints);
+static_assert(sizeof(uint16_t) * kSmallPoints <= sizeof(double) * 3 * kSmallAtoms, "LDS overlay");
+static_assert(kSmallUnits == 2 * kScan1Threads && kSmallBoxes == 4 * kScan1Threads &&
+                  kSmallTriples == kScan1Threads,
+              "items a thread");
+static_assert(kSmallPoints < 1 << 16 && kSmallAtoms < 1 << 15, "16-bit halves");
+
+struct SmallTables {  // what the later kernels read of a Seg
+    int atom_off[2], pt_off[2], box_off[2];
+    SegGeom geo;
+};
+
+struct SmallBuild {
+    int n;
+    int rng[3];         // image indices -rng[k] .. rng[k]
+    double basis[9];    // columns in walk order
+    Cell cell;
+    double cutoff;
+    const double *pos;  // pinned host memory
+    const int *types;
+    double *pts;
+    int *orig, *items, *box_start, *rank, *centre_box, *cnt, *center_type, *scal;
+    SmallTables *tab;
+};
+
+// The smaller (kMax: larger) of v and the lane that the DPP control selects
+// within the lane's row of 16; row16_extreme: over the row, in every lane.
+// Lane moves instead of shuffles: sixteen waves share one LDS pipe here.
+template <bool kMax, int kCtrl>
+__device__ __forceinline__ double dpp_extreme(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, 0xf, 0xf, false);
+    const double o = __hiloint2double(hi, lo);
+    return (kMax ? o > v : o < v) ? o : v;
+}
+template <bool kMax>
+__device__ __forceinline__ double row16_extreme(double v)
+{
+    v = dpp_extreme<kMax, 0xB1>(v);   // quad_perm [1,0,3,2]
+    v = dpp_extreme<kMax, 0x4E>(v);   // quad_perm [2,3,0,1]
+    v = dpp_extreme<kMax, 0x141>(v);  // row_half_mirror
+    v = dpp_extreme<kMax, 0x140>(v);  // row_mirror
+    return v;
+}
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+__global__ __launch_bounds__(kScan1Threads) void small_prepare_kernel(SmallBuild a)
+{
+    extern __shared__ double lds[];
+    double *P = lds;                    // wrapped positions [n][3]
+    double *T = P + 3 * kSmallAtoms;    // image translations
+    uint64_t *ball = reinterpret_cast<uint64_t *>(T + 3 * kSmallImages);
+    // points of each box in the low half, its originals in the high half:
+    // one scan gives both prefixes
+    unsigned *count = reinterpret_cast<unsigned *>(ball + kSmallUnits);
+    uint16_t *upre = reinterpret_cast<uint16_t *>(count + kSmallBoxes);
+    uint16_t *box = upre + kSmallUnits;
+    uint16_t *unsorted = reinterpret_cast<uint16_t *>(P);  // after the box indices
+    __shared__ int wsum[3][kScan1Waves];
+    __shared__ double wlo[3][64], whi[3][64];  // of the 64 rows of 16 threads
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, n = a.n;
+
+    // positions and species from pinned host memory, all loads of a thread in
+    // flight together (a round trip takes about two microseconds)
+    constexpr int kPer = 3 * kSmallAtoms / kScan1Threads, kTypes = kSmallAtoms / kScan1Threads;
+    double pv[kPer];
+    int tv[kTypes];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+        pv[j] = j * kScan1Threads + t < 3 * n ? a.pos[j * kScan1Threads + t] : 0.0;
+#pragma unroll
+    for (int j = 0; j < kTypes; ++j)
+        tv[j] = j * kScan1Threads + t < n ? a.types[j * kScan1Threads + t] : 0;
+    if (t < 4)
+        a.scal[10 + t] = 0;
+    for (int k = t; k <= n; k += kScan1Threads)
+        a.cnt[k] = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        count[k * kScan1Threads + t] = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+        if (j * kScan1Threads + t < 3 * n)
+            P[j * kScan1Threads + t] = pv[j];
+#pragma unroll
+    for (int j = 0; j < kTypes; ++j)
+        if (j * kScan1Threads + t < n) {
+            a.center_type[j * kScan1Threads + t] = tv[j];
+            a.orig[j * kScan1Threads + t] = j * kScan1Threads + t;
+        }
+    __syncthreads();
+    // load_positions (neighborhoods_base.h:113-127) and the AABB
+    double l[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
+    double h[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
+    for (int i = t; i < n; i += kScan1Threads) {
+        double f[3], p[3] = {P[3 * i], P[3 * i + 1], P[3 * i + 2]};
+        dev_row_times(p, a.cell.inv, f);
+        f[0] -= floor(f[0]);
+        f[1] -= floor(f[1]);
+        f[2] -= floor(f[2]);
+        dev_row_times(f, a.cell.m, p);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            P[3 * i + d] = p[d];
+            a.pts[3 * i + d] = p[d];
+            l[d] = p[d] < l[d] ? p[d] : l[d];
+            h[d] = p[d] > h[d] ? p[d] : h[d];
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        l[d] = row16_extreme<false>(l[d]);
+        h[d] = row16_extreme<true>(h[d]);
+        if ((t & 15) == 0) {
+            wlo[d][t >> 4] = l[d];
+            whi[d][t >> 4] = h[d];
+        }
+    }
+    __syncthreads();
+    SegGeom b;
+    b.cutoff = a.cutoff;
+    double nbox_d = 1.0;
+    bool ok = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double rl = row16_extreme<false>(wlo[d][lane]);
+        const double rh = row16_extreme<true>(whi[d][lane]);
+        double lo = lane_value(rl, 0), hi = lane_value(rh, 0);
+#pragma unroll
+        for (int k = 16; k < 64; k += 16) {
+            const double pl = lane_value(rl, k), ph = lane_value(rh, k);
+            lo = pl < lo ? pl : lo;
+            hi = ph > hi ? ph : hi;
+        }
+        if (hi - lo < a.cutoff)  // extent_impl, :140-143
+            hi = lo + a.cutoff;
+        b.lo[d] = lo;
+        b.hi[d] = hi;
+        b.xd[d] = hi - lo;
+        const double cells = floor((hi - lo) / a.cutoff) + 2;
+        ok = ok && cells <= kSmallBoxes;  // also false for a NaN
+        b.bl[d] = ok ? (int)cells : 3;
+        if (b.bl[d] == 2)
+            b.bl[d] = 3;
+        nbox_d *= b.bl[d];
+    }
+    ok = ok && nbox_d <= kSmallBoxes;
+    const int nbox = ok ? b.bl[0] * b.bl[1] * b.bl[2] : 0;
+
+    // image triples in walk order (the last axis outermost) whose translated
+    // box meets [lo - rc, hi + rc]: the arithmetic of image_candidates
+    const int w0 = 2 * a.rng[0] + 1, w1 = 2 * a.rng[1] + 1, w2 = 2 * a.rng[2] + 1;
+    bool reach = false;
+    double tr[3] = {0, 0, 0};
+    if (t < w0 * w1 * w2) {
+        const int i0 = t % w0 - a.rng[0], i1 = (t / w0) % w1 - a.rng[1],
+                  i2 = t / (w0 * w1) - a.rng[2];
+        reach = i0 != 0 || i1 != 0 || i2 != 0;
+        double q[3][3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            q[r][0] = a.basis[3 * r] * (double)i0;
+            q[r][1] = a.basis[3 * r + 1] * (double)i1;
+            q[r][2] = a.basis[3 * r + 2] * (double)i2;
+        }
+        tr[0] = (q[0][0] + q[0][1]) + q[0][2];
+        tr[1] = (q[1][0] + q[1][1]) + q[1][2];
+        tr[2] = q[2][0] + (q[2][1] + q[2][2]);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            if (b.hi[d] + tr[d] < b.lo[d] - a.cutoff - 1e-9 * (1 + fabs(tr[d])) ||
+                b.lo[d] + tr[d] > b.hi[d] + a.cutoff + 1e-9 * (1 + fabs(tr[d])))
+                reach = false;
+    }
+    int ncand;
+    const int slot = block_excl_scan(reach ? 1 : 0, wsum[0], ncand);
+    if (reach && slot < kSmallImages) {
+        T[3 * slot] = tr[0];
+        T[3 * slot + 1] = tr[1];
+        T[3 * slot + 2] = tr[2];
+    }
+    const int ntile = (n + 63) / 64, units = ncand * ntile;
+    if (!ok || ncand > kSmallImages || units > kSmallUnits) {  // uniform over the workgroup
+        if (t == 0)
+            a.scal[10] = 2;
+        return;
+    }
+    __syncthreads();
+    // image q of atom i lies in [lo - rc, hi + rc] (append_images,
+    // neighborhoods_base.h:72-80): one ballot a unit.  A wave keeps a tile of
+    // 64 atoms and walks the images; with fewer tiles than waves several waves
+    // share a tile's images.
+    const int share = ntile < kScan1Waves ? kScan1Waves / ntile : 1;
+    const int tile0 = wv % ntile, q0 = wv / ntile;  // with share == 1: tile wv, q0 0
+    const int tile_step = ntile < kScan1Waves ? ntile : kScan1Waves;
+    auto walk = [&](auto &&body) {
+        if (ntile < kScan1Waves ? q0 >= share : wv >= ntile)
+            return;
+        for (int tile = ntile < kScan1Waves ? tile0 : wv; tile < ntile; tile += tile_step) {
+            const int i = tile * 64 + lane;
+            const bool valid = i < n;
+            const double x = valid ? P[3 * i] : 0.0, y = valid ? P[3 * i + 1] : 0.0,
+                         z = valid ? P[3 * i + 2] : 0.0;
+            for (int q = ntile < kScan1Waves ? q0 : 0; q < ncand; q += share)
+                body(q * ntile + tile, q, i, valid, x, y, z);
+        }
+    };
+    walk([&](int u, int q, int, bool valid, double x, double y, double z) {
+        const double p0 = x + T[3 * q], p1 = y + T[3 * q + 1], p2 = z + T[3 * q + 2];
+        const bool out = p0 < b.lo[0] - b.cutoff || p1 < b.lo[1] - b.cutoff ||
+                         p2 < b.lo[2] - b.cutoff || p0 > b.hi[0] + b.cutoff ||
+                         p1 > b.hi[1] + b.cutoff || p2 > b.hi[2] + b.cutoff;
+        const uint64_t m = __ballot(valid && !out);
+        if (lane == 0)
+            ball[u] = m;
+    });
+    __syncthreads();
+    int nimg;
+    {
+        const int c0 = 2 * t < units ? __popcll(ball[2 * t]) : 0;
+        const int c1 = 2 * t + 1 < units ? __popcll(ball[2 * t + 1]) : 0;
+        const int pre = block_excl_scan(c0 + c1, wsum[1], nimg);
+        upre[2 * t] = (uint16_t)pre;  // exact up to kSmallPoints
+        upre[2 * t + 1] = (uint16_t)(pre + c0);
+    }
+    const int npts = n + nimg;
+    if (npts > kSmallPoints) {  // uniform
+        if (t == 0)
+            a.scal[10] = 2;
+        return;
+    }
+    __syncthreads();
+    walk([&](int u, int q, int i, bool, double x, double y, double z) {
+        const uint64_t m = ball[u];
+        if ((m >> lane) & 1) {
+            const int o = n + upre[u] + __popcll(m & ((1ull << lane) - 1));
+            a.pts[3 * o] = x + T[3 * q];
+            a.pts[3 * o + 1] = y + T[3 * q + 1];
+            a.pts[3 * o + 2] = z + T[3 * q + 2];
+            a.orig[o] = i;
+        }
+    });
+    __syncthreads();
+    // the points' boxes (box_index_kernel's formula and clamps), every lane
+    // busy: the images of a unit are few
+    for (int p = t; p < npts; p += kScan1Threads) {
+        const bool original = p < n;
+        int ix[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            ix[d] = box_of(b, d, a.pts[3 * p + d], original);
+        const int gb = (ix[0] * b.bl[1] + ix[1]) * b.bl[2] + ix[2];
+        box[p] = (uint16_t)gb;
+        atomicAdd(&count[gb], original ? 0x10001u : 1u);
+    }
+    if (t == 0) {
+        a.tab->atom_off[0] = a.tab->pt_off[0] = a.tab->box_off[0] = 0;
+        a.tab->atom_off[1] = n;
+        a.tab->pt_off[1] = npts;
+        a.tab->box_off[1] = nbox + 1;
+        a.tab->geo = b;
+    }
+    __syncthreads();
+    // box starts; the originals lie in interior boxes, whose walk order is
+    // the order of the boxes, so their ranks follow from a prefix over all
+    {
+        unsigned c[4], cs = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            c[k] = count[4 * t + k];
+            cs += c[k];
+        }
+        int tot;
+        unsigned cp = (unsigned)block_excl_scan((int)cs, wsum[2], tot);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            count[4 * t + k] = cp;
+            if (4 * t + k <= nbox)
+                a.box_start[4 * t + k] = (int)(cp & 0xffff);
+            cp += c[k];
+        }
+        if (t == 0 && nbox == kSmallBoxes)
+            a.box_start[nbox] = npts;
+    }
+    __syncthreads();
+    for (int p = t; p < npts; p += kScan1Threads)
+        unsorted[atomicAdd(&count[box[p]], 1u) & 0xffff] = (uint16_t)p;
+    __syncthreads();
+    // The low half of count[b] is now the end of box b.  A point's slot is the
+    // number of its box's points with a smaller index (box_rank_kernel); the
+    // originals come first in their box.
+    for (int p = t; p < npts; p += kScan1Threads) {
+        const int gb = box[p];
+        const int s = gb ? count[gb - 1] & 0xffff : 0, e = count[gb] & 0xffff;
+        int r = 0;
+#pragma unroll 8
+        for (int u = s; u < e; ++u)
+            r += unsorted[u] < p;
+        a.items[s + r] = p;
+        if (p < n) {
+            a.rank[p] = (int)(count[gb] >> 16) + r;
+            a.centre_box[p] = gb;
+        }
+    }
+}
+
 // Clears the list counters [n], the 64-bit entry total and the longest
 // list before a counted build that follows a one-pass build.
 __global__ void zero_counts_kernel(int *cnt, int n, unsigned long long *z64, int *largest)
@@ -1222,6 +1608,150 @@ struct Upload {
 // Entries that the bins of a one-pass build may hold (6.4 GB of staging).
 constexpr long long kBinEntries = 1LL << 27;
 
+// Staging and list buffers for n entries.
+hipError_t ensure_entries(NeighborStore &out, NeighborScratch &w, size_t n)
+{
+    const size_t nz = std::max<size_t>(n, 1);
+    for (DBuf *b : {&out.idx, &out.type, &out.mirror, &w.st_nbr, &w.st_ctr, &w.st_mate,
+                    &w.st_final})
+        if (hipError_t e = b->ensure(sizeof(int) * nz))
+            return e;
+    for (DBuf *b : {&out.x, &out.y, &out.z, &out.d})
+        if (hipError_t e = b->ensure(sizeof(double) * nz))
+            return e;
+    return w.key.ensure(sizeof(uint64_t) * nz);
+}
+
+// Ranks the staged lists: their offsets are there, or with cnt are formed on
+// the way.
+void rank_lists(NeighborStore &out, NeighborScratch &w, int ntot, const int *cnt, int cap,
+                const int *overflow, int *status, hipStream_t s)
+{
+    const dim3 grid((ntot + 3) / 4), block(256);
+    hipLaunchKernelGGL(list_rank_kernel, grid, block, 0, s, out.offsets.as<int>(), cnt, ntot, cap,
+                       overflow, w.key.as<uint64_t>(), w.st_nbr.as<int>(), w.st_ctr.as<int>(),
+                       w.pts.as<double>(), w.orig.as<int>(), out.center_type.as<int>(),
+                       out.idx.as<int>(), out.type.as<int>(), out.x.as<double>(),
+                       out.y.as<double>(), out.z.as<double>(), out.d.as<double>(),
+                       w.st_final.as<int>());
+    hipLaunchKernelGGL(mirror_kernel, grid, block, 0, s, out.offsets.as<int>(), ntot, cap,
+                       overflow, w.st_mate.as<int>(), w.st_final.as<int>(), out.mirror.as<int>(),
+                       status);
+}
+
+// One fully periodic structure of n <= kSmallAtoms atoms: four launches and
+// one synchronisation (3,072 atoms: 99 us a build, 152 the general way with its
+// fourteen launches and two synchronisations; 1,000 atoms 66 us, of which 27 in
+// the preparation, bound by latency and the one CU).  *built stays false when the
+// structure does not fit the limits or a list its bin; it is then built the
+// general way, which also reports every error.
+int build_small(const double cell[9], const int pbc[3], int n, const double *pos,
+                const int *types, double cutoff, hipStream_t s, NeighborStore &out,
+                NeighborScratch &w, bool *built, std::string &err)
+{
+    SmallBuild a{};
+    std::copy(cell, cell + 9, a.cell.m);
+    // a wrapped point lies in the cell, so the AABB spans at most the sum of
+    // the vectors' components (or the cutoff, to which it is widened)
+    double ext[3], volume;
+    for (int d = 0; d < 3; ++d) {
+        const double span = std::fabs(cell[d]) + std::fabs(cell[3 + d]) + std::fabs(cell[6 + d]);
+        ext[d] = std::max(span * (1 + 1e-6), cutoff) + cutoff;
+    }
+    std::string none;
+    int dims;
+    long rng[3];
+    if (!cell_inverse(a.cell.m, a.cell.inv) ||
+        image_ranges(cell, pbc, ext, a.basis, dims, rng, none) != MTPX_OK)
+        return MTPX_OK;
+    long triples = 1;
+    for (int k = 0; k < 3; ++k) {
+        if (rng[k] > kSmallTriples)
+            return MTPX_OK;
+        triples *= 2 * rng[k] + 1;
+        if (triples > kSmallTriples)
+            return MTPX_OK;
+        a.rng[k] = (int)rng[k];
+    }
+    volume = std::fabs(cell[0] * (cell[4] * cell[8] - cell[5] * cell[7]) -
+                       cell[1] * (cell[3] * cell[8] - cell[5] * cell[6]) +
+                       cell[2] * (cell[3] * cell[7] - cell[4] * cell[6]));
+    // bins sized from the previous build, or one and a half times the mean
+    // list and a margin when there is none
+    long long cap = w.bin_cap;
+    if (cap <= 0) {
+        const double mean = n / volume * (4.0 / 3.0 * M_PI) * cutoff * cutoff * cutoff;
+        if (!(mean < 4096))
+            return MTPX_OK;
+        cap = (long long)(1.5 * mean) + 32;
+    }
+    if (n * cap > kBinEntries)
+        return MTPX_OK;
+    const size_t pos_bytes = sizeof(double) * 3 * (size_t)n;
+    DTRY(w.up_pos.ensure(pos_bytes + sizeof(int) * (size_t)n));
+    std::memcpy(w.up_pos.p, pos, pos_bytes);
+    std::memcpy(w.up_pos.as<unsigned char>() + pos_bytes, types, sizeof(int) * (size_t)n);
+    void *hpos = nullptr, *hdown = nullptr;
+    DTRY(hipHostGetDevicePointer(&hpos, w.up_pos.p, 0));
+    DTRY(w.down.ensure(sizeof(int) * 16));
+    DTRY(hipHostGetDevicePointer(&hdown, w.down.p, 0));
+    DTRY(w.scalars.ensure(sizeof(int) * 16));
+    DTRY(w.seg_tabs.ensure(sizeof(SmallTables)));
+    DTRY(w.pts.ensure(sizeof(double) * 3 * kSmallPoints));
+    DTRY(w.orig.ensure(sizeof(int) * kSmallPoints));
+    DTRY(w.box_items.ensure(sizeof(int) * kSmallPoints));
+    DTRY(w.box_start.ensure(sizeof(int) * (kSmallBoxes + 1)));
+    DTRY(w.rank.ensure(sizeof(int) * 2 * (size_t)n));
+    DTRY(w.cursor.ensure(sizeof(int) * ((size_t)n + 1)));
+    DTRY(ensure_entries(out, w, (size_t)n * cap));
+    a.n = n;
+    a.cutoff = cutoff;
+    a.pos = static_cast<const double *>(hpos);
+    a.types = reinterpret_cast<const int *>(static_cast<unsigned char *>(hpos) + pos_bytes);
+    a.pts = w.pts.as<double>();
+    a.orig = w.orig.as<int>();
+    a.items = w.box_items.as<int>();
+    a.box_start = w.box_start.as<int>();
+    a.rank = w.rank.as<int>();
+    a.centre_box = a.rank + n;
+    a.cnt = w.cursor.as<int>();
+    a.center_type = out.center_type.as<int>();
+    a.scal = w.scalars.as<int>();
+    a.tab = w.seg_tabs.as<SmallTables>();
+    hipLaunchKernelGGL(small_prepare_kernel, dim3(1), dim3(kScan1Threads), kSmallLds, s, a);
+    Seg g{};
+    g.nconf = 1;
+    g.atom_off = a.tab->atom_off;  // addresses only: the table is in device memory
+    g.pt_off = a.tab->pt_off;
+    g.box_off = a.tab->box_off;
+    g.geo = &a.tab->geo;
+    Construct cb{};
+    cb.pts = a.pts;
+    cb.orig = a.orig;
+    cb.box_start = a.box_start;
+    cb.items = a.items;
+    cb.types = a.center_type;
+    cb.rank = a.rank;
+    cb.centre_box = a.centre_box;
+    cb.ntot = n;
+    cb.cutoffsq = cutoff * cutoff;
+    cb.cap = (int)cap;
+    cb.overflow = a.scal + 10;
+    cb.mate = w.st_mate.as<int>();
+    hipLaunchKernelGGL(construct_kernel<2>, dim3((n + 3) / 4), dim3(256), 0, s, g, cb, nullptr,
+                       a.cnt, w.key.as<uint64_t>(), w.st_nbr.as<int>(), w.st_ctr.as<int>());
+    rank_lists(out, w, n, a.cnt, (int)cap, a.scal + 10, static_cast<int *>(hdown), s);
+    DTRY(hipGetLastError());
+    DTRY(hipStreamSynchronize(s));
+    const int *down = w.down.as<int>();
+    if (down[0] != 0)
+        return MTPX_OK;
+    out.P = down[1];
+    out.has_mirror = true;
+    *built = true;
+    return MTPX_OK;
+}
+
 // Atoms per chunk: kChunkAtoms, or less when MTPX_NEIGHBOR_CHUNK_ATOMS asks
 // for it (a smaller peak of builder scratch for very large batches).
 int chunk_atoms()
@@ -1255,6 +1785,13 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     pbc += 3 * (size_t)c0;
     pos += 3 * (size_t)base;
     types += base;
+    if (nconf == 1 && ntot <= kSmallAtoms && pbc[0] && pbc[1] && pbc[2]) {
+        bool built = false;
+        if (int rc = build_small(cells, pbc, ntot, pos, types, cutoff, s, out, w, &built, err))
+            return rc;
+        if (built)
+            return MTPX_OK;
+    }
     // host tables: offsets, cells
     std::vector<int> atom_off((size_t)nconf + 1), wrapf((size_t)nconf);
     for (int c = 0; c <= nconf; ++c)
@@ -1505,43 +2042,20 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     cb.mate = nullptr;  // set once the staging is sized
     DTRY(w.down.ensure(sizeof(int) * 16));
     int *down = w.down.as<int>();
-    auto ensure_entries = [&](size_t n) -> hipError_t {
-        const size_t nz = std::max<size_t>(n, 1);
-        for (DBuf *b : {&out.idx, &out.type, &out.mirror, &w.st_nbr, &w.st_ctr, &w.st_mate,
-                        &w.st_final})
-            if (hipError_t e = b->ensure(sizeof(int) * nz))
-                return e;
-        for (DBuf *b : {&out.x, &out.y, &out.z, &out.d})
-            if (hipError_t e = b->ensure(sizeof(double) * nz))
-                return e;
-        return w.key.ensure(sizeof(uint64_t) * nz);
-    };
-    auto rank_lists = [&](int cap, const int *overflow) {
-        hipLaunchKernelGGL(list_rank_kernel, dim3((ntot + 3) / 4), dim3(256), 0, s,
-                           out.offsets.as<int>(), ntot, cap, overflow, w.key.as<uint64_t>(),
-                           w.st_nbr.as<int>(), w.st_ctr.as<int>(), w.pts.as<double>(),
-                           w.orig.as<int>(), dtypes, out.idx.as<int>(), out.type.as<int>(),
-                           out.x.as<double>(), out.y.as<double>(), out.z.as<double>(),
-                           out.d.as<double>(), w.st_final.as<int>());
-        hipLaunchKernelGGL(mirror_kernel, dim3((ntot + 3) / 4), dim3(256), 0, s,
-                           out.offsets.as<int>(), ntot, cap, overflow, w.st_mate.as<int>(),
-                           w.st_final.as<int>(), out.mirror.as<int>());
-    };
-
     // One pass into bins sized from the previous counted build: the entry
     // total comes back with the final synchronisation.  A list that outgrows
     // its bin sends the chunk through the counted build below.
     const long long cap = w.bin_cap;
     if (cap > 0 && (long long)ntot * cap <= kBinEntries) {
         cb.cap = (int)cap;
-        DTRY(ensure_entries((size_t)ntot * cap));
+        DTRY(ensure_entries(out, w, (size_t)ntot * cap));
         cb.mate = w.st_mate.as<int>();
         hipLaunchKernelGGL(construct_kernel<2>, dim3((ntot + 3) / 4), dim3(256), 0, s, g, cb,
                            nullptr, cnt, w.key.as<uint64_t>(), w.st_nbr.as<int>(),
                            w.st_ctr.as<int>());
         DTRY(scan_exclusive(cnt, (int64_t)ntot + 1, out.offsets.as<int>(), w.tmp, scal + 12, s,
                             nullptr, (int)cap));
-        rank_lists((int)cap, scal + 10);
+        rank_lists(out, w, ntot, nullptr, (int)cap, scal + 10, nullptr, s);
         DTRY(hipMemcpyAsync(down, scal + 10, sizeof(int) * 3, hipMemcpyDeviceToHost, s));
         DTRY(hipGetLastError());
         DTRY(hipStreamSynchronize(s));
@@ -1576,7 +2090,7 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     w.bin_cap = (long long)longest + longest / 4 + 8;
     const int64_t P = (int64_t)P64;
     out.P = P;
-    DTRY(ensure_entries((size_t)P));
+    DTRY(ensure_entries(out, w, (size_t)P));
     out.has_mirror = true;
     if (P == 0)
         return MTPX_OK;
@@ -1584,7 +2098,7 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     hipLaunchKernelGGL(construct_kernel<1>, dim3((ntot + 3) / 4), dim3(256), 0, s, g, cb,
                        nullptr, cnt, w.key.as<uint64_t>(), w.st_nbr.as<int>(),
                        w.st_ctr.as<int>());
-    rank_lists(0, nullptr);
+    rank_lists(out, w, ntot, nullptr, 0, nullptr, nullptr, s);
     DTRY(hipGetLastError());
     DTRY(hipStreamSynchronize(s));
     return MTPX_OK;
