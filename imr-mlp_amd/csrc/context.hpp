@@ -4,6 +4,7 @@
 #include "mtpx.h"
 #include "mtpx_internal.hpp"
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -52,6 +53,7 @@ struct mtpx_context {
 
     // outputs
     DBuf forces, site_energy, partial, pair_ders, out10;
+    HBuf out_host;  // pinned staging of the outputs a call returns
     DBuf site_virial, benergy, bstress;  // batch: [N][9], [nconf], [nconf][9]
     EfsLaunch launch{};
     bool has_batch_out = false;          // compute_batch outputs match model and topology
@@ -136,6 +138,7 @@ struct mtpx_context {
                         &lin_pair, &lin_site, &lin_flevel, &lin_fsteps, &lin_lw, &lin_tiles})
             b->release();
         scratch.release_all();
+        out_host.release();
         sites.release();
         for (auto &e : ev)
             if (e)
@@ -216,11 +219,24 @@ hipError_t upload(DBuf &b, const std::vector<T> &v, hipStream_t s)
 int copy_out(mtpx_context *ctx, double *dst, const void *src, size_t count, bool add,
              const char *what);
 
+// One output of a call: count doubles from the device to dst (skipped when
+// null), added onto what dst holds with add.
+struct OutPart {
+    double *dst;
+    const DBuf &src;
+    size_t count;
+    bool add;
+};
+// Waits for the work queued on the context's stream and returns its outputs
+// (at most kOutParts).
+int finish_outputs(mtpx_context *ctx, std::initializer_list<OutPart> parts, const char *what);
+
 // Runs the E/F/S kernel over the resident topology (capi.cpp); with
 // site_virial the per-atom virials are written too; energy_only skips the
-// gradient (site energies and the total only).
+// gradient (site energies and the total only).  Without wait the launches
+// are only queued (a context with timings on waits all the same).
 int run_efs(mtpx_context *ctx, bool deterministic, bool site_virial = false,
-            bool energy_only = false);
+            bool energy_only = false, bool wait = true);
 // Marks the topology as one structure of all atoms.
 int set_single_structure(mtpx_context *ctx);
 // Reverse index of the resident lists (and their offsets on the host).

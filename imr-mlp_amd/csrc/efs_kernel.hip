@@ -378,6 +378,22 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(double *p, size_t count)
         p[k] = 0.0;
 }
 
+__global__ __launch_bounds__(256) void pack_outputs_kernel(OutParts p, double *dst)
+{
+    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= p.end[kOutParts - 1])
+        return;
+    const double *src = p.src[0];
+    size_t first = 0;
+#pragma unroll
+    for (int j = 1; j < kOutParts; ++j)
+        if (k >= p.end[j - 1]) {
+            src = p.src[j];
+            first = p.end[j - 1];
+        }
+    dst[k] = src[k - first];
+}
+
 // Kernel variants: shell profile x table placement.  The profiles whose
 // kernels fit 256 registers run eight waves per workgroup, the larger ones four.
 template <class P>
@@ -484,6 +500,15 @@ hipError_t launch_efs(const DevModel &m, const DevNeighbors &nb, const EfsOut &o
 hipError_t noalloc_scratch_address(double **ptr)
 {
     return hipGetSymbolAddress(reinterpret_cast<void **>(ptr), HIP_SYMBOL(scratch));
+}
+
+hipError_t launch_pack_outputs(const OutParts &p, double *dst, hipStream_t s)
+{
+    const size_t count = p.end[kOutParts - 1];
+    if (count)
+        hipLaunchKernelGGL(pack_outputs_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256),
+                           0, s, p, dst);
+    return hipGetLastError();
 }
 
 hipError_t launch_fill_zero(double *p, size_t count, hipStream_t s)

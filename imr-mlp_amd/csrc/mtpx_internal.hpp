@@ -601,6 +601,14 @@ hipError_t launch_site_gather(const DevNeighbors &nb, int ntotal, const int *ato
 constexpr size_t kNoAllocScratchDoubles = size_t(1) << 16;  // 512 KiB
 // Device address of that array on the current device (hipGetSymbolAddress).
 hipError_t noalloc_scratch_address(double **ptr);
+// Up to kOutParts device arrays written one after the other to dst (pinned
+// host memory) by one launch.
+constexpr int kOutParts = 4;
+struct OutParts {
+    const double *src[kOutParts];
+    size_t end[kOutParts];  // running count; unused parts repeat the last
+};
+hipError_t launch_pack_outputs(const OutParts &p, double *dst, hipStream_t s);
 // Zero-fill kernel (used where a caller may capture the launches).
 hipError_t launch_fill_zero(double *p, size_t count, hipStream_t s);
 

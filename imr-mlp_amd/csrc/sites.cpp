@@ -260,10 +260,16 @@ int mtpx_compute_sites(mtpx_context *ctx, const mtpx_site_request *req)
                         "clear site virials");
         }
     }
-    HIP_TRY(hipStreamSynchronize(s), "site request");
-
     double o10[10];
-    HIP_TRY(hipMemcpy(o10, S.out10.p, sizeof o10, hipMemcpyDeviceToHost), "copy outputs");
+    std::vector<double> se(r.site_energy && r.nlocal > 0 ? (size_t)nr : 0);
+    if (int rc = finish_outputs(ctx,
+                                {{o10, S.out10, 10, false},
+                                 {r.force, S.forces, 3 * (size_t)ntot, r.accumulate_force != 0},
+                                 {se.empty() ? nullptr : se.data(), S.site_energy, se.size(), false},
+                                 {want_v6 ? r.site_virial : nullptr, S.site_virial6,
+                                  6 * (size_t)ntot, false}},
+                                "site request"))
+        return rc;
     if (r.total_energy)
         *r.total_energy = o10[0];
     if (r.global_virial) {
@@ -275,24 +281,11 @@ int mtpx_compute_sites(mtpx_context *ctx, const mtpx_site_request *req)
         r.global_virial[4] = 0.5 * (St[2] + St[6]);
         r.global_virial[5] = 0.5 * (St[5] + St[7]);
     }
-    if (r.force)
-        if (int rc = copy_out(ctx, r.force, S.forces.p, 3 * (size_t)ntot,
-                              r.accumulate_force != 0, "copy forces"))
-            return rc;
     if (r.site_energy && r.nlocal > 0) {
-        std::vector<double> se((size_t)std::max(nr, 1));
-        if (nr > 0)
-            HIP_TRY(hipMemcpy(se.data(), S.site_energy.p, sizeof(double) * nr,
-                              hipMemcpyDeviceToHost),
-                    "copy site energies");
         std::fill(r.site_energy, r.site_energy + r.nlocal, 0.0);
         for (int k = 0; k < nr; ++k)
             r.site_energy[S.row_atom[k]] = se[k];
     }
-    if (want_v6)
-        if (int rc = copy_out(ctx, r.site_virial, S.site_virial6.p, 6 * (size_t)ntot, false,
-                              "copy site virials"))
-            return rc;
     return MTPX_OK;
 }
 

@@ -83,7 +83,7 @@ int need_topology(mtpx_context *ctx)
 // E/F/S of the batch and the per-structure energy and virial.
 int batch_forward(mtpx_context *ctx, bool deterministic)
 {
-    int rc = run_efs(ctx, deterministic, true);
+    int rc = run_efs(ctx, deterministic, true, false, false);
     if (rc != MTPX_OK)
         return rc;
     const int nc = std::max(ctx->nconf, 1);
@@ -247,16 +247,12 @@ int mtpx_compute_batch(mtpx_context *ctx, int deterministic, double *energy, dou
         return rc;
     const size_t nc = (size_t)ctx->nconf, n = (size_t)ctx->n;
     const bool add = ctx->add_efs;
-    HIP_TRY(hipStreamSynchronize(ctx->stream), "compute batch");
-    if (energy)
-        rc = copy_out(ctx, energy, ctx->benergy.p, nc, add, "copy energies");
-    if (rc == MTPX_OK && stress)
-        rc = copy_out(ctx, stress, ctx->bstress.p, 9 * nc, add, "copy stresses");
-    if (rc == MTPX_OK && forces)
-        rc = copy_out(ctx, forces, ctx->forces.p, 3 * n, add, "copy forces");
-    if (rc == MTPX_OK && site_energies)
-        rc = copy_out(ctx, site_energies, ctx->site_energy.p, n, add, "copy site energies");
-    return rc;
+    return finish_outputs(ctx,
+                          {{energy, ctx->benergy, nc, add},
+                           {stress, ctx->bstress, 9 * nc, add},
+                           {forces, ctx->forces, 3 * n, add},
+                           {site_energies, ctx->site_energy, n, add}},
+                          "compute batch");
 }
 
 int mtpx_loss_weights(const mtpx_loss_settings *s, int nconf, const int *atom_offsets,
