@@ -75,7 +75,7 @@ struct mtpx_context {
     DevLin dl{};
     DBuf lin_level, lin_steps, lin_ent, lin_estart, lin_chunk, lin_maskw,
         lin_clist, lin_flevel, lin_fsteps, lin_walk, lin_walk_off, lin_cscal;
-    DBuf comp, row_src, row_sw, row_y, rowsA, rowsY, gram_part, gram_out, lin_pair, lin_site;
+    DBuf comp, row_src, row_sw, row_y, rowsA, rowsY, gram_part, gram_out, lin_pair, lin_site, lin_part;
     // tile path: walk-order Jacobian values per site, structure lists per size class
     DBuf lin_lw, lin_tiles;
     long rows_gen = -1;  // label_gen and p of the uploaded row descriptors
@@ -135,7 +135,7 @@ struct mtpx_context {
                         &lin_level, &lin_steps, &lin_ent, &lin_estart, &lin_chunk, &lin_maskw, &lin_clist,
                         &lin_walk, &lin_walk_off, &lin_cscal,
                         &comp, &row_src, &row_sw, &row_y, &rowsA, &rowsY, &gram_part, &gram_out,
-                        &lin_pair, &lin_site, &lin_flevel, &lin_fsteps, &lin_lw, &lin_tiles})
+                        &lin_pair, &lin_site, &lin_part, &lin_flevel, &lin_fsteps, &lin_lw, &lin_tiles})
             b->release();
         scratch.release_all();
         out_host.release();

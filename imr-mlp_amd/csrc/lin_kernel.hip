@@ -423,11 +423,14 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
     const int lane = threadIdx.x;
     // chunk-major: the waves that run at the same time mostly walk the same
     // chunk, whose code then stays in the instruction cache
-    const int item = blockIdx.x;
+    const int item = blockIdx.x / t.parts, part = blockIdx.x % t.parts;
     if (item >= t.count * t.nchunks)
         return;
     const int c = t.structs[item % t.count], ch = item / t.count;
     const int i0 = t.soff[c], i1 = t.soff[c + 1], N = i1 - i0;
+    // this wave's sites
+    const int s0 = i0 + (int)((int64_t)N * part / t.parts);
+    const int s1 = i0 + (int)((int64_t)N * (part + 1) / t.parts);
     // the chunk's scalars: its output columns are Z + cols[k]
     const int q0 = L.chunk_s0[ch], w = L.chunk_s0[ch + 1] - q0;
     const int *cols = L.chunk_scalar + q0;
@@ -495,20 +498,20 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
     double nl0 = 0.0, nl1 = 0.0;
     EntryRaw nx{0.0, 0.0, 0.0, 0.0, 0, -1};
     int cbeg = 0, cend = 0, cti = 0;  // this site's
-    if (i0 < i1) {
-        fetch_bounds(i0);
+    if (s0 < s1) {
+        fetch_bounds(s0);
         take_bounds();
         cbeg = nbeg;
         cend = nend;
         cti = nti;
-        fetch_l(i0, nl0, nl1);
+        fetch_l(s0, nl0, nl1);
         nx = fetch_entry(nb, cbeg + lane, lane < cend - cbeg);
-        if (i0 + 1 < i1)
-            fetch_bounds(i0 + 1);
+        if (s0 + 1 < s1)
+            fetch_bounds(s0 + 1);
     }
-    for (int i = i0; i < i1; ++i) {
+    for (int i = s0; i < s1; ++i) {
         const double cl0 = nl0, cl1 = nl1;
-        if (i + 1 < i1)
+        if (i + 1 < s1)
             take_bounds();  // the next site's, loaded at the end of the last walk
         if constexpr (!kLaneL) {
             if (lane < ne)
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
             // The next site's loads are issued once this batch's entry is in
             // registers: loads still in flight at the top of this loop would
             // make its wait for the entry wait for them too.
-            if (base == 0 && i + 1 < i1) {
+            if (base == 0 && i + 1 < s1) {
                 fetch_l(i + 1, nl0, nl1);
                 nx = fetch_entry(nb, nbeg + lane, lane < nend - nbeg);
                 cbeg = nbeg;
@@ -568,7 +571,7 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
             // value loaded before it could be moved between registers inside
             // the walk, which then waits for every load in flight), taken at
             // the top of the next site
-            if (base == 0 && i + 2 < i1)
+            if (base == 0 && i + 2 < s1)
                 fetch_bounds(i + 2);
             // the neighbour's row: minus this entry's derivatives
             const int jl = valid ? en.j - i0 : -1;
@@ -612,7 +615,14 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
         if constexpr (!kLaneL)
             wave_sync();  // the next site's values overwrite the stage
     }
-    if (lds_tile) {
+    double *out = nullptr;  // a part's sums
+    if (t.parts > 1) {
+        out = t.part + lin_part_doubles(t.rows_cap) * blockIdx.x;
+        wave_sync();
+        for (int k = lane; k < N * 3 * kLinChunk; k += kWave)
+            out[k] = tile[(size_t)(k / (3 * kLinChunk)) * kRow + k % (3 * kLinChunk)];
+        out += (size_t)3 * kLinChunk * t.rows_cap;
+    } else if (lds_tile) {
         wave_sync();
         for (int k = lane; k < N * 3 * w; k += kWave) {
             const int j = k / (3 * w), r = k % (3 * w), a = r / w, kk = r % w;
@@ -626,7 +636,10 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
         for (int k = 0; k < kLinChunk; ++k)
             if (k < w) {
                 const double v = wave_sum(st[u * kLinChunk + k]);
-                if (lane == 0) {
+                if (out) {
+                    if (lane == 0)
+                        out[u * kLinChunk + k] = v;
+                } else if (lane == 0) {
                     const int a = kSymA[u], b = kSymB[u];
                     t.sc[((size_t)c * 9 + 3 * a + b) * t.p + t.Z + col[k]] = v;
                     if (a != b)
@@ -636,6 +649,35 @@ __global__ __launch_bounds__(kWave) void lin_tile_kernel(DevModel m, DevLin L, D
 }
 
 #if MTPX_LIN_PART == 1
+// The rows and stress of the launch's (chunk, structure) blockIdx.y from its
+// parts: one thread per element, its parts added in order.
+__global__ __launch_bounds__(256) void lin_parts_kernel(DevLin L, LinTile t)
+{
+    const int item = blockIdx.y, c = t.structs[item % t.count], ch = item / t.count;
+    const int i0 = t.soff[c], N = t.soff[c + 1] - i0;
+    const int q0 = L.chunk_s0[ch], w = L.chunk_s0[ch + 1] - q0;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    const int rows = 3 * kLinChunk * N, k = e % kLinChunk;
+    if (e >= rows + 6 * kLinChunk || k >= w)
+        return;
+    const size_t stride = lin_part_doubles(t.rows_cap);
+    const bool force = e < rows;
+    const int u = (e - rows) / kLinChunk;  // stress component
+    const double *src = t.part + stride * t.parts * item +
+                        (force ? e : 3 * kLinChunk * t.rows_cap + (e - rows));
+    double v = 0.0;
+    for (int q = 0; q < t.parts; ++q)
+        v += src[stride * q];
+    const int col = t.Z + L.chunk_scalar[q0 + k];
+    if (force) {
+        t.fc[((size_t)3 * i0 + e / kLinChunk) * t.p + col] = v;
+    } else {
+        const int a = u < 3 ? 0 : u < 5 ? 1 : 2, b = u < 3 ? u : u < 5 ? u - 2 : 2;
+        t.sc[((size_t)c * 9 + 3 * a + b) * t.p + col] = v;
+        t.sc[((size_t)c * 9 + 3 * b + a) * t.p + col] = v;
+    }
+}
+
 // Energy components of a group's structures: ordered sums of the sites'
 // scalar moments over each structure's atoms, and the species counts.
 // Threads [0, nc S) take the sums, one per (structure, scalar), and the
@@ -742,7 +784,7 @@ template <class P, class CP = void>
 void launch_tile_variant(const DevModel &m, const DevLin &L, const DevNeighbors &nb,
                          const LinTile &t, size_t lds_bytes, hipStream_t s)
 {
-    const int items = t.count * t.nchunks;
+    const int items = t.count * t.nchunks * t.parts;
     const unsigned grid = (unsigned)((items + 7) / 8 * 8);
     hipLaunchKernelGGL((lin_tile_kernel<P, CP>), dim3(grid), dim3(kWave), lds_bytes, s, m, L, nb,
                        t);
@@ -861,6 +903,11 @@ hipError_t launch_lin_tile(const DevModel &m, const DevLin &L, const DevNeighbor
     case 2: launch_tile_variant<ProfLevel10>(m, L, nb, t, lds, s); break;
     case 3: launch_tile_variant<ProfSmall>(m, L, nb, t, lds, s); break;
     default: launch_tile_variant<ProfGeneric>(m, L, nb, t, lds, s); break;
+    }
+    if (t.parts > 1) {
+        const unsigned elements = (unsigned)lin_part_doubles(t.rows_cap);
+        hipLaunchKernelGGL(lin_parts_kernel, dim3((elements + 255) / 256, t.count * t.nchunks),
+                           dim3(256), 0, s, L, t);
     }
     return hipGetLastError();
 }

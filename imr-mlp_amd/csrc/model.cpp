@@ -989,7 +989,6 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     p.max_partials = std::max(fwd.max_partials, bwd.max_partials);
     const int P4 = (p.max_partials + 3) & ~3;
     p.red0 = p.part0 + P4;
-    const int N4 = (p.nslots + 3) & ~3;
     // The moment reduction's transpose buffer lies over the adjoint block
     // (unused until the seeds are written; the zero slot and the partial sums
     // under it are cleared again after the neighbour pass) and the force

@@ -514,7 +514,10 @@ struct LinGroup {
 // One launch of the tile kernel: `count` structures of a group, every chunk
 // of each (one wave per structure and chunk), force rows accumulated in LDS
 // tiles of rows_cap atoms (rows_cap 0: in the rows of fc, for structures
-// larger than a tile).
+// larger than a tile).  With parts > 1 each such wave's sites are split over
+// that many waves, whose tiles and stress sums go to `part`
+// [chunk][structure][part][lin_part_doubles(rows_cap)] and are added in part
+// order by a second launch.
 struct LinTile {
     const int *structs;   // [count] structures of this launch
     int count, nchunks, rows_cap;
@@ -523,7 +526,14 @@ struct LinTile {
     int a0;               // first atom of the group
     int p, Z;
     double *fc, *sc;      // force [N][3][p] and stress [nconf][9][p] components
+    int parts = 1;
+    double *part = nullptr;
 };
+constexpr int kLinPartSites = 8;  // sites of a part, at least (of the largest structure)
+__host__ __device__ constexpr size_t lin_part_doubles(int rows)
+{
+    return (size_t)kLinChunk * (3 * (size_t)rows + 6);
+}
 bool lin_configure(const DevModel &m, const DevLin &L, int n, int num_cus, size_t lds_limit,
                    EfsLaunch &cfg);
 bool lin_walk_compiled(const LinPlan &lp, int nslots);

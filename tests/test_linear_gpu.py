@@ -400,3 +400,30 @@ def test_duplicate_scalar_mapping_rows(ctx):
     eo, fo, so = O.efs_components(m, nb)
     assert rel_err(ec[0], eo) < 1e-10 and rel_err(fc, fo) < 1e-10 and rel_err(sc[0], so) < 1e-10
     assert np.array_equal(fc[..., m.Z + 1], fc[..., m.Z + 4])
+
+
+@pytest.mark.parametrize("name,Z,R", [("shapeev-16.mtp", 2, 8), ("shapeev-20.mtp", 2, 10), ("shapeev-10.mtp", 2, 8),
+                                      ("shapeev-06.mtp", 2, 6)])
+def test_structures_split_over_waves(ctx, name, Z, R):
+    """Few structures: each structure's sites go to several waves whose tiles
+    are added afterwards.  The same structures among enough copies that every
+    wave keeps a whole structure give the same components to rounding (sums of
+    some 10^3 terms in another order: 1e-13 of the largest), and the split is
+    repeatable bit for bit.  Sizes around the eight sites of a part."""
+    rng = S.rng_for(92)
+    text = S.random_model(name, Z, R, 1.9, 5.0, -0.1, 0.1, rng)
+    structs = []
+    for n in (1, 7, 8, 9, 31, 64, 65, 130):
+        s = S.displace(S.lattice("fcc", (4, 3, 3), 3.56), rng, 0.1)
+        keep = np.sort(rng.permutation(s.n)[:n])
+        structs.append(S.Structure(s.cell, s.pos[keep], (S.uniform(rng, len(keep)) * Z).astype(np.int32), s.pbc))
+    ctx.load_model_text(text)
+    off = ctx.set_structures(structs, 5.0)
+    few, again = ctx.efs_components(), ctx.efs_components()
+    copies = 160
+    ctx.set_structures(structs * copies, 5.0)
+    many = ctx.efs_components()
+    for k, (a, b, c) in enumerate(zip(few, again, many)):
+        assert np.array_equal(a, b)
+        c = c[:off[-1] if k == 1 else len(structs)]
+        assert np.abs(a - c).max() <= 1e-13 * np.abs(a).max()
