@@ -98,7 +98,7 @@ struct NeighborStore {
     bool has_mirror = false;
 };
 struct NeighborScratch {
-    DBuf pts, orig, flags, scan, tmp, minmax, box, box_start, box_cur, box_items, rank, cnt,
+    DBuf pts, orig, flags, scan, tmp, box, box_start, box_cur, box_items, rank, cnt,
         cursor, key, st_nbr, st_ctr, st_mate, st_final, scalars;
     // per-structure tables of a batch with the positions and species (atom
     // offsets, wrap flags and cells; candidate, box, interior-box and flag
@@ -113,7 +113,7 @@ struct NeighborScratch {
     long long bin_cap = 0;
     void release_all()
     {
-        for (DBuf *b : {&pts, &orig, &flags, &scan, &tmp, &minmax, &box, &box_start, &box_cur,
+        for (DBuf *b : {&pts, &orig, &flags, &scan, &tmp, &box, &box_start, &box_cur,
                         &box_items, &rank, &cnt, &cursor, &key, &st_nbr, &st_ctr, &st_mate,
                         &st_final, &scalars, &seg_head, &seg_tabs, &seg_imgs, &seg_pts, &wrapped})
             b->release();

@@ -67,22 +67,6 @@ __global__ void box_place_kernel(const int *box, const int *npts, int *box_cur, 
     items[q] = i;
 }
 
-// One thread per point: its slot in its box is the number of the box's
-// points with a smaller index (a box of a small cell can hold every point).
-__global__ void box_rank_kernel(const int *box, const int *box_start, const int *npts,
-                                const int *unsorted, int *items)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *npts)
-        return;
-    const int b = box[i];
-    const int s = box_start[b], e = box_start[b + 1];
-    int r = 0;
-    for (int u = s; u < e; ++u)
-        r += unsorted[u] < i;
-    items[s + r] = i;
-}
-
 // Inclusive prefix sum over the 64 lanes of a wave: rows of 16 by DPP row
 // shifts (lanes without a source add 0), then each row adds the totals of
 // the rows before it (lane reads).
@@ -368,9 +352,16 @@ __host__ __device__ constexpr size_t scan_lds_bytes(int n)
     return sizeof(int) * ((size_t)n + (size_t)n / 32 + 1);
 }
 
-__global__ __launch_bounds__(kScan1Threads) void scan_one_block(const int *in, int n, int clamp,
+// A second workgroup scans in place the n values that follow in.
+__global__ __launch_bounds__(kScan1Threads) void scan_one_block(int *in, int n, int clamp,
                                                                 int *out, int *out2, int *total)
 {
+    if (blockIdx.x == 1) {
+        in += n;
+        out = in;
+        out2 = nullptr;
+        total = nullptr;
+    }
     extern __shared__ int buf[];
     __shared__ int wsum[kScan1Waves];
     const int t = threadIdx.x;
@@ -398,19 +389,22 @@ __global__ __launch_bounds__(kScan1Threads) void scan_one_block(const int *in, i
         if (out2)
             out2[i] = v;
     }
-    if (t == 0)
+    if (t == 0 && total)
         *total = tot;
 }
 
 // Exclusive scan into out (and out2 when given, which may be in: every
 // value is read before its slot is written); *total receives the sum
 // (device); returns the error.
-hipError_t scan_exclusive(const int *in, int64_t n, int *out, DBuf &tmp, int *total,
-                          hipStream_t s, int *out2 = nullptr, int clamp = INT_MAX)
+//
+// With pair, the n values after in are scanned too, in place (their sum goes
+// nowhere).
+hipError_t scan_exclusive(int *in, int64_t n, int *out, DBuf &tmp, int *total, hipStream_t s,
+                          int *out2 = nullptr, int clamp = INT_MAX, bool pair = false)
 {
     if (n <= kScanLdsMax) {
-        hipLaunchKernelGGL(scan_one_block, dim3(1), dim3(kScan1Threads), scan_lds_bytes((int)n), s,
-                           in, (int)n, clamp, out, out2, total);
+        hipLaunchKernelGGL(scan_one_block, dim3(pair ? 2 : 1), dim3(kScan1Threads),
+                           scan_lds_bytes((int)n), s, in, (int)n, clamp, out, out2, total);
         return hipGetLastError();
     }
     const int64_t ntiles = std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile);
@@ -422,6 +416,11 @@ hipError_t scan_exclusive(const int *in, int64_t n, int *out, DBuf &tmp, int *to
     hipLaunchKernelGGL(scan_sums, dim3(1), dim3(1024), 0, s, tmp.as<int>(), (int)ntiles, total);
     hipLaunchKernelGGL(scan_tiles, dim3((unsigned)ntiles), dim3(kScanBlock), 0, s, in, n, clamp,
                        tmp.as<int>(), out, out2);
+    if (pair) {  // (the total is overwritten: callers that pair do not read it)
+        const hipError_t pe = scan_exclusive(in + n, n, in + n, tmp, total, s, nullptr, clamp);
+        if (pe != hipSuccess)
+            return pe;
+    }
     return hipGetLastError();
 }
 
@@ -655,7 +654,7 @@ hipError_t launch_site_prepare(int nrows, const int *offsets, const int *center_
 //
 // Every kernel runs over the concatenation of a chunk's structures with a
 // table of per-structure offsets (atoms, points, image flags, image
-// candidates, box counters with one closing counter each, interior boxes)
+// candidates, box counters with one closing counter each)
 // and geometry; a thread finds its structure by binary search over the
 // offsets.  Points are numbered structure by structure (originals, then
 // images), atoms and list entries over the chunk, so the lists come out as
@@ -673,7 +672,7 @@ struct SegGeom {      // per structure, after the AABB
 
 struct Seg {
     int nconf;
-    const int *atom_off, *pt_off, *cand_off, *box_off, *int_off;  // [nconf + 1]
+    const int *atom_off, *pt_off, *cand_off, *box_off;            // [nconf + 1]
     const long long *flag_off;                                    // [nconf + 1]
     const Cell *cell;                                             // [nconf]
     const int *wrap;                                              // [nconf]
@@ -919,7 +918,8 @@ __device__ __forceinline__ int box_of(const SegGeom &b, int d, double x, bool or
     return v;
 }
 
-__global__ void box_index_kernel(Seg g, const double *pts, int *box, int *box_count)
+// Counts each box's points and, in ocount, its originals.
+__global__ void box_index_kernel(Seg g, const double *pts, int *box, int *box_count, int *ocount)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= g.pt_off[g.nconf])
@@ -935,70 +935,34 @@ __global__ void box_index_kernel(Seg g, const double *pts, int *box, int *box_co
     const int gb = g.box_off[c] + (ix[0] * b.bl[1] + ix[1]) * b.bl[2] + ix[2];
     box[p] = gb;
     atomicAdd(&box_count[gb], 1);
+    if (original)
+        atomicAdd(&ocount[gb], 1);
 }
 
-// interior box w of structure c (walk order i, j, k from 1)
-__device__ __forceinline__ int interior_box(const SegGeom &b, int w)
+// One thread per point: its slot in its box is the number of the box's
+// points with a smaller index (a box of a small cell can hold every point).
+// The originals come first in their box, and they lie in interior boxes,
+// whose walk order is the order of the boxes: an original's processing rank
+// is the originals in the boxes before (obefore) plus its slot.
+__global__ void box_rank_kernel(Seg g, const int *box, const int *box_start, const int *obefore,
+                                const int *orig, const int *unsorted, int *items, int *rank,
+                                int *centre_box)
 {
-    const int nj = b.bl[1] - 2, nk = b.bl[2] - 2;
-    const int i = w / (nj * nk) + 1, j = (w / nk) % nj + 1, k = w % nk + 1;
-    return (i * b.bl[1] + j) * b.bl[2] + k;
-}
-
-// Originals in interior box w (walk order over the chunk), and its box
-// within the structure (bl) and over the chunk (gb).
-__device__ __forceinline__ int interior_originals(const Seg &g, const int *box_start,
-                                                  const int *items, int w, int &c, int &bl,
-                                                  int &gb)
-{
-    c = seg_of(g.int_off, g.nconf, w);
-    bl = interior_box(g.geo[c], w - g.int_off[c]);
-    gb = g.box_off[c] + bl;
-    const int lim = g.pt_off[c] + (g.atom_off[c + 1] - g.atom_off[c]);
-    int k = 0;
-    for (int q = box_start[gb]; q < box_start[gb + 1]; ++q)
-        k += items[q] < lim;
-    return k;
-}
-
-// The originals of interior box w take the processing ranks prefix,
-// prefix + 1, ... in box order.
-__device__ __forceinline__ void rank_interior(const Seg &g, const int *box_start,
-                                              const int *items, int c, int bl, int gb, int r,
-                                              int *rank, int *centre_box)
-{
-    const int p0 = g.pt_off[c], lim = p0 + (g.atom_off[c + 1] - g.atom_off[c]);
-    for (int q = box_start[gb]; q < box_start[gb + 1]; ++q) {
-        const int p = items[q];
-        if (p < lim) {
-            const int a = g.atom_off[c] + (p - p0);
-            rank[a] = r++;
-            centre_box[a] = bl;
-        }
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= g.pt_off[g.nconf])
+        return;
+    const int b = box[i];
+    const int s = box_start[b], e = box_start[b + 1];
+    int r = 0;
+    for (int u = s; u < e; ++u)
+        r += unsorted[u] < i;
+    items[s + r] = i;
+    const int c = seg_of(g.pt_off, g.nconf, i);
+    if (i - g.pt_off[c] < g.atom_off[c + 1] - g.atom_off[c]) {
+        const int a = orig[i];
+        rank[a] = obefore[b] + r;
+        centre_box[a] = b - g.box_off[c];
     }
-}
-
-// Originals per interior box, in the lexicographic walk order of construct().
-__global__ void interior_count_kernel(Seg g, const int *box_start, const int *items,
-                                            int nint, int *count)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nint)
-        return;
-    int c, bl, gb;
-    count[w] = interior_originals(g, box_start, items, w, c, bl, gb);
-}
-
-// Processing rank of every original: prefix over interior boxes + slot.
-__global__ void centre_rank_kernel(Seg g, const int *box_start, const int *items,
-                                         const int *prefix, int nint, int *rank, int *centre_box)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nint)
-        return;
-    int c, bl, gb;
-    (void)interior_originals(g, box_start, items, w, c, bl, gb);
-    rank_interior(g, box_start, items, c, bl, gb, prefix[w], rank, centre_box);
 }
 
 struct Construct {
@@ -1540,7 +1504,7 @@ __global__ void zero_counts_kernel(int *cnt, int n, unsigned long long *z64, int
 }
 
 // Budgets of one chunk: its atoms (set before the build), its image flags,
-// boxes and interior boxes (the chunk ends early at the structure that would
+// boxes (the chunk ends early at the structure that would
 // pass them), so every point, box and flag index fits in int32.
 constexpr int kChunkAtoms = 1 << 21;
 // Point buffers sized by the bound ntot + nflags up to this many points
@@ -1805,7 +1769,7 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
             return fail_at(c, "singular cell", MTPX_E_INVALID);
     }
     // scalars: [0] scan totals, [8..9] the 64-bit entry total, [10] bin
-    // overflow, [11] longest list, [12] entry total of a one-pass build
+    // overflow, [11] longest list, [12] scan total of a one-pass build
     DTRY(w.scalars.ensure(sizeof(int) * 16));
     int *scal = w.scalars.as<int>();
     // the structure tables: one copy; the positions and species are staged
@@ -1837,11 +1801,13 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
         nmax = std::max(nmax, atom_off[c + 1] - atom_off[c]);
     const int B = std::min(64, std::max(1, (nmax + 2047) / 2048));
     const size_t npart = 6 * (size_t)nconf * B;
-    DTRY(w.minmax.ensure(sizeof(double) * npart));
-    DTRY(w.down.ensure(sizeof(double) * npart));
+    DTRY(w.down.ensure(sizeof(double) * std::max<size_t>(npart, 8)));
+    void *hdown = nullptr;  // pinned: the kernel writes the partials there
+    DTRY(hipHostGetDevicePointer(&hdown, w.down.p, 0));
     hipLaunchKernelGGL(wrap_minmax_kernel, dim3((unsigned)((size_t)nconf * B)), dim3(256), 0, s, g,
-                       dpos, dtypes_host, B, wr, w.minmax.as<double>(), out.center_type.as<int>());
-    DTRY(hipMemcpyAsync(w.down.p, w.minmax.p, sizeof(double) * npart, hipMemcpyDeviceToHost, s));
+                       dpos, dtypes_host, B, wr, static_cast<double *>(hdown),
+                       out.center_type.as<int>());
+    DTRY(hipGetLastError());
     DTRY(hipStreamSynchronize(s));
     const double *part = w.down.as<double>();
     std::vector<double> mm(6 * (size_t)nconf);
@@ -1861,7 +1827,7 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     // per structure: AABB with the extent fix, image candidates, boxes
     std::vector<SegGeom> geo((size_t)nconf);
     std::vector<double> cand, cc;
-    std::vector<int> cand_off(1, 0), box_off(1, 0), int_off(1, 0);
+    std::vector<int> cand_off(1, 0), box_off(1, 0);
     std::vector<long long> flag_off(1, 0);
     for (int c = 0; c < nconf; ++c) {
         const int n = atom_off[c + 1] - atom_off[c];
@@ -1869,7 +1835,7 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
         gc = SegGeom{};
         gc.cutoff = cutoff;
         long long nflag = 0;
-        long long nbox = 0, nint = 0;
+        long long nbox = 0;
         if (n > 0) {
             for (int d = 0; d < 3; ++d) {
                 gc.lo[d] = mm[6 * (size_t)c + d];
@@ -1899,11 +1865,9 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
             if (nbox > INT_MAX / 2)
                 return fail_at(c, "Neighbor spatial box count exceeds integer range",
                                MTPX_E_RANGE);
-            nint = (long long)(gc.bl[0] - 2) * (gc.bl[1] - 2) * (gc.bl[2] - 2);
             nbox += 1;  // the structure's closing counter
         }
-        if (flag_off.back() + nflag > kChunkFlags || box_off.back() + nbox > kChunkBoxes ||
-            int_off.back() + nint > kChunkBoxes) {
+        if (flag_off.back() + nflag > kChunkFlags || box_off.back() + nbox > kChunkBoxes) {
             if (c == 0)
                 return fail_at(c, "too many periodic images or boxes for the neighbour builder",
                                MTPX_E_CAPACITY);
@@ -1915,7 +1879,6 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
         cand_off.push_back((int)(cand.size() / 3));
         flag_off.push_back(flag_off.back() + nflag);
         box_off.push_back(box_off.back() + (int)nbox);
-        int_off.push_back(int_off.back() + (int)nint);
     }
     if (nconf < c1 - c0) {
         *done = nconf;
@@ -1924,15 +1887,14 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
         g.nconf = nconf;
     }
     const long long nflags = flag_off.back();
-    const int nboxes = box_off.back(), nint = int_off.back();
+    const int nboxes = box_off.back();
     Upload tabs;
     const size_t o_cand_off = tabs.add(cand_off), o_box_off = tabs.add(box_off),
-                 o_int_off = tabs.add(int_off), o_flag_off = tabs.add(flag_off),
+                 o_flag_off = tabs.add(flag_off),
                  o_geo = tabs.add(geo.data(), (size_t)nconf), o_cand = tabs.add(cand);
     DTRY(tabs.send(w.up_tabs, w.seg_tabs, s));
     g.cand_off = at<int>(w.seg_tabs, o_cand_off);
     g.box_off = at<int>(w.seg_tabs, o_box_off);
-    g.int_off = at<int>(w.seg_tabs, o_int_off);
     g.flag_off = at<long long>(w.seg_tabs, o_flag_off);
     g.geo = at<SegGeom>(w.seg_tabs, o_geo);
     g.cand = at<double>(w.seg_tabs, o_cand);
@@ -1982,14 +1944,15 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     }
     DTRY(w.pts.ensure(sizeof(double) * 3 * (size_t)npts_max));
     DTRY(w.orig.ensure(sizeof(int) * (size_t)npts_max));
-    DTRY(w.cnt.ensure(sizeof(int) * ((size_t)nboxes + 1)));
+    DTRY(w.cnt.ensure(sizeof(int) * 2 * ((size_t)nboxes + 1)));
     DTRY(w.cursor.ensure(sizeof(int) * ((size_t)ntot + 1)));
     int *box_count = w.cnt.as<int>();
+    int *ocount = box_count + (nboxes + 1);
     int *cnt = w.cursor.as<int>();
     unsigned long long *total64 = reinterpret_cast<unsigned long long *>(scal + 8);
     hipLaunchKernelGGL(points_kernel, dim3(blocks(std::max<long long>(ntot, nflags), 256)),
                        dim3(256), 0, s, g, wr, ntot, nflags, w.flags.as<int>(), w.scan.as<int>(),
-                       w.pts.as<double>(), w.orig.as<int>(), box_count, nboxes + 1, cnt, ntot + 1,
+                       w.pts.as<double>(), w.orig.as<int>(), box_count, 2 * (nboxes + 1), cnt, ntot + 1,
                        total64, scal + 10);
 
     // boxes: counts, starts, stable placement
@@ -1998,33 +1961,22 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     DTRY(w.box_cur.ensure(sizeof(int) * ((size_t)nboxes + 1)));
     DTRY(w.box_items.ensure(sizeof(int) * (size_t)npts_max));
     hipLaunchKernelGGL(box_index_kernel, dim3(blocks(npts_max, 256)), dim3(256), 0, s, g,
-                       w.pts.as<double>(), w.box.as<int>(), box_count);
+                       w.pts.as<double>(), w.box.as<int>(), box_count, ocount);
     DTRY(scan_exclusive(box_count, (int64_t)nboxes + 1, w.box_start.as<int>(), w.tmp,
-                        w.scalars.as<int>(), s, w.box_cur.as<int>()));
+                        w.scalars.as<int>(), s, w.box_cur.as<int>(), INT_MAX, true));
     // the image flags are dead after points_kernel: their buffer takes
     // the unsorted placement (growing it waits for the queued work)
     DTRY(w.flags.ensure(sizeof(int) * (size_t)std::max<long long>(npts_max, 1)));
     int *unsorted = w.flags.as<int>();
     hipLaunchKernelGGL(box_place_kernel, dim3(blocks(npts_max, 256)), dim3(256), 0, s,
                        w.box.as<int>(), npts, w.box_cur.as<int>(), unsorted);
-    hipLaunchKernelGGL(box_rank_kernel, dim3(blocks(npts_max, 256)), dim3(256), 0, s,
-                       w.box.as<int>(), w.box_start.as<int>(), npts, unsorted,
-                       w.box_items.as<int>());
-
-    // processing ranks of the centres
-    DTRY(w.rank.ensure(sizeof(int) * (2 * (size_t)ntot + 2 * ((size_t)nint + 1))));
+    // the slots, and the processing ranks of the centres
+    DTRY(w.rank.ensure(sizeof(int) * 2 * (size_t)ntot));
     int *rank = w.rank.as<int>();
     int *centre_box = rank + ntot;
-    int *icount = centre_box + ntot;
-    int *iprefix = icount + (nint + 1);
-    if (nint > 0) {
-        hipLaunchKernelGGL(interior_count_kernel, dim3(blocks(nint, 256)), dim3(256), 0, s,
-                           g, w.box_start.as<int>(), w.box_items.as<int>(), nint, icount);
-        DTRY(scan_exclusive(icount, nint, iprefix, w.tmp, scal, s));
-        hipLaunchKernelGGL(centre_rank_kernel, dim3(blocks(nint, 256)), dim3(256), 0, s, g,
-                           w.box_start.as<int>(), w.box_items.as<int>(), iprefix, nint, rank,
-                           centre_box);
-    }
+    hipLaunchKernelGGL(box_rank_kernel, dim3(blocks(npts_max, 256)), dim3(256), 0, s, g,
+                       w.box.as<int>(), w.box_start.as<int>(), ocount, w.orig.as<int>(), unsorted,
+                       w.box_items.as<int>(), rank, centre_box);
 
     // construct: count, offsets, fill, rank within lists
     Construct cb;
@@ -2040,7 +1992,6 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     cb.cap = 0;
     cb.overflow = scal + 10;
     cb.mate = nullptr;  // set once the staging is sized
-    DTRY(w.down.ensure(sizeof(int) * 16));
     int *down = w.down.as<int>();
     // One pass into bins sized from the previous counted build: the entry
     // total comes back with the final synchronisation.  A list that outgrows
@@ -2055,12 +2006,11 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
                            w.st_ctr.as<int>());
         DTRY(scan_exclusive(cnt, (int64_t)ntot + 1, out.offsets.as<int>(), w.tmp, scal + 12, s,
                             nullptr, (int)cap));
-        rank_lists(out, w, ntot, nullptr, (int)cap, scal + 10, nullptr, s);
-        DTRY(hipMemcpyAsync(down, scal + 10, sizeof(int) * 3, hipMemcpyDeviceToHost, s));
+        rank_lists(out, w, ntot, nullptr, (int)cap, scal + 10, static_cast<int *>(hdown), s);
         DTRY(hipGetLastError());
         DTRY(hipStreamSynchronize(s));
         if (down[0] == 0) {
-            out.P = down[2];
+            out.P = down[1];
             out.has_mirror = true;
             return MTPX_OK;
         }
