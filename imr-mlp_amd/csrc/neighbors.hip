@@ -1164,7 +1164,7 @@ __global__ __launch_bounds__(256) void construct_kernel(Seg g, Construct cb, int
 // ---- small structures: the whole preparation in one workgroup -------------
 //
 // A fully periodic structure of at most kSmallAtoms atoms needs about a
-// microsecond of work in each of the eleven launches from the wrap to the
+// microsecond of work in each of the eight launches from the wrap to the
 // centre ranks, but every launch costs about five, and the host waits for the
 // AABB in between.  One workgroup of 16 waves does all of it with the
 // positions, image tests and box counters in LDS, and the host gives it only
@@ -1604,8 +1604,8 @@ void rank_lists(NeighborStore &out, NeighborScratch &w, int ntot, const int *cnt
 }
 
 // One fully periodic structure of n <= kSmallAtoms atoms: four launches and
-// one synchronisation (3,072 atoms: 99 us a build, 152 the general way with its
-// fourteen launches and two synchronisations; 1,000 atoms 66 us, of which 27 in
+// one synchronisation (3,072 atoms: 99 us a build, 135 the general way with its
+// eleven launches and two synchronisations; 1,000 atoms 66 us, of which 27 in
 // the preparation, bound by latency and the one CU).  *built stays false when the
 // structure does not fit the limits or a list its bin; it is then built the
 // general way, which also reports every error.
@@ -1795,11 +1795,13 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     g.cell = at<Cell>(w.seg_head, o_cell);
     DTRY(w.wrapped.ensure(sizeof(double) * 3 * (size_t)ntot));
     double *wr = w.wrapped.as<double>();
-    // workgroups per structure: about 2048 atoms each, at most 64
+    // workgroups per structure: about 512 atoms each, at most 64 (two round
+    // trips to the pinned positions a thread; 32,000 atoms: 22 us, 28 with
+    // eight round trips)
     int nmax = 0;
     for (int c = 0; c < nconf; ++c)
         nmax = std::max(nmax, atom_off[c + 1] - atom_off[c]);
-    const int B = std::min(64, std::max(1, (nmax + 2047) / 2048));
+    const int B = std::min(64, std::max(1, (nmax + 511) / 512));
     const size_t npart = 6 * (size_t)nconf * B;
     DTRY(w.down.ensure(sizeof(double) * std::max<size_t>(npart, 8)));
     void *hdown = nullptr;  // pinned: the kernel writes the partials there
