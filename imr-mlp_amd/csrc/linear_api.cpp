@@ -196,19 +196,20 @@ int run_lin(mtpx_context *ctx)
             t.sc = comp + cl.sc;
             // A class of few structures leaves most of the chip idle while its
             // waves walk their sites one after the other (3.6 us a site): its
-            // sites are split until there is a wave for every place (one per
-            // SIMD and as many tiles as the LDS holds), down to eight sites a
-            // wave, below which clearing and adding the tiles costs more than
-            // the walk.  The class counts over all groups, so that grouping
-            // changes no sum.  One structure of 650 atoms, 16 chunks: 2.35 ms
+            // sites are split until there are two waves for every place (one
+            // per SIMD and as many tiles as the LDS holds; two even out the
+            // structures' sizes: 60 structures 802 us a call unsplit, 553 with
+            // two, 557 with three), down to eight sites a wave, below which
+            // clearing and adding the tiles costs more than the walk.  The
+            // class counts over all groups, so that grouping changes no sum.  One structure of 650 atoms, 16 chunks: 2.35 ms
             // on 16 waves, 0.18 on 256 and 0.01 for the sums; normal
-            // equations of 4 structures of 100 atoms 724 -> 199 us a call.
+            // equations of 4 structures of 100 atoms 724 -> 206 us a call.
             if (lds_tile && t.count > 0) {
                 const int places =
                     ctx->num_cus *
                     (int)std::clamp<size_t>(ctx->lds_limit / lin_tile_lds(m, L, t.rows_cap), 1, 4);
                 const int64_t items = (int64_t)cls_count[k] * t.nchunks;
-                t.parts = (int)std::clamp<int64_t>(places / items, 1,
+                t.parts = (int)std::clamp<int64_t>((2 * places + items - 1) / items, 1,
                                                    std::max(1, t.rows_cap / kLinPartSites));
                 if (t.parts > 1) {
                     HIP_TRY(ctx->lin_part.ensure(sizeof(double) * lin_part_doubles(t.rows_cap) * items *
