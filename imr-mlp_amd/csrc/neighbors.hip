@@ -1604,7 +1604,7 @@ void rank_lists(NeighborStore &out, NeighborScratch &w, int ntot, const int *cnt
 }
 
 // One fully periodic structure of n <= kSmallAtoms atoms: four launches and
-// one synchronisation (3,072 atoms: 99 us a build, 135 the general way with its
+// one synchronisation (3,072 atoms: 99 us a build, 119 the general way with its
 // eleven launches and two synchronisations; 1,000 atoms 66 us, of which 27 in
 // the preparation, bound by latency and the one CU).  *built stays false when the
 // structure does not fit the limits or a list its bin; it is then built the
@@ -1617,10 +1617,12 @@ int build_small(const double cell[9], const int pbc[3], int n, const double *pos
     std::copy(cell, cell + 9, a.cell.m);
     // a wrapped point lies in the cell, so the AABB spans at most the sum of
     // the vectors' components (or the cutoff, to which it is widened)
-    double ext[3], volume;
+    double ext[3], volume, boxes = 1, reach = 1;
     for (int d = 0; d < 3; ++d) {
         const double span = std::fabs(cell[d]) + std::fabs(cell[3 + d]) + std::fabs(cell[6 + d]);
         ext[d] = std::max(span * (1 + 1e-6), cutoff) + cutoff;
+        boxes *= std::floor(ext[d] / cutoff) + 1;
+        reach *= ext[d] + cutoff;
     }
     std::string none;
     int dims;
@@ -1640,6 +1642,22 @@ int build_small(const double cell[9], const int pbc[3], int n, const double *pos
     volume = std::fabs(cell[0] * (cell[4] * cell[8] - cell[5] * cell[7]) -
                        cell[1] * (cell[3] * cell[8] - cell[5] * cell[6]) +
                        cell[2] * (cell[3] * cell[7] - cell[4] * cell[6]));
+    // A cell that its atoms fill must fit the kernel's limits, so that the
+    // attempt is not made in vain on every call: the boxes, the images that
+    // reach the cell's bounding box and their points at the mean density.
+    int images = 0;
+    for (int i2 = -a.rng[2]; i2 <= a.rng[2]; ++i2)
+        for (int i1 = -a.rng[1]; i1 <= a.rng[1]; ++i1)
+            for (int i0 = -a.rng[0]; i0 <= a.rng[0]; ++i0) {
+                bool in = true;
+                for (int d = 0; d < 3; ++d)
+                    in = in && std::fabs(a.basis[3 * d] * i0 + a.basis[3 * d + 1] * i1 +
+                                         a.basis[3 * d + 2] * i2) <= ext[d];
+                images += in;
+            }
+    if (!(boxes <= kSmallBoxes) || images > kSmallImages ||
+        (long)images * ((n + 63) / 64) > kSmallUnits || !(n / volume * reach <= kSmallPoints))
+        return MTPX_OK;
     // bins sized from the previous build, or one and a half times the mean
     // list and a margin when there is none
     long long cap = w.bin_cap;
