@@ -62,7 +62,7 @@ def sources():
 
 
 def _newest_header() -> float:
-    hs = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hpp")]
+    hs = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hpp", ".inc"))]
     hs.append(os.path.join(ROOT, "include", "mtpx.h"))
     return max(os.path.getmtime(h) for h in hs)
 

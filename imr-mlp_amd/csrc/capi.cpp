@@ -122,8 +122,7 @@ void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm,
     dm.efs_head = P.efs_head;
     dm.head = M.head.kind;
     dm.hd = nullptr;
-    dm.tr_red1 = P.tr_red1;
-    dm.tr_red4 = P.tr_red4;
+    dm.tr_red = P.tr_red;
     dm.tr_stage = P.tr_stage;
     dm.tr_grad = P.tr_grad;
     dm.tr_ctype = P.tr_ctype;
@@ -132,7 +131,6 @@ void fill_model_sizes(const Model &M, const Plan &P, DevModel &dm,
     dm.ncoef = M.ncoef();
     dm.rb_general = M.general_basis() ? 1 : 0;
     dm.rb_table = nullptr;
-    std::memcpy(dm.slot_base, P.slot_base, sizeof dm.slot_base);
     moment_table(M, P, efs_profile_degree(dm), mono, shift, dm.mono_groups);
     dm.nmono = (int)mono.size();
     dm.fwd_nsteps = (int)(P.fwd_steps.size() / (2 * kWave));
@@ -154,7 +152,31 @@ int install_model(mtpx_context *ctx, Model &&m)
     std::vector<unsigned> shift;
     fill_model_sizes(m, p, dm, mono, shift);
     EfsLaunch probe;
-    if (!efs_configure(dm, 1, 1, 0, ctx->lds_limit, probe))
+    // linear-fit plan: optional (the linear entry points report its error)
+    LinPlan lin;
+    std::string lin_err;
+    const bool lin_ok = build_lin_plan(m, p, lin, lin_err);
+    DevLin lin_sizes{};
+    lin_sizes.priv = lin.priv;
+    lin_sizes.lane_walk = lin.lane_walk ? 1 : 0;
+    // The moment tables go to LDS unless one of the kernels then has no room
+    // for a wave that it has without them.
+    auto only_without = [&](auto fits) {
+        dm.mono_lds = 1;
+        if (fits())
+            return false;
+        dm.mono_lds = 0;
+        return fits();
+    };
+    auto efs_fits = [&] { return efs_configure(dm, 1, 1, 0, ctx->lds_limit, probe); };
+    const bool outside =
+        only_without(efs_fits) ||
+        only_without([&] { return grad_configure(dm, 1, 1, ctx->lds_limit, probe); }) ||
+        (lin_ok && only_without([&] {
+             return lin_configure(dm, lin_sizes, 1, 1, ctx->lds_limit, probe);
+         }));
+    dm.mono_lds = outside ? 0 : 1;
+    if (!efs_fits())
         return set_error(ctx, MTPX_E_CAPACITY, "model needs more LDS than a CU provides");
     // From here on the old model is gone: until every upload has succeeded the
     // context holds no model (a failed upload leaves MTPX_E_NO_MODEL behind,
@@ -165,6 +187,8 @@ int install_model(mtpx_context *ctx, Model &&m)
     ctx->has_adjoints = false;
     ctx->model = std::move(m);
     ctx->plan = std::move(p);
+    ctx->lin = std::move(lin);
+    ctx->lin_err = std::move(lin_err);
     const Model &M = ctx->model;
     const Plan &P = ctx->plan;
     hipStream_t s = ctx->stream;
@@ -175,11 +199,10 @@ int install_model(mtpx_context *ctx, Model &&m)
         std::memcpy(packed.data() + at, v.data(), v.size() * sizeof v[0]);
     };
     pack(o.map, M.map);
-    pack(o.slot, P.slot_basic);
     pack(o.force, P.force_basic);
     pack(o.mono, mono);
-    pack(o.fwd, device_steps(P.fwd_steps, P.fwd_level_step, P.fwd_comb, P.fwd_level_comb));
-    pack(o.bwd, device_steps(P.bwd_steps, P.bwd_level_step, P.bwd_comb, P.bwd_level_comb));
+    pack(o.fwd, P.fwd_steps);
+    pack(o.bwd, P.bwd_steps);
     HIP_TRY(upload(ctx->shared, packed, s), "upload model");
     HIP_TRY(upload(ctx->mono_shift, shift, s), "upload model");
     HIP_TRY(upload(ctx->dup, P.dup, s), "upload model");
@@ -228,7 +251,6 @@ int install_model(mtpx_context *ctx, Model &&m)
     dm.seed = base + o.seed;
     dm.moment = base + o.moment;
     dm.map = reinterpret_cast<int *>(base + o.map);
-    dm.slot_basic = reinterpret_cast<int *>(base + o.slot);
     dm.force_basic = reinterpret_cast<int *>(base + o.force);
     dm.mono_tab = reinterpret_cast<unsigned short *>(base + o.mono);
     dm.fwd_steps = reinterpret_cast<int2 *>(base + o.fwd);
@@ -237,14 +259,10 @@ int install_model(mtpx_context *ctx, Model &&m)
     dm.dup = ctx->dup.as<int>();
     dm.fwd_level_step = ctx->fwd_level.as<int>();
     dm.bwd_level_step = ctx->bwd_level.as<int>();
-    // linear-fit plan: optional (the linear entry points report its error)
-    const bool lin_ok = build_lin_plan(M, P, ctx->lin, ctx->lin_err);
     if (lin_ok) {
         const LinPlan &lp = ctx->lin;
         HIP_TRY(upload(ctx->lin_level, lp.level_step, s), "upload model");
-        HIP_TRY(upload(ctx->lin_steps,
-                       device_steps(lp.steps, lp.level_step, lp.comb, lp.level_comb), s),
-                "upload model");
+        HIP_TRY(upload(ctx->lin_steps, lp.steps, s), "upload model");
         HIP_TRY(upload(ctx->lin_ent, lp.slot_L, s), "upload model");
         HIP_TRY(upload(ctx->lin_estart, lp.slot_mask, s), "upload model");
         HIP_TRY(upload(ctx->lin_chunk, lp.chunk_s0, s), "upload model");
@@ -254,9 +272,7 @@ int install_model(mtpx_context *ctx, Model &&m)
         HIP_TRY(upload(ctx->lin_walk, lp.walk, s), "upload model");
         HIP_TRY(upload(ctx->lin_walk_off, lp.walk_off, s), "upload model");
         HIP_TRY(upload(ctx->lin_flevel, lp.fwd_level_step, s), "upload model");
-        HIP_TRY(upload(ctx->lin_fsteps,
-                       device_steps(lp.fwd_steps, lp.fwd_level_step, lp.fwd_comb, lp.fwd_level_comb), s),
-                "upload model");
+        HIP_TRY(upload(ctx->lin_fsteps, lp.fwd_steps, s), "upload model");
         DevLin &L = ctx->dl;
         L.dummy = lp.dummy;
         L.red0 = lp.red0;
@@ -266,8 +282,6 @@ int install_model(mtpx_context *ctx, Model &&m)
         L.nL = lp.nL;
         L.one = lp.one;
         L.L0 = lp.L0;
-        L.part0 = lp.part0;
-        L.acc = lp.acc;
         L.priv = lp.priv;
         L.CH = lp.CH;
         L.nchunks = lp.nchunks;

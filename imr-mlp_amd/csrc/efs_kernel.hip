@@ -47,10 +47,18 @@ namespace mtpx {
 
 namespace {
 
-template <class P, bool kTabLds, int kMaxWaves, bool kHead>
+// Where the tables that not every model has LDS for lie.
+enum TablePlace {
+    kStepsLds,     // moment and step tables in LDS
+    kMomentsLds,   // moment tables in LDS, step tables in global memory
+    kTablesGlobal  // both in global memory (DevModel::mono_lds 0)
+};
+
+template <class P, TablePlace kTabs, int kMaxWaves, bool kHead>
 __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNeighbors nb,
                                                                EfsOut out, int flags)
 {
+    constexpr bool kTabLds = kTabs == kStepsLds;
     const bool deterministic = flags & kEfsDeterministic;
     extern __shared__ double lds[];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
@@ -69,6 +77,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
     using Steps = std::conditional_t<kTabLds, LdsSteps, GlobalSteps>;
     const Steps fwd_tab(kTabLds ? L.fwd_steps : m.fwd_steps, lane);
     const Steps bwd_tab(kTabLds ? L.bwd_steps : m.bwd_steps, lane);
+    const MonoTab<kTabs != kTablesGlobal> mono(m, L.mono);
 
     const int row = blockIdx.x * nwaves + wave;
     for (int i = row; i < nb.n; i += gridDim.x * nwaves) {
@@ -85,7 +94,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNe
             Nbr<P::M> q;
             const bool valid = lane < n - base;
             load_neighbor<P>(m, nb, L.coef, ti, beg + base + lane, valid, q);
-            add_moments<P>(m, red, L.mono, mom, q, n - base, lane);
+            add_moments<P>(m, red, mono, mom, q, n - base, lane);
         }
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
@@ -413,24 +422,25 @@ template <class P>
 void launch_variant(const DevModel &m, const DevNeighbors &nb, const EfsOut &out,
                     const EfsLaunch &cfg, int det, hipStream_t s)
 {
-    // MTP-M heads get kernels of their own: a linear model's kernel holds no
-    // call of the out-of-line head (a call site costs registers and a stack)
     constexpr int W = VariantWaves<P>::value;
     const dim3 grid(cfg.grid), block(kWave * cfg.waves);
-    if (m.head) {
-        if (cfg.lds_tables)
-            hipLaunchKernelGGL((efs_kernel<P, true, W, true>), grid, block, cfg.lds_bytes, s, m,
+    // MTP-M heads get kernels of their own: a linear model's kernel holds no
+    // call of the out-of-line head (a call site costs registers and a stack)
+    auto launch = [&](auto tabs) {
+        constexpr TablePlace kTabs = decltype(tabs)::value;
+        if (m.head)
+            hipLaunchKernelGGL((efs_kernel<P, kTabs, W, true>), grid, block, cfg.lds_bytes, s, m,
                                nb, out, det);
         else
-            hipLaunchKernelGGL((efs_kernel<P, false, W, true>), grid, block, cfg.lds_bytes, s, m,
+            hipLaunchKernelGGL((efs_kernel<P, kTabs, W, false>), grid, block, cfg.lds_bytes, s, m,
                                nb, out, det);
-    } else if (cfg.lds_tables) {
-        hipLaunchKernelGGL((efs_kernel<P, true, W, false>), grid, block, cfg.lds_bytes, s, m, nb,
-                           out, det);
-    } else {
-        hipLaunchKernelGGL((efs_kernel<P, false, W, false>), grid, block, cfg.lds_bytes, s, m, nb,
-                           out, det);
-    }
+    };
+    if (cfg.lds_tables)
+        launch(std::integral_constant<TablePlace, kStepsLds>{});
+    else if (m.mono_lds)
+        launch(std::integral_constant<TablePlace, kMomentsLds>{});
+    else
+        launch(std::integral_constant<TablePlace, kTablesGlobal>{});
 }
 
 int variant_max_waves(int v)

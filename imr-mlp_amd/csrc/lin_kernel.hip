@@ -351,6 +351,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void lin_jac_kernel(DevModel m, D
     double *mom = ws, *red = ws + L.red0;
 
     stage_shared(m, Ls, false, tid, blockDim.x);
+    const MonoTab<false> mono(m, Ls.mono);
     if (lane == 0)
         ws[L.dummy] = 0.0;
     // the walk order's work-space indices, the same for every site: held in
@@ -375,7 +376,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void lin_jac_kernel(DevModel m, D
         for (int base = 0; base < n; base += kWave) {
             Nbr<P::M> q;
             load_neighbor<P>(m, nb, Ls.coef, ti, beg + base + lane, lane < n - base, q);
-            add_moments<P>(m, red, Ls.mono, mom, q, n - base, lane);
+            add_moments<P>(m, red, mono, mom, q, n - base, lane);
         }
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)

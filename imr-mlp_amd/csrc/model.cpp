@@ -110,26 +110,22 @@ bool fail(std::string &err, const char *msg)
 }
 
 // ---- lane-major step tables (shared by the rule plans) -------------------
-// A step entry before encoding: {l, r, c, w, first}; w >= 0 is the task's
-// target, w <= -2 partial -w - 2.
+// A step entry before encoding: {l, r, c, w, first}, w the task's target.
 using Ent = std::array<int, 5>;
 using Task = std::vector<Ent>;
 struct RawTables {
     std::vector<Ent> steps;                 // lane-major
     std::vector<int> level_step;            // per level: first step
-    std::vector<std::array<int, 3>> comb;   // {target, first partial, count}
-    std::vector<int> level_comb;
-    int max_partials = 0;
-    RawTables() : level_step{0}, level_comb{0} {}
+    RawTables() : level_step{0} {}
 };
 
-// One dependency level: tasks longer than a cap are split into pieces
-// ending in partial sums, the pieces are spread over the 64 lanes by
+// One dependency level: tasks longer than a cap are split into pieces, which
+// all add to the task's target, the pieces are spread over the 64 lanes by
 // longest-processing-time, and the level takes as many steps as its
 // longest lane.  The cap is the one, from the fair share (entries / 64, at
 // least kMinPiece) up to the longest task, that gives the fewest steps and
-// then the fewest partial sums: a split that does not shorten the level
-// only adds combine work.
+// then the fewest pieces: a split that does not shorten the level only adds
+// additions.
 void emit_level(std::vector<Task> &tasks, RawTables &raw)
 {
     size_t total = 0, longest = 0;
@@ -139,8 +135,7 @@ void emit_level(std::vector<Task> &tasks, RawTables &raw)
     }
     struct Layout {
         std::vector<Task> pieces;
-        std::vector<std::array<int, 3>> comb;  // target, first partial, count
-        int npart = 0;
+        int npart = 0;  // pieces of split tasks
         std::vector<Task> lane;
         size_t nst = 0;
     };
@@ -151,17 +146,12 @@ void emit_level(std::vector<Task> &tasks, RawTables &raw)
                 L.pieces.push_back(t);
                 continue;
             }
-            const int target = t[0][3];
-            const int first = L.npart;
             for (size_t b0 = 0; b0 < t.size(); b0 += cap) {
                 Task piece(t.begin() + b0, t.begin() + std::min(t.size(), b0 + cap));
-                for (Ent &e : piece)
-                    e[3] = -2 - L.npart;
                 piece[0][4] = 1;
                 ++L.npart;
                 L.pieces.push_back(std::move(piece));
             }
-            L.comb.push_back({target, first, L.npart - first});
         }
         std::vector<int> order(L.pieces.size());
         for (size_t i = 0; i < order.size(); ++i)
@@ -186,10 +176,6 @@ void emit_level(std::vector<Task> &tasks, RawTables &raw)
         if (L.nst < best.nst || (L.nst == best.nst && L.npart < best.npart))
             best = std::move(L);
     }
-    for (const auto &c : best.comb)
-        raw.comb.push_back(c);
-    raw.max_partials = std::max(raw.max_partials, best.npart);
-    raw.level_comb.push_back((int)raw.comb.size());
     const size_t nst = best.nst;
     const size_t base = raw.steps.size() / kWave;
     raw.steps.resize((base + nst) * kWave, Ent{-1, -1, 0, -1, 1});  // padding
@@ -200,16 +186,13 @@ void emit_level(std::vector<Task> &tasks, RawTables &raw)
 }
 
 // Encodes raw entries into int2 work-space steps: x = l | r << 16,
-// y = w | first << 16 | last << 17 | c << 18.  map_l / map_r / map_w
-// translate raw operands and targets to work-space indices; partial p goes
-// to part0 + p and padding reads `dummy` and writes nothing.  kRulePad
-// padding steps follow the last level.
+// y = w | c << 17 | last << 31.  map_l / map_r / map_w translate raw operands
+// and targets to work-space indices; padding reads `dummy` and writes
+// nothing.  kRulePad padding steps follow the last level.
 template <class ML, class MR, class MW>
-void encode_tables(const RawTables &raw, int part0, int dummy, ML map_l, MR map_r, MW map_w,
-                   std::vector<int> &steps, std::vector<int> &level_step, std::vector<int> &comb,
-                   std::vector<int> &level_comb)
+void encode_tables(const RawTables &raw, int dummy, ML map_l, MR map_r, MW map_w,
+                   std::vector<int> &steps, std::vector<int> &level_step)
 {
-    auto target = [&](int w) { return w <= -2 ? part0 + (-w - 2) : map_w(w); };
     const size_t nraw = raw.steps.size();
     steps.assign((nraw + (size_t)kRulePad * kWave) * 2, 0);
     const size_t nst = nraw / kWave;
@@ -221,7 +204,7 @@ void encode_tables(const RawTables &raw, int part0, int dummy, ML map_l, MR map_
         } else {
             l = map_l(e[0]);
             r = map_r(e[1]);
-            w = target(e[3]);
+            w = map_w(e[3]);
             // last entry of its task or piece: the lane's next step starts
             // another one, is padding, or the level ends
             const size_t st = i / kWave, q = i % kWave;
@@ -236,13 +219,10 @@ void encode_tables(const RawTables &raw, int part0, int dummy, ML map_l, MR map_
             }
         }
         steps[2 * i] = l | (r << 16);
-        steps[2 * i + 1] = w | (e[4] << 16) | (last << 17) | (int)((unsigned)e[2] << 18);
+        steps[2 * i + 1] =
+            (int)((unsigned)w | ((unsigned)e[2] & 0x3fffu) << 17 | (unsigned)last << 31);
     }
     level_step = raw.level_step;
-    level_comb = raw.level_comb;
-    comb.clear();
-    for (auto &c : raw.comb)
-        comb.insert(comb.end(), {target(c[0]), part0 + c[1], c[2], 0});
 }
 
 }  // namespace
@@ -923,17 +903,6 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
         if (p.force_basic.size() & 1)
             p.force_basic.push_back(-1);
     }
-    for (int k = 0; k < (kMaxNu + 1) * kMaxMu; ++k)
-        p.slot_base[k] = -1;
-    {
-        int s = 0;
-        for (int nu = 0; nu <= p.numax_all; ++nu)
-            for (int mu = 0; mu < m.M; ++mu)
-                if (p.numax[mu] >= nu) {
-                    p.slot_base[nu * kMaxMu + mu] = s;
-                    s += (nu + 1) * (nu + 2) / 2;
-                }
-    }
 
     // Dependency levels.  The reference applies the rules in file order
     // (potential_mtp.cpp:2918-2924), so every operand must be complete before
@@ -954,11 +923,11 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     p.max_level = maxl;
 
     // Private LDS layout of one wave (in doubles): moments, adjoints, a zero
-    // slot that padding steps read and write, then the partial sums.
+    // slot that padding steps read.
     const int K4 = (m.K + 3) & ~3;
     p.K4 = K4;
     p.dummy = 2 * K4;
-    p.part0 = 2 * K4 + 4;
+    p.red0 = 2 * K4 + 4;
 
     RawTables fwd, bwd;
     forward_tables(m, level, maxl, fwd);
@@ -986,33 +955,24 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     }
 
     // Encode against the private layout (indices in doubles).
-    p.max_partials = std::max(fwd.max_partials, bwd.max_partials);
-    const int P4 = (p.max_partials + 3) & ~3;
-    p.red0 = p.part0 + P4;
     // The moment reduction's transpose buffer lies over the adjoint block
-    // (unused until the seeds are written; the zero slot and the partial sums
-    // under it are cleared again after the neighbour pass) and the force
-    // pass's adjoints over the moments (not read after the
-    // reverse rules), where they fit; then the wave's energy/virial sums.
+    // (unused until the seeds are written; the zero slot under it is cleared
+    // again after the neighbour pass), the force pass's adjoints over the
+    // moments (not read after the reverse rules) where they fit, else after
+    // the zero slot; then the wave's energy/virial sums.
     const int RB = kChunk * kRedStride;
     const int F4 = ((int)p.force_basic.size() + 3) & ~3;
-    int end;
-    if (F4 <= p.K4) {
-        p.efs_red = p.K4;
-        p.efs_stage = 0;
-        end = std::max(p.red0, p.K4 + RB);
-    } else {
-        p.efs_red = p.efs_stage = p.red0;
-        end = p.red0 + std::max(RB, F4);
-    }
+    p.efs_red = K4;
+    p.efs_stage = F4 <= K4 ? 0 : p.red0;
+    int end = std::max(K4 + RB, p.red0 + (F4 <= K4 ? 0 : F4));
     p.efs_acc = (end + 3) & ~3;
     p.priv_doubles = p.efs_acc + 12;  // energy, virial[9], padding
     if (!m.linear()) {
         // The head's work space lives from the end of the forward rules to
         // the seeds.  Over that span the moment transpose buffer past the
-        // partial sums (and the slot-ordered adjoints, written only after
-        // the seeds) are dead: the head goes there where it fits, so the
-        // launch keeps its waves and its LDS step tables.
+        // zero slot (and the force pass's adjoints, written only after the
+        // seeds) are dead: the head goes there where it fits, so the launch
+        // keeps its waves and its LDS step tables.
         const long long hd = 2LL * m.head.P + 2LL * m.head.h1 + m.head.h2;
         if (hd > 0xffff)
             return fail(err, "MTP-M head too large: its work space exceeds 65535 doubles");
@@ -1030,36 +990,23 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
             return fail(err, "product-rule multiplicity outside [-8192, 8191]");
     auto same = [](int x) { return x; };
     auto adj = [&p](int x) { return p.K4 + x; };
-    encode_tables(fwd, p.part0, p.dummy, same, same, same, p.fwd_steps, p.fwd_level_step,
-                  p.fwd_comb, p.fwd_level_comb);
-    encode_tables(bwd, p.part0, p.dummy, adj, same, adj, p.bwd_steps, p.bwd_level_step,
-                  p.bwd_comb, p.bwd_level_comb);
+    encode_tables(fwd, p.dummy, same, same, same, p.fwd_steps, p.fwd_level_step);
+    encode_tables(bwd, p.dummy, adj, same, adj, p.bwd_steps, p.bwd_level_step);
 
     // Training work space: the E/F/S work space without its transpose
     // buffer with its dual copy (tangents and second adjoints) interleaved,
     // element x's value and dual in doubles 2x and 2x + 1, then the wave's
     // radial gradient accumulator and the species of the neighbours in
-    // flight.  Three more buffers lie over blocks that are dead in the phase
-    // that uses them, where they fit: the first neighbour pass's transpose
-    // buffer over the adjoint pairs (written with the seeds later), the
-    // slot-ordered {A, G} stage over the moment pairs (dead after the reverse
-    // rules) and the last pass's transpose buffer over the adjoint pairs
-    // (dead after the staging).  Otherwise they get room of their own after
-    // the gradient accumulator.
-    p.tr_grad = 2 * p.red0;
+    // flight.  Two more buffers lie over blocks that are dead in the phase
+    // that uses them: the neighbour passes' transpose buffer over the adjoint
+    // pairs (the first pass ends before the seeds are written, the last one
+    // begins after the adjoints are staged), with room behind them where they
+    // are shorter, and the {A, G} stage over the moment pairs (dead after the
+    // reverse rules) where it fits, else after the species.
+    p.tr_red = 2 * K4;
+    p.tr_grad = std::max(2 * p.red0, p.tr_red + RB);
     p.tr_ctype = p.tr_grad + ((m.nradial() + 3) & ~3);
     end = p.tr_ctype + kWave / 2;  // 64 ints: neighbour species of a batch
-    int own_red = -1;
-    auto red_region = [&] {
-        if (own_red < 0) {
-            own_red = end;
-            end += RB;
-        }
-        return own_red;
-    };
-    const bool over_adjoints = 2 * (p.red0 - K4) >= RB;
-    p.tr_red1 = over_adjoints ? 2 * K4 : red_region();
-    p.tr_red4 = over_adjoints ? 2 * K4 : red_region();
     if (F4 <= K4) {
         p.tr_stage = 0;
     } else {
@@ -1068,34 +1015,6 @@ bool build_plan(const Model &m, Plan &p, std::string &err)
     }
     p.tr_priv = end;
     return true;
-}
-
-std::vector<int> device_steps(const std::vector<int> &steps, const std::vector<int> &level_step,
-                              const std::vector<int> &comb, const std::vector<int> &level_comb)
-{
-    std::vector<int> out(steps);
-    size_t i = 0;
-    for (size_t L = 0; L < level_step.size(); ++L) {
-        // the targets of the level's partial sums (numbered anew per level);
-        // the padding after the last level has none
-        std::map<int, int> target;
-        const bool level = L + 1 < level_step.size();
-        if (level)
-            for (int c = 4 * level_comb[L]; c < 4 * level_comb[L + 1]; c += 4)
-                for (int k = 0; k < comb[c + 2]; ++k)
-                    target[comb[c + 1] + k] = comb[c];
-        const size_t end = level ? (size_t)level_step[L + 1] * kWave : steps.size() / 2;
-        for (; i < end; ++i) {
-            const int y = steps[2 * i + 1], last = (y >> 17) & 1, c = y >> 18;
-            int w = y & 0xffff;
-            const auto t = target.find(w);
-            if (last && t != target.end())
-                w = t->second;
-            out[2 * i + 1] =
-                (int)((unsigned)w | ((unsigned)c & 0x3fffu) << 17 | (unsigned)last << 31);
-        }
-    }
-    return out;
 }
 
 void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
@@ -1114,11 +1033,15 @@ void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned sh
         const int n = a + b + c;
         if (mu >= m.M || n > p.numax[mu])
             return 0xffff;
-        // position in the slot order: a = n..0, b = n-a..0
+        // position in the slot order: the shells below, then a = n..0, b = n-a..0
         int pos = 0;
+        for (int nu = 0; nu <= n; ++nu)
+            for (int q = 0; q < (nu < n ? m.M : mu); ++q)
+                if (p.numax[q] >= nu)
+                    pos += (nu + 1) * (nu + 2) / 2;
         for (int ap = n; ap > a; --ap)
             pos += n - ap + 1;
-        const int i = p.slot_basic[p.slot_base[n * kMaxMu + mu] + pos + (n - a - b)];
+        const int i = p.slot_basic[pos + (n - a - b)];
         return i < 0 ? 0xffff : (unsigned)i;
     };
     for (size_t ch = 0; ch * kChunk < mono.size(); ++ch)
@@ -1329,15 +1252,14 @@ bool build_lin_plan(const Model &m, const Plan &p, LinPlan &lp, std::string &err
         if (need[r[3]])
             need[r[0]] = need[r[1]] = 1;
     }
-    // Work-space layout (doubles): moments, a zero slot, the forward
-    // partials, then the transpose buffer of the moment reduction, with
-    // {one, L, L partials} over it (they are set after the moments).  The
-    // forward rules are encoded again for this layout (no adjoint block).
+    // Work-space layout (doubles): moments, a zero slot, then the transpose
+    // buffer of the moment reduction, with {one, L} over it (they are set
+    // after the moments).  The forward rules are encoded again for this
+    // layout (no adjoint block).
     RawTables fwd;
     forward_tables(m, level, p.max_level, fwd);
     lp.dummy = p.K4;
-    lp.fpart0 = lp.dummy + 4;
-    lp.red0 = lp.fpart0 + ((fwd.max_partials + 3) & ~3);
+    lp.red0 = lp.dummy + 4;
     lp.one = lp.red0;
     lp.L0 = lp.one + 4;
     std::vector<int> lbase((size_t)K, -1);
@@ -1384,18 +1306,13 @@ bool build_lin_plan(const Model &m, const Plan &p, LinPlan &lp, std::string &err
         }
         emit_level(tasks, raw);
     }
-    lp.part0 = lp.L0 + ((nL + 3) & ~3);
-    const int P4 = (raw.max_partials + 3) & ~3;
-    lp.acc = lp.part0 + P4;
     lp.CH = kLinChunk;
-    lp.priv = std::max(lp.acc, lp.red0 + kChunk * kRedStride);
+    lp.priv = std::max(lp.L0 + ((nL + 3) & ~3), lp.red0 + kChunk * kRedStride);
     if (lp.priv > 0xffff)
         return fail(err, "model too large for the linear-fit work space");
     auto same = [](int x) { return x; };
-    encode_tables(fwd, lp.fpart0, lp.dummy, same, same, same, lp.fwd_steps, lp.fwd_level_step,
-                  lp.fwd_comb, lp.fwd_level_comb);
-    encode_tables(raw, lp.part0, lp.dummy, same, same, same, lp.steps, lp.level_step, lp.comb,
-                  lp.level_comb);
+    encode_tables(fwd, lp.dummy, same, same, same, lp.fwd_steps, lp.fwd_level_step);
+    encode_tables(raw, lp.dummy, same, same, same, lp.steps, lp.level_step);
     // Chunks of scalars (group_scalars): at most kLinChunk scalars and at
     // most kLinEntries (slot, scalar) entries each.  Per chunk and slot: a
     // mask of the chunk's scalars whose support holds the slot's basic, and

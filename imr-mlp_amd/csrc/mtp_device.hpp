@@ -80,24 +80,6 @@ __device__ __forceinline__ double xor16_sum(double v)
     return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
 }
 
-// Sum of one row of a reduction chunk (kChunk = 16 rows of 64 columns,
-// stride kRedStride): lane l sums row l & 15 over columns 16 (l >> 4) .. +15
-// with 16-byte reads, then the four column groups are combined (lanes l ^ 32,
-// l ^ 16); every lane of the row's group ends with the row total.
-__device__ __forceinline__ double chunk_row_sum(const double *red, int lane)
-{
-    const double2 *row =
-        reinterpret_cast<const double2 *>(red + (lane & (kChunk - 1)) * kRedStride + (lane >> 4) * 16);
-    double a0 = 0.0, a1 = 0.0;
-#pragma unroll
-    for (int jj = 0; jj < 8; ++jj) {
-        const double2 v = row[jj];
-        a0 += v.x;
-        a1 += v.y;
-    }
-    return xor16_sum(xor32_sum(a0 + a1));
-}
-
 // v plus the value of the lane that the DPP control kCtrl selects within the
 // lane's row of 16 (VALU lane move, no LDS crossbar).
 template <int kCtrl>
@@ -701,14 +683,39 @@ __device__ __forceinline__ void lds_write(double *p, double v)
     *(volatile __attribute__((address_space(3))) double *)p = v;
 }
 
+// The moment tables (DevModel::mono_tab): in LDS after the other shared
+// tables, or in global memory for a model whose work space leaves no room for
+// them (m.mono_lds; with them there the E/F/S kernel of a level-20 model is
+// 1 to 2 % slower, on a general basis up to 9 %).  kLds: in LDS in any case;
+// without it the choice is made at run time, which costs the E/F/S kernel up
+// to 1.5 % and the gradient and linear-fit kernels nothing.
+template <bool kLds>
+struct MonoTab {
+    const unsigned short *lds, *global;
+    bool in_lds;
+    __device__ __forceinline__ MonoTab(const DevModel &m, const unsigned short *l)
+        : lds(l), global(m.mono_tab), in_lds(kLds || m.mono_lds)
+    {
+    }
+    __device__ __forceinline__ unsigned operator[](int k) const
+    {
+        if (in_lds)  // uniform; volatile keeps it apart from the global load
+            return *(const volatile __attribute__((address_space(3))) unsigned short *)(lds + k);
+        const unsigned v = global[k];
+        // waited for here: past the branch a wait would be for both counters
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        return v;
+    }
+};
+
 // The chunk of kChunk monomials in the transpose buffer, against the radial
 // functions of group G (rows 4 G .. 4 G + 3): the sums go to the moments of
 // the chunk's table entries (0xffff: no such moment).  Columns past the
 // batch's neighbours hold zero radial functions, so whole groups of sixteen
 // neighbours past the end are left out.
-template <int G>
+template <int G, class Tab>
 __device__ __forceinline__ void moment_chunk(const double *red, const double (&af)[G][kWave / 4],
-                                             unsigned groups, const unsigned short *tab, int cnt,
+                                             unsigned groups, const Tab &tab, int at, int cnt,
                                              double *mom, int lane)
 {
     wave_sync();
@@ -738,21 +745,21 @@ __device__ __forceinline__ void moment_chunk(const double *red, const double (&a
 #pragma unroll
     for (int g = 0; g < G; ++g)
         if (groups >> g & 1) {
-            const int t = tab[lane];
-            tab += kWave;
-            if (t != 0xffff)
+            const unsigned t = tab[at + lane];
+            at += kWave;
+            if (t != 0xffffu)
                 mom[t] += s0[g] + s1[g];
         }
     wave_sync();
 }
 
 // Adds one batch of neighbours (cnt <= 64, lane j holds neighbour j) to the
-// basic moments.  red: 16 rows of kRedStride doubles; tab: m.mono_tab.
-template <class P>
-__device__ __forceinline__ void add_moments(const DevModel &m, double *red,
-                                            const unsigned short *tab, double *mom,
-                                            const Nbr<P::M> &q, int cnt, int lane)
+// basic moments.  red: 16 rows of kRedStride doubles; tab: a MonoTab.
+template <class P, class Tab>
+__device__ __forceinline__ void add_moments(const DevModel &m, double *red, const Tab &tab,
+                                            double *mom, const Nbr<P::M> &q, int cnt, int lane)
 {
+    int at = 0;
     constexpr int G = (P::M + 3) / 4;
     // the radial functions through the transpose buffer into the A operands
 #pragma unroll
@@ -775,8 +782,8 @@ __device__ __forceinline__ void add_moments(const DevModel &m, double *red,
         lds_write(red + (e % kChunk) * kRedStride + lane, v);
         if constexpr (e % kChunk == kChunk - 1 || e == mono_count(P::NUMAX) - 1) {
             const unsigned groups = mono_groups<P>(m, ch);
-            moment_chunk<G>(red, af, groups, tab, cnt, mom, lane);
-            tab += kWave * __builtin_popcount(groups);
+            moment_chunk<G>(red, af, groups, tab, at, cnt, mom, lane);
+            at += kWave * __builtin_popcount(groups);
         }
     });
 }
@@ -1122,20 +1129,27 @@ __device__ __forceinline__ void run_rules(const Steps tab, const int *level_step
 }
 
 // The block-shared model tables in LDS, laid out as the device's packed copy
-// m.shared (SharedOffsets), the adjoint seeds and the step tables left out
-// where a kernel does not take them.
+// m.shared (SharedOffsets), the adjoint seeds left out where a kernel does
+// not take them, the step tables (and without m.mono_lds the moment tables)
+// where they stay in global memory.
 struct Shared {
     double *coef, *seed, *moment;
-    int *map, *slot_basic, *force_basic;
+    int *map, *force_basic;
     unsigned short *mono;
     int2 *fwd_steps, *bwd_steps;
 };
+
+__device__ __host__ __forceinline__ size_t shared_end(const DevModel &m, const SharedOffsets &o,
+                                                      bool tables)
+{
+    return tables ? o.end : m.mono_lds ? o.fwd : o.mono;
+}
 
 __device__ __host__ __forceinline__ size_t shared_doubles(const DevModel &m, bool tables,
                                                           bool seeds = true)
 {
     const SharedOffsets o(m);
-    return ((tables ? o.end : o.fwd) - (seeds ? 0 : o.moment - o.seed) + 3) & ~size_t(3);
+    return (shared_end(m, o, tables) - (seeds ? 0 : o.moment - o.seed) + 3) & ~size_t(3);
 }
 
 __device__ __forceinline__ Shared shared_layout(const DevModel &m, double *base,
@@ -1148,7 +1162,6 @@ __device__ __forceinline__ Shared shared_layout(const DevModel &m, double *base,
     L.seed = seeds ? base + o.seed : nullptr;
     L.moment = rest + o.moment;
     L.map = reinterpret_cast<int *>(rest + o.map);
-    L.slot_basic = reinterpret_cast<int *>(rest + o.slot);
     L.force_basic = reinterpret_cast<int *>(rest + o.force);
     L.mono = reinterpret_cast<unsigned short *>(rest + o.mono);
     L.fwd_steps = reinterpret_cast<int2 *>(rest + o.fwd);
@@ -1167,7 +1180,7 @@ __device__ __forceinline__ void stage_shared(const DevModel &m, const Shared &L,
     const v2d *src = reinterpret_cast<const v2d *>(m.shared);
     v2d *dst = reinterpret_cast<v2d *>(L.coef);
     const int skip = L.seed ? 0 : (int)(o.moment - o.seed) / 2, cut = (int)o.seed / 2;
-    const int n = (int)(tables ? o.end : o.fwd) / 2 - skip;
+    const int n = (int)shared_end(m, o, tables) / 2 - skip;
     for (int k0 = tid; k0 < n; k0 += 8 * nthreads) {
         v2d v[8];
 #pragma unroll

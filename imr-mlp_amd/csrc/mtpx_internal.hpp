@@ -266,57 +266,42 @@ struct Plan {
     std::vector<int> force_basic;
     std::vector<int> dup;          // [ndup][2] {duplicate basic, source basic}
     // Each wave owns a private LDS work space (indices in doubles):
-    //   [0, K4) moments | [K4, 2 K4) adjoints | dummy (a zero slot) |
-    //   [part0, red0) partial sums | [red0, priv_doubles) transpose buffer.
-    int K4 = 0, dummy = 0, part0 = 0, red0 = 0, priv_doubles = 0;
-    // Training work space (doubles): [0, tr_grad) the E/F/S work space
-    // without its transpose buffer and its dual copy as pairs (element x at
-    // 2x, its dual at 2x + 1), the radial gradient accumulator (tr_grad,
-    // nradial) and 64 neighbour species (tr_ctype, as ints).  The transpose
-    // buffers of the first and the last neighbour pass (tr_red1, tr_red4) and
-    // the slot-ordered {A, G} pairs (tr_stage, nslots4) lie over blocks that
-    // are dead in their phase, or after the species where they do not fit
-    // there.
-    int tr_red1 = 0, tr_red4 = 0, tr_stage = 0, tr_grad = 0, tr_ctype = 0, tr_priv = 0;
-    // E/F/S kernel: transpose buffer, slot-ordered adjoints, the wave's
+    //   [0, K4) moments | [K4, 2 K4) adjoints | dummy (a zero slot) | red0;
+    // the transpose buffer and the staged adjoints lie over dead blocks of it
+    // or behind red0, up to priv_doubles.
+    int K4 = 0, dummy = 0, red0 = 0, priv_doubles = 0;
+    // Training work space (doubles): the moments, adjoints and zero slot and
+    // their dual copy as pairs (element x at 2x, its dual at 2x + 1), under
+    // the neighbour passes' transpose buffer from tr_red on; the radial
+    // gradient accumulator (tr_grad, nradial) and 64 neighbour species
+    // (tr_ctype, as ints).  The {A, G} pairs (tr_stage, nforce) lie over the
+    // moment pairs, or after the species where they do not fit there.
+    int tr_red = 0, tr_stage = 0, tr_grad = 0, tr_ctype = 0, tr_priv = 0;
+    // E/F/S kernel: transpose buffer, the force pass's adjoints, the wave's
     // energy/virial sums and, with an MTP-M head, the head's work space
     // (descriptors, their adjoints, hidden activations and derivatives, the
     // second layer's adjoints: over the dead transpose buffer where it fits)
     // (offsets in doubles).
     int efs_red = 0, efs_stage = 0, efs_acc = 0, efs_head = 0;
-    // first slot of each (nu, mu) block, -1 where absent: [nu * kMaxMu + mu]
-    int slot_base[(kMaxNu + 1) * kMaxMu];
     // Lane-major step tables, one per direction.  Level L owns steps
     // [level_step[L], level_step[L+1]) and kRulePad padding steps follow
     // the last level; step s of lane q is
     // entry s * 64 + q, an int2 of work-space indices:
-    //   x = l | r << 16,  y = w | first << 16 | last << 17 | c << 18  (c signed)
-    //   acc += c * ws[l] * ws[r];  if (last) { ws[w] = init + acc; acc = 0; }
-    // with init = ws[w] for targets that start from a value (adjoints and
-    // their seeds) and 0 otherwise (a task's sum starts from zero; the first
-    // flag marks a task's first entry and is not needed by the kernels).
-    // Forward entries read two moments and write a rule output; reverse
-    // entries read an adjoint and a moment and write an adjoint (whose
-    // initial value is its seed).  A task (all rules of one output, or all
-    // reverse entries of one destination) longer than the level's fair share
-    // (entries / 64) is split into pieces that write zeroed partial sums; the
-    // level's combine list {target, first partial, count, 0} then adds them
-    // in order to the target (the kernels add the pieces to the target as
-    // they end: device_steps).  Padding steps have c = 0 and
-    // read the dummy slot and write nothing.  Tasks and pieces are spread over the
-    // lanes by longest-processing-time assignment.
-    std::vector<int> fwd_level_step, fwd_steps, fwd_level_comb, fwd_comb;
-    std::vector<int> bwd_level_step, bwd_steps, bwd_level_comb, bwd_comb;
-    int max_partials = 0;
+    //   x = l | r << 16,  y = w | c << 17 | last << 31  (c in 14 bits, signed)
+    //   acc += c * ws[l] * ws[r];  if (last) { ws[w] += acc; acc = 0; }
+    // Forward entries read two moments and add to a rule output, which starts
+    // from zero; reverse entries read an adjoint and a moment and add to an
+    // adjoint, which starts from its seed.  A task (all rules of one output,
+    // or all reverse entries of one destination) longer than the level's fair
+    // share (entries / 64) is split into pieces that add to the target one by
+    // one.  Padding steps have c = 0, read the dummy slot and write nothing.
+    // Tasks and pieces are spread over the lanes by longest-processing-time
+    // assignment.
+    std::vector<int> fwd_level_step, fwd_steps;
+    std::vector<int> bwd_level_step, bwd_steps;
     int max_level = 0;
 };
 bool build_plan(const Model &m, Plan &p, std::string &err);
-// A step table as the kernels read it (run_rules): x as in the plan,
-// y = w | c << 17 | last << 31, and an entry that ends a piece of a split
-// task names the task's target (the kernels add the pieces there; the
-// combine list is not needed).
-std::vector<int> device_steps(const std::vector<int> &steps, const std::vector<int> &level_step,
-                              const std::vector<int> &comb, const std::vector<int> &level_comb);
 // The moment tables of a kernel profile whose monomials reach degree nu
 // (numbered by c, b, a, a fastest): see DevModel::mono_tab, mono_shift.
 void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned short> &tab,
@@ -324,8 +309,8 @@ void moment_table(const Model &m, const Plan &p, int nu, std::vector<unsigned sh
 
 // Linear-fit plan (sparse Jacobian of the scalar moments w.r.t. the basic
 // moments, see build_lin_plan).  Work space per wave (doubles): the E/F/S
-// block [0, red0), the transpose buffer, `one` (1.0), the Jacobian values
-// [L0, L0 + nL), the step partials [part0, acc); priv = acc.
+// moments and a zero slot [0, red0), then the moments' transpose buffer with
+// `one` (1.0) and the Jacobian values [L0, L0 + nL) over it, up to priv.
 // Scalars per pass: their derivatives live in registers, and a tile row of
 // 3 kLinChunk + 1 doubles keeps a 256-atom structure's tile (with the
 // radial coefficients) within a quarter of the 160 KB LDS, one wave per SIMD.
@@ -334,12 +319,12 @@ constexpr int kLinAcc = (3 * kLinChunk + 3) & ~3;  // derivative registers, a mu
 constexpr int kLinEntries = 128;   // (slot, scalar) entries per pass: two lane registers
 constexpr int kLinMaskWords = 128; // slot masks of a pass, 4 per word: two lane registers
 struct LinPlan {
-    int dummy = 0, fpart0 = 0, red0 = 0;  // zero slot, forward partials, transpose buffer
-    int nL = 0, one = 0, L0 = 0, part0 = 0, acc = 0, priv = 0;
+    int dummy = 0, red0 = 0;  // zero slot, transpose buffer
+    int nL = 0, one = 0, L0 = 0, priv = 0;
     int CH = kLinChunk, nchunks = 0, max_chunk_entries = 0;
     bool lane_walk = false;  // maskw/clist valid (nslots <= 4 kLinMaskWords)
-    std::vector<int> level_step, steps, level_comb, comb;  // L rules, as Plan's rule tables
-    std::vector<int> fwd_level_step, fwd_steps, fwd_level_comb, fwd_comb;  // forward rules
+    std::vector<int> level_step, steps;          // L rules, as Plan's rule tables
+    std::vector<int> fwd_level_step, fwd_steps;  // forward rules
     std::vector<int> chunk_s0;   // [nchunks+1] first position of each chunk in chunk_scalar
     std::vector<int> chunk_scalar;  // [S] the scalars of chunk after chunk
     std::vector<int> slot_mask;  // [nchunks][nslots] bit k: scalar k of the chunk uses the slot
@@ -383,13 +368,13 @@ struct DevModel {
     const double *moment;   // [S]
     const int *map;         // [S]
     const double *seed;     // [K] sum of moment coefficients mapped to each moment
-    const int *slot_basic;  // [nslots]
     const int *force_basic; // [nforce]
     // moment tables of the kernel's profile (moment_table): per chunk of
     // kChunk monomials and group of four radial functions with a moment in
     // it, the basic of lane l (function 4 g + (l >> 4), monomial l & 15) or
     // 0xffff; two mask bits (groups) per chunk
     int nmono;
+    int mono_lds;  // the tables lie in LDS (MonoTab)
     unsigned mono_groups;
     const unsigned short *mono_tab;  // [nmono]
     // per table entry, for x, y and z: the basic whose monomial has one power
@@ -397,28 +382,27 @@ struct DevModel {
     const unsigned *mono_shift;      // [nmono / 64][3][64]
     const int *dup;         // [ndup][2]
     int K4, dummy, red0, priv_doubles;  // per-wave work space (Plan)
-    int tr_red1, tr_red4, tr_stage, tr_grad, tr_ctype, tr_priv;
+    int tr_red, tr_stage, tr_grad, tr_ctype, tr_priv;
     int efs_red, efs_stage, efs_acc;
     // MTP-M head (kHeadNone: the linear MTP of species, moment and seed),
     // the per-wave head work space (offset in doubles) and the head itself
     int head, efs_head;
     const DevHead *hd;
     int nradial, ncoef;
-    int slot_base[(kMaxNu + 1) * kMaxMu];
     int fwd_nsteps, bwd_nsteps;  // steps per lane, all levels and the padding
     const int *fwd_level_step;  // [nfwd+1]
-    const int2 *fwd_steps;      // device_steps
+    const int2 *fwd_steps;      // (Plan)
     const int *bwd_level_step;  // [nbwd+1]
     const int2 *bwd_steps;
 };
 
 // The block-shared model tables (offsets in doubles, every part a multiple of
 // 16 bytes): radial coefficients | adjoint seeds | moment coefficients | map |
-// slot_basic | force_basic | mono_tab | forward | reverse step tables.  The
-// device keeps them packed in this order (DevModel::shared), so a workgroup
-// copies them into LDS as one block.
+// force_basic | mono_tab | forward | reverse step tables.  The device keeps
+// them packed in this order (DevModel::shared), so a workgroup copies them
+// into LDS as one block, without the last tables where those do not fit.
 struct SharedOffsets {
-    size_t coef, seed, moment, map, slot, force, mono, fwd, bwd, end;
+    size_t coef, seed, moment, map, force, mono, fwd, bwd, end;
     __host__ __device__ explicit SharedOffsets(const DevModel &m)
     {
         auto four = [](int n) { return ((size_t)n + 3) & ~size_t(3); };
@@ -426,8 +410,7 @@ struct SharedOffsets {
         seed = four(m.Z * m.Z * m.M * m.R);
         moment = seed + m.K4;
         map = moment + four(m.S);
-        slot = map + four(m.S) / 2;
-        force = slot + four(m.nslots) / 2;
+        force = map + four(m.S) / 2;
         mono = force + four(m.nforce) / 2;
         fwd = mono + (size_t)m.nmono / 4;
         bwd = fwd + (size_t)m.fwd_nsteps * kWave;
@@ -486,13 +469,13 @@ hipError_t launch_efs(const DevModel &m, const DevNeighbors &nb, const EfsOut &o
 // Linear fit (lin_kernel.hip).
 struct DevLin {
     int dummy, red0, nfwd;
-    int nL, one, L0, part0, acc, priv, CH, nchunks, nlev;
+    int nL, one, L0, priv, CH, nchunks, nlev;
     int lane_walk;
     int compiled_walk;  // the plan equals the compiled level-16 walk (lin_walk_compiled)
     const int *fwd_level_step;  // [nfwd + 1]
-    const int2 *fwd_steps;      // device_steps
+    const int2 *fwd_steps;      // (LinPlan)
     const int *level_step;      // [nlev + 1]
-    const int2 *steps;          // device_steps
+    const int2 *steps;          // (LinPlan)
     const int *chunk_s0;    // [nchunks + 1] into chunk_scalar
     const int *chunk_scalar;  // [S] the scalars of chunk after chunk
     const int *slot_mask;   // [nchunks][nslots]

@@ -213,9 +213,9 @@ __device__ __forceinline__ GradNbr pair_weight(const DevNeighbors &nb, const Tra
 // neighbour.  Sums go to the pairs {m, q} with LDS adds: tab as add_moments,
 // shift (m.mono_shift, from global memory) the basic moment and factor that a
 // gradient sum adds to.
-template <class P>
-__device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red,
-                                                 const unsigned short *tab, unsigned base,
+template <class P, class Tab>
+__device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red, const Tab &tab,
+                                                 unsigned base,
                                                  const Nbr<P::M> &q, const GradNbr &g, int cnt,
                                                  int lane)
 {
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
     double *ws = lds + shared_doubles(m, kTabLds, false) + (size_t)wave * m.tr_priv;
     // {value, dual} pairs: {m, Q} for the moments, {A, G} for the adjoints
     double2 *wp = reinterpret_cast<double2 *>(ws);
-    double *red1 = ws + m.tr_red1, *red4 = ws + m.tr_red4;
+    double *red = ws + m.tr_red;
     double2 *AG = reinterpret_cast<double2 *>(ws + m.tr_stage);
     double *grad = ws + m.tr_grad;  // radial part of the gradient
     const int rowid = blockIdx.x * nwaves + wave;
@@ -540,6 +540,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
     using Steps = std::conditional_t<kTabLds, LdsSteps, GlobalSteps>;
     const Steps fwd_tab(kTabLds ? L.fwd_steps : m.fwd_steps, lane);
     const Steps bwd_tab(kTabLds ? L.bwd_steps : m.bwd_steps, lane);
+    const MonoTab<kTabLds> mono(m, L.mono);
     const int MR = P::exact ? P::M * P::RMAX : m.M * m.R;
 
     for (int i = rowid; i < nb.n; i += gridDim.x * nwaves) {
@@ -566,13 +567,13 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
             const int64_t p = beg + base + lane;
             load_neighbor<P>(m, nb, L.coef, ti, p, valid, q);
             const GradNbr g = pair_weight<P>(nb, t, fi, S, p, valid, q);
-            add_dual_moments<P>(m, red1, L.mono, lds_address(ws), q, g, n - base, lane);
+            add_dual_moments<P>(m, red, mono, lds_address(ws), q, g, n - base, lane);
         }
         wave_sync();
         if (lane == 0)
             for (int k = 0; k < m.ndup; ++k)
                 wp[m.dup[2 * k]] = wp[m.dup[2 * k + 1]];
-        // the zero slot may lie under a transpose buffer
+        // the zero slot may lie under the transpose buffer
         if (lane == 0)
             wp[m.dummy] = double2{0.0, 0.0};
         wave_sync();
@@ -616,8 +617,7 @@ __global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevN
             const int64_t p = beg + base + lane;
             const double win = load_geometry<P::M, !P::exact>(m, nb, p, valid, q, tj, ti);
             const GradNbr g = pair_weight<P>(nb, t, fi, S, p, valid, q);
-            add_radial_gradient<P>(m, red4, ctype, AG, grad, MR, ti, tj, win, q, g, n - base,
-                                   lane);
+            add_radial_gradient<P>(m, red, ctype, AG, grad, MR, ti, tj, win, q, g, n - base, lane);
         }
         wave_sync();
     }

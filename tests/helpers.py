@@ -2,6 +2,7 @@
 import numpy as np
 
 import oracle as O
+from mtpx import capi
 from mtpx import synth as S
 
 
@@ -33,6 +34,38 @@ def assert_efs_close(got, ref, tol):
     assert rel_err(se, ref["se"]) < tol
     assert rel_err(F, ref["F"]) < tol, rel_err(F, ref["F"])
     assert rel_err(St, ref["S"]) < tol, (St, ref["S"])
+
+
+def loss_case(model_text, structs, seed):
+    """Structures with the oracle's lists and labels (the model's own E/F/S
+    plus noise of the size of early training residuals), every label weighed."""
+    m = O.Model(model_text)
+    rng = S.rng_for(seed)
+    nbs, labels = [], []
+    for s in structs:
+        s.pos = O.wrap(s.cell, s.pbc, s.pos) if np.any(s.pbc) else s.pos
+        nb = O.Neighbors.build(s.cell, s.pbc, s.pos, s.types, m.cutoff)
+        E, F, St, _ = O.efs(m, nb)
+        e, f, st = S.noisy_labels(rng, s.n, E, F, St)
+        nbs.append(nb)
+        labels.append(O.Labels(s.n, energy=e, forces=f, stress=st))
+    return dict(text=model_text, model=m, structs=structs, nbs=nbs, labels=labels)
+
+
+def assert_loss_grad_close(ctx, case, tol):
+    """mtpx_loss_grad of a loss_case against the oracle; the model is loaded."""
+    labels, structs = case["labels"], case["structs"]
+    f_o, g_o = O.loss_grad_batch(case["model"], case["nbs"], labels, O.LossSettings.make(),
+                                 penalty_weight=1e-4, reg_l2=1e-6, threads=8)
+    off = ctx.set_structures(structs, case["model"].cutoff)
+    tf = np.concatenate([lb.forces for lb in labels])
+    active, wE, wF, wS = capi.loss_weights(capi.LossSettings.make(), off,
+                                           np.ones((len(structs), 3), np.int32), tf)
+    ctx.set_labels(active, np.array([lb.energy for lb in labels]), wE, tf, wF,
+                   np.array([lb.stress for lb in labels]), wS)
+    f, g, _ = ctx.loss_grad(penalty_weight=1e-4, reg_l2=1e-6)
+    assert rel_err(f, f_o) < tol
+    assert rel_err(g, g_o) < tol, rel_err(g, g_o)
 
 
 class DeviceArray:

@@ -1,31 +1,35 @@
-// Prints a model's product rules and the library's lane-major rule tables
-// (build_plan in imr-mlp_amd/csrc/model.cpp) as plain text for the host
-// tests in test_capi_host.py:
-//   K B T K4 dummy part0 red0 pad
-//   times: T lines "l r c o"
-//   per direction (fwd, then bwd): "nlev ncomb nsteps", the level_step and
-//   level_comb lines, nsteps * 64 lines "x y", ncomb lines "target first count"
+// Prints a model's product rules and the tables the kernels read (build_plan,
+// build_lin_plan and moment_table in imr-mlp_amd/csrc/model.cpp) as plain
+// text for the host tests in test_capi_host.py:
+//   K B T K4 dummy red0 pad M
+//   basic: B lines "mu a b c";  times: T lines "l r c o"
+//   forward and reverse rules: a step table each ("nlev nsteps", the
+//   level_step line, nsteps * 64 lines "x y")
+//   linear fit: "dummy one L0 nL priv nslots nchunks S", slot_basic, map,
+//   chunk_s0, chunk_scalar, slot_mask, slot_L, then the step tables of the
+//   forward rules and of the Jacobian (nchunks -1: no linear plan)
+//   moment tables: the count, then per degree "nu entries groups", the table
+//   and its shifts
 #include "mtpx_internal.hpp"
 
 #include <cstdio>
 #include <fstream>
 #include <sstream>
 
-static void tables(const std::vector<int> &level_step, const std::vector<int> &level_comb,
-                   const std::vector<int> &steps, const std::vector<int> &comb)
+template <class T>
+static void line(const std::vector<T> &v)
 {
-    const size_t nsteps = steps.size() / (2 * mtpx::kWave);
-    std::printf("%zu %zu %zu\n", level_step.size() - 1, comb.size() / 4, nsteps);
-    for (int v : level_step)
-        std::printf("%d ", v);
+    for (T x : v)
+        std::printf("%lld ", (long long)x);
     std::printf("\n");
-    for (int v : level_comb)
-        std::printf("%d ", v);
-    std::printf("\n");
+}
+
+static void table(const std::vector<int> &level_step, const std::vector<int> &steps)
+{
+    std::printf("%zu %zu\n", level_step.size() - 1, steps.size() / (2 * mtpx::kWave));
+    line(level_step);
     for (size_t i = 0; i < steps.size(); i += 2)
         std::printf("%d %d\n", steps[i], steps[i + 1]);
-    for (size_t i = 0; i < comb.size(); i += 4)
-        std::printf("%d %d %d\n", comb[i], comb[i + 1], comb[i + 2]);
 }
 
 int main(int argc, char **argv)
@@ -44,12 +48,39 @@ int main(int argc, char **argv)
         std::fprintf(stderr, "%s\n", err.c_str());
         return 1;
     }
-    std::printf("%d %d %d %d %d %d %d %d\n", m.K, m.B, m.T, p.K4, p.dummy, p.part0, p.red0,
-                mtpx::kRulePad);
-    for (int t = 0; t < m.T; ++t)
-        std::printf("%d %d %d %d\n", m.times[4 * t], m.times[4 * t + 1], m.times[4 * t + 2],
-                    m.times[4 * t + 3]);
-    tables(p.fwd_level_step, p.fwd_level_comb, p.fwd_steps, p.fwd_comb);
-    tables(p.bwd_level_step, p.bwd_level_comb, p.bwd_steps, p.bwd_comb);
+    std::printf("%d %d %d %d %d %d %d %d\n", m.K, m.B, m.T, p.K4, p.dummy, p.red0,
+                mtpx::kRulePad, m.M);
+    line(m.basic);
+    line(m.times);
+    table(p.fwd_level_step, p.fwd_steps);
+    table(p.bwd_level_step, p.bwd_steps);
+    mtpx::LinPlan lp;
+    const bool lin = mtpx::build_lin_plan(m, p, lp, err);
+    std::printf("%d %d %d %d %d %d %d %d\n", lp.dummy, lp.one, lp.L0, lp.nL, lp.priv, p.nslots,
+                lin ? lp.nchunks : -1, m.S);
+    if (lin) {
+        line(p.slot_basic);
+        line(m.map);
+        line(lp.chunk_s0);
+        line(lp.chunk_scalar);
+        line(lp.slot_mask);
+        line(lp.slot_L);
+        table(lp.fwd_level_step, lp.fwd_steps);
+        table(lp.level_step, lp.steps);
+    }
+    std::vector<int> degrees;
+    for (int nu : {3, 6, 8})
+        if (nu >= p.numax_all)
+            degrees.push_back(nu);
+    std::printf("%zu\n", degrees.size());
+    for (int nu : degrees) {
+        std::vector<unsigned short> tab;
+        std::vector<unsigned> shift;
+        unsigned groups;
+        mtpx::moment_table(m, p, nu, tab, shift, groups);
+        std::printf("%d %zu %u\n", nu, tab.size() / mtpx::kWave, groups);
+        line(tab);
+        line(shift);
+    }
     return 0;
 }

@@ -266,88 +266,195 @@ def rule_dump(tmp_path_factory):
     return root, exe
 
 
-def _replay(ws, tab, init):
-    """The rule tables applied level by level as the kernels apply them: a
-    level's operands are read as they stood when the level began, a task's
-    sum goes to its target on the task's last entry, then the level's
-    combines add the partial sums in order and clear them."""
-    nlev, ls, lc, steps, comb = tab
-    for L in range(nlev):
+NAMES = ["shapeev-02.mtp", "shapeev-10.mtp", "shapeev-16.mtp", "shapeev-20.mtp", "pot4b.mtp",
+         "ps1-7b-517.mtp", "dup-scalar.mtp"]
+
+
+class _Dump:
+    """The dump of one template, read in order."""
+
+    def __init__(self, rule_dump, name):
+        import os
+        import subprocess
+        root, exe = rule_dump
+        out = subprocess.run([exe, os.path.join("tests", "golden", "templates", name)], cwd=root,
+                             check=True, capture_output=True, text=True).stdout
+        self.v = np.array(out.split(), dtype=np.int64)
+        self.pos = 0
+        self.K, self.B, self.T, self.K4, self.dummy, self.red0, self.pad, self.M = self.take(8)
+        self.basic = self.take(4 * self.B).reshape(-1, 4)
+        self.times = self.take(4 * self.T).reshape(-1, 4)
+        self.fwd, self.bwd = self.table(), self.table()
+        (self.lin_dummy, self.one, self.L0, self.nL, self.lin_priv, nslots, nchunks,
+         S) = self.take(8)
+        self.lin = nchunks >= 0
+        if self.lin:
+            self.slot_basic, self.map = self.take(nslots), self.take(S)
+            self.chunk_s0, self.chunk_scalar = self.take(nchunks + 1), self.take(S)
+            self.slot_mask = self.take(nchunks * nslots).reshape(nchunks, nslots)
+            self.slot_L = self.take(nchunks * nslots * 6).reshape(nchunks, nslots, 6)
+            self.lin_fwd, self.lin_tab = self.table(), self.table()
+        self.moments = []
+        for _ in range(self.take(1)[0]):
+            nu, n, groups = self.take(3)
+            self.moments.append((nu, groups, self.take(64 * n).reshape(n, 64),
+                                 self.take(192 * n).reshape(n, 3, 64)))
+        assert self.pos == len(self.v)
+
+    def take(self, n):
+        self.pos += n
+        return self.v[self.pos - n:self.pos]
+
+    def table(self):
+        nlev, nsteps = self.take(2)
+        ls = self.take(nlev + 1)
+        return ls, self.take(128 * nsteps).reshape(nsteps, 64, 2)
+
+
+def _fields(x, y):
+    """l, r, w, c, last of a step entry."""
+    c = (y >> 17) & 0x3FFF
+    return x & 0xFFFF, (x >> 16) & 0xFFFF, y & 0xFFFF, c - (c >> 13 << 14), y < 0
+
+
+def _check_shape(tab, dummy, pad):
+    """A level is as long as its longest lane; the padding after the last
+    level reads the zero slot and writes nothing."""
+    ls, steps = tab
+    assert len(steps) == ls[-1] + pad
+    l, r, _, c, last = _fields(steps[..., 0], steps[..., 1])
+    blank = (l == dummy) & (r == dummy) & (c == 0) & ~last
+    assert blank[ls[-1]:].all()
+    for a, b in zip(ls[:-1], ls[1:]):
+        assert b == a or not blank[b - 1].all()
+
+
+def _replay(ws, tab):
+    """A step table applied level by level as run_rules applies it: a level's
+    operands are read as they stood when the level began, and a lane's sum is
+    added to the target of the entry that ends a task or a piece of one."""
+    ls, steps = tab
+    for a, b in zip(ls[:-1], ls[1:]):
         snap = ws.copy()
-        for q in range(64):
-            acc = 0.0
-            for st in range(ls[L], ls[L + 1]):
-                x, y = steps[st * 64 + q]
-                acc += (y >> 18) * snap[x & 0xFFFF] * snap[x >> 16]
-                if (y >> 17) & 1:
-                    w = y & 0xFFFF
-                    ws[w] = ws[w] + acc if init else acc
-                    acc = 0.0
-        for tgt, first, cnt in comb[lc[L]:lc[L + 1]]:
-            s = ws[tgt]
-            for j in range(cnt):
-                s += ws[first + j]
-                ws[first + j] = 0.0
-            ws[tgt] = s
+        acc = np.zeros(64)
+        for st in range(a, b):
+            l, r, w, c, last = _fields(steps[st, :, 0], steps[st, :, 1])
+            acc += c * snap[l] * snap[r]
+            np.add.at(ws, w[last], acc[last])
+            acc[last] = 0.0
+        assert not acc.any()  # every sum found its target
 
 
-@pytest.mark.parametrize("name", ["shapeev-10.mtp", "shapeev-16.mtp", "shapeev-20.mtp",
-                                  "pot4b.mtp"])
+@pytest.mark.parametrize("name", NAMES)
 def test_rule_tables_apply_the_product_rules(rule_dump, name):
-    """The lane-major rule tables: each level is as long as its longest lane
-    (no step of padding alone), the padding steps after the last level read
-    and write the zero slot only, and the tables replayed on random basic
-    moments and seeds give the moments of the product rules in file order
+    """The step tables the kernels read, replayed on random basic moments and
+    seeds, give the moments of the product rules in file order
     (potential_mtp.cpp:2918-2924) and the adjoints of backpropagate_moments
-    (:3292-3305, reverse file order)."""
-    import os
-    import subprocess
-    root, exe = rule_dump
-    out = subprocess.run([exe, os.path.join("tests", "golden", "templates", name)], cwd=root,
-                         check=True, capture_output=True, text=True).stdout
-    v = [int(t) for t in out.split()]
-    K, B, T, K4, dummy, part0, red0, pad = v[:8]
-    pos = 8
-    times = np.array(v[pos:pos + 4 * T]).reshape(T, 4)
-    pos += 4 * T
-    tabs = []
-    for _ in range(2):
-        nlev, ncomb, nsteps = v[pos:pos + 3]
-        pos += 3
-        ls = v[pos:pos + nlev + 1]
-        pos += nlev + 1
-        lc = v[pos:pos + nlev + 1]
-        pos += nlev + 1
-        steps = [(v[pos + 2 * i], v[pos + 2 * i + 1]) for i in range(nsteps * 64)]
-        pos += 2 * nsteps * 64
-        comb = [tuple(v[pos + 3 * i:pos + 3 * i + 3]) for i in range(ncomb)]
-        pos += 3 * ncomb
-        assert nsteps == ls[-1] + pad
-        pad_entry = (dummy | dummy << 16, dummy | 1 << 16)
-        assert all(s == pad_entry for s in steps[ls[-1] * 64:])
-        for L in range(nlev):
-            if ls[L + 1] > ls[L]:
-                last = steps[(ls[L + 1] - 1) * 64:ls[L + 1] * 64]
-                assert any(s != pad_entry for s in last)
-        tabs.append((nlev, ls, lc, steps, comb))
-    assert pos == len(v)
-
+    (:3292-3305, reverse file order); the zero slot stays zero."""
+    d = _Dump(rule_dump, name)
+    for tab in (d.fwd, d.bwd):
+        _check_shape(tab, d.dummy, d.pad)
     rng = np.random.default_rng(11)
-    ws = np.zeros(red0)
-    ws[:B] = rng.uniform(0.5, 1.5, B)
-    m = ws[:K].copy()
-    for l, r, c, o in times:
+    ws = np.zeros(d.red0)
+    ws[:d.B] = rng.uniform(0.5, 1.5, d.B)
+    m = ws[:d.K].copy()
+    for l, r, c, o in d.times:
         m[o] += c * m[l] * m[r]
-    _replay(ws, tabs[0], init=False)
-    assert np.allclose(ws[:K], m, rtol=1e-12, atol=1e-12 * np.abs(m).max())
-    assert not ws[dummy] and not ws[part0:red0].any()
+    _replay(ws, d.fwd)
+    assert np.allclose(ws[:d.K], m, rtol=1e-12, atol=1e-12 * np.abs(m).max())
+    assert not ws[d.dummy:].any()
 
-    seed = rng.uniform(-1.0, 1.0, K)
-    ws[K4:K4 + K] = seed
+    seed = rng.uniform(-1.0, 1.0, d.K)
+    ws[d.K4:d.K4 + d.K] = seed
     A = seed.copy()
-    for l, r, c, o in times[::-1]:
+    for l, r, c, o in d.times[::-1]:
         A[r] += c * A[o] * m[l]
         A[l] += c * A[o] * m[r]
-    _replay(ws, tabs[1], init=True)
-    assert np.allclose(ws[K4:K4 + K], A, rtol=1e-11, atol=1e-12 * np.abs(A).max())
-    assert not ws[dummy] and not ws[part0:red0].any()
+    _replay(ws, d.bwd)
+    assert np.allclose(ws[d.K4:d.K4 + d.K], A, rtol=1e-11, atol=1e-12 * np.abs(A).max())
+    assert not ws[d.dummy:].any()
+
+
+@pytest.mark.parametrize("name", ["shapeev-10.mtp", "shapeev-16.mtp", "ps1-7b-517.mtp",
+                                  "dup-scalar.mtp"])
+def test_linear_tables_give_the_scalar_jacobian(rule_dump, name):
+    """The linear fit's step tables: the forward rules again, then
+    L[s][b] = dm_s/dm_b at the work-space index that slot_L names for every
+    scalar of a chunk and every slot of its mask, and 0 outside the masks."""
+    d = _Dump(rule_dump, name)
+    assert d.lin
+    for tab in (d.lin_fwd, d.lin_tab):
+        _check_shape(tab, d.lin_dummy, d.pad)
+    canon = np.arange(d.B)
+    for b in range(d.B):
+        canon[b] = next(k for k in range(b + 1) if np.array_equal(d.basic[k], d.basic[b]))
+    rng = np.random.default_rng(12)
+    ws = np.zeros(d.lin_priv)
+    ws[:d.B] = rng.uniform(0.5, 1.5, d.B)[canon]
+    m, J = ws[:d.K].copy(), np.zeros((d.K, d.B))
+    J[np.arange(d.B), canon] = 1.0
+    for l, r, c, o in d.times:
+        m[o] += c * m[l] * m[r]
+        J[o] += c * (m[r] * J[l] + m[l] * J[r])
+    _replay(ws, d.lin_fwd)
+    assert np.allclose(ws[:d.K], m, rtol=1e-12, atol=1e-12 * np.abs(m).max())
+    ws[d.one:d.L0 + d.nL] = 0.0
+    ws[d.one] = 1.0
+    _replay(ws, d.lin_tab)
+    assert not ws[d.lin_dummy] and ws[d.one] == 1.0
+    scale = 1e-12 * np.abs(J).max()
+    for ch in range(len(d.chunk_s0) - 1):
+        for k, s in enumerate(d.chunk_scalar[d.chunk_s0[ch]:d.chunk_s0[ch + 1]]):
+            got = np.zeros(d.B)
+            for sl, b in enumerate(d.slot_basic):
+                if d.slot_mask[ch, sl] >> k & 1:
+                    got[b] = ws[d.slot_L[ch, sl, k]]
+            assert np.allclose(got, J[d.map[s]], rtol=1e-12, atol=scale)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_moment_tables_place_every_moment_and_tangent(rule_dump, name):
+    """moment_table for every profile degree that holds the model: the sums of
+    f Y, h Y and t Y over the table's (function, monomial) entries, with its
+    shifts and factors, are the basic moments f_mu u^a and their tangents
+    h_mu u^a + t_mu . grad u^a, each moment that occurs once or first in the
+    file.  (Values for one neighbour; the sums over neighbours are linear.)"""
+    d = _Dump(rule_dump, name)
+    rng = np.random.default_rng(13)
+    u = rng.uniform(0.4, 0.9, 3)
+    f, h, t = rng.uniform(0.5, 1.5, d.M), rng.uniform(0.5, 1.5, d.M), rng.uniform(0.5, 1.5, (d.M, 3))
+    Y = lambda p: np.prod([u[k] ** p[k] for k in range(3)]) if min(p) >= 0 else 0.0
+    want, wantq, seen = np.zeros(d.B), np.zeros(d.B), set()
+    for b, (mu, *p) in enumerate(d.basic.tolist()):
+        if (mu, *p) in seen:
+            continue
+        seen.add((mu, *p))
+        want[b] = f[mu] * Y(p)
+        wantq[b] = h[mu] * Y(p) + sum(
+            t[mu, k] * p[k] * Y([p[j] - (j == k) for j in range(3)]) for k in range(3))
+    assert d.moments
+    for nu, groups, tab, shift in d.moments:
+        mono = [(a, b, c) for c in range(nu + 1) for b in range(nu - c + 1)
+                for a in range(nu - c - b + 1)]
+        got, gotq, entry = np.zeros(d.B), np.zeros(d.B), 0
+        for ch in range((len(mono) + 15) // 16):
+            for g in range(2):
+                if not groups >> (2 * ch + g) & 1:
+                    continue
+                for lane in range(64):
+                    mu, e = 4 * g + lane // 16, 16 * ch + lane % 16
+                    to = [tab[entry, lane], *(shift[entry, :, lane] & 0xFFFF)]
+                    if mu >= d.M or e >= len(mono):
+                        assert all(w == 0xFFFF for w in to)
+                        continue
+                    y = Y(mono[e])
+                    if to[0] != 0xFFFF:
+                        got[to[0]] += f[mu] * y
+                        gotq[to[0]] += h[mu] * y
+                    for k in range(3):
+                        if to[1 + k] != 0xFFFF:
+                            gotq[to[1 + k]] += (shift[entry, k, lane] >> 16) * t[mu, k] * y
+                entry += 1
+            assert groups >> (2 * ch) & 1  # the compile-time profiles count on group 0
+        assert entry == len(tab)
+        assert np.allclose(got, want, rtol=1e-13) and np.allclose(gotq, wantq, rtol=1e-13)
