@@ -173,6 +173,23 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const double *rows, in
 
 // ---- gradient kernel ---------------------------------------------------
 
+// Neighbours whose five operand tables (add_dual_moments) a wave holds at a
+// time, and the waves per SIMD the gradient kernel is compiled for.  With 64
+// the tables take 160 registers.  At level 10, whose other phases are small
+// and whose work space leaves room for two workgroups on a CU, halves of 32
+// fit two waves on a SIMD: a training batch of 30,000 atoms takes 418 us
+// (64 neighbours and one wave: 479; 64 and two waves: 450, with spills), one
+// of 100,000 1,135 (1,355; 1,260).  Level 16 spills at two waves either way
+// (30,000 atoms 920 us against 815) and is slower in halves at one wave (880).
+template <class P>
+struct GradShape {
+    static constexpr int batch = 64, waves_per_simd = 1;
+};
+template <>
+struct GradShape<ProfLevel10> {
+    static constexpr int batch = 32, waves_per_simd = 2;
+};
+
 struct GradNbr {
     double wx, wy, wz, wu;  // W_ij and W_ij . u
 };
@@ -212,18 +229,20 @@ __device__ __forceinline__ GradNbr pair_weight(const DevNeighbors &nb, const Tra
 // and the factors a, b, c applied once per atom instead of once per
 // neighbour.  Sums go to the pairs {m, q} with LDS adds: tab as add_moments,
 // shift (m.mono_shift, from global memory) the basic moment and factor that a
-// gradient sum adds to.
+// gradient sum adds to.  The neighbours come in parts of GradShape::batch: a
+// part holds its columns of the five tables in registers.
 template <class P, class Tab>
 __device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red, const Tab &tab,
                                                  unsigned base,
                                                  const Nbr<P::M> &q, const GradNbr &g, int cnt,
                                                  int lane)
 {
-    constexpr int G = (P::M + 3) / 4, S = kWave / 4;
+    constexpr int G = (P::M + 3) / 4, NB = GradShape<P>::batch, S = NB / 4;
     const double tx = (g.wx - g.wu * q.ux) * q.invd, ty = (g.wy - g.wu * q.uy) * q.invd,
                  tz = (g.wz - g.wu * q.uz) * q.invd;
-#pragma unroll
-    for (int grp = 0; grp < G; ++grp) {
+    // (part p: the neighbours p NB .. p NB + NB - 1)
+    auto group = [&](int grp, int part) __attribute__((always_inline)) {
+        const int col = part * NB + (lane >> 4);
         // neighbour values of four radial functions: f, h, t_x, t_y, t_z
         constexpr int T = 5;
         double af[T][S];
@@ -231,7 +250,7 @@ __device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red,
             wave_sync();
 #pragma unroll
             for (int t = t0; t < t0 + n; ++t) {
-                const double *a = red + (4 * (t - t0) + (lane & 3)) * kRedStride + (lane >> 4);
+                const double *a = red + (4 * (t - t0) + (lane & 3)) * kRedStride + col;
 #pragma unroll
                 for (int s = 0; s < S; ++s)
                     af[t][s] = lds_read(a + 4 * s);
@@ -263,7 +282,7 @@ __device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red,
 #pragma unroll
             for (int t = 0; t < 3; ++t)
                 sh[t] = m.mono_shift[(3 * entry + t) * kWave + lane];
-            const double *b = red + (lane & (kChunk - 1)) * kRedStride + (lane >> 4);
+            const double *b = red + (lane & (kChunk - 1)) * kRedStride + col;
             double v[S], s0[T], s1[T];
 #pragma unroll
             for (int s = 0; s < S; ++s)
@@ -273,7 +292,7 @@ __device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red,
                 s0[t] = s1[t] = 0.0;
 #pragma unroll
             for (int k = 0; k < S; k += 4)
-                if (4 * k < cnt) {
+                if (4 * k < cnt - part * NB) {
 #pragma unroll
                     for (int s = k; s < k + 4; s += 2)
 #pragma unroll
@@ -309,6 +328,18 @@ __device__ __forceinline__ void add_dual_moments(const DevModel &m, double *red,
                         chunk(mono_entry<P>(m, e / kChunk, grp));
                 }
             });
+    };
+    auto groups = [&](int part) __attribute__((always_inline)) {
+#pragma unroll
+        for (int grp = 0; grp < G; ++grp)
+            group(grp, part);
+    };
+    if constexpr (NB == kWave) {
+        groups(0);
+    } else {
+#pragma unroll 1
+        for (int part = 0; part < kWave / NB && part * NB < cnt; ++part)
+            groups(part);
     }
 }
 
@@ -513,8 +544,8 @@ __device__ __forceinline__ void add_radial_gradient(const DevModel &m, double *r
 }
 
 template <class P, bool kTabLds, int kMaxWaves>
-__global__ __launch_bounds__(kWave *kMaxWaves) void grad_kernel(DevModel m, DevNeighbors nb,
-                                                                TrainArgs t)
+__global__ __launch_bounds__(kWave *kMaxWaves, GradShape<P>::waves_per_simd) void grad_kernel(
+    DevModel m, DevNeighbors nb, TrainArgs t)
 {
     extern __shared__ double lds[];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
