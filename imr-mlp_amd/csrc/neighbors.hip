@@ -672,7 +672,8 @@ struct SegGeom {      // per structure, after the AABB
 
 struct Seg {
     int nconf;
-    const int *atom_off, *pt_off, *cand_off, *box_off;            // [nconf + 1]
+    const int *atom_off, *pt_off, *cand_off, *box_off, *wg_off;   // [nconf + 1]
+    const int *wg_of;                                             // [wg_off[nconf]]
     const long long *flag_off;                                    // [nconf + 1]
     const Cell *cell;                                             // [nconf]
     const int *wrap;                                              // [nconf]
@@ -697,17 +698,19 @@ __device__ __forceinline__ int seg_of(const T *off, int n, T k)
 }
 
 // load_positions (neighborhoods_base.h:113-127) and the AABB; the centres'
-// species are copied on the way.  Workgroup k
-// of structure c (B per structure) wraps the atoms [k m, (k+1) m) of it,
-// m = ceil(n_c / B), into the cell if the structure is fully periodic, and
-// writes their component-wise min and max (+inf / -inf for an empty range);
-// the host takes the min / max of the B partials.  Min and max are exact.
+// species are copied on the way.  The B workgroups of structure c are
+// g.wg_off[c] .. g.wg_off[c + 1] (wg_of names each one's structure); the k-th
+// wraps the atoms [k m, (k+1) m) of it, m = ceil(n_c / B), into the cell if
+// the structure is fully periodic, and writes their component-wise min and
+// max (+inf / -inf for an empty range); the host takes the min / max of the B
+// partials.  Min and max are exact.
 __global__ __launch_bounds__(256) void wrap_minmax_kernel(Seg g, const double *pos,
-                                                          const int *types, int B, double *wr,
+                                                          const int *types, double *wr,
                                                           double *part, int *center_type)
 {
     __shared__ double lo[256][3], hi[256][3];
-    const int c = blockIdx.x / B, k = blockIdx.x % B, t = threadIdx.x;
+    const int c = g.wg_of[blockIdx.x], t = threadIdx.x;
+    const int k = blockIdx.x - g.wg_off[c], B = g.wg_off[c + 1] - g.wg_off[c];
     const int a0 = g.atom_off[c], n = g.atom_off[c + 1] - a0;
     const int m = (n + B - 1) / B;
     const int i0 = min(n, k * m), i1 = min(n, i0 + m);
@@ -1794,7 +1797,20 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     // in pinned memory, which the wrap kernel reads in place (it copies the
     // species to the centre types, which the later kernels read)
     Upload head;
-    const size_t o_atoms = head.add(atom_off), o_wrap = head.add(wrapf), o_cell = head.add(cl);
+    // workgroups of the wrap kernel: about 512 atoms each, at most 64 a
+    // structure (two round trips to the pinned positions a thread; 32,000
+    // atoms: 22 us, 28 with eight round trips); a structure's own size
+    // decides, so that one large structure does not multiply the workgroups
+    // of many small ones (2,000 structures of 24 atoms and one of 32,000:
+    // 3.26 ms a build, 3.72 with 63 workgroups for each)
+    std::vector<int> wg_off(1, 0), wg_of;
+    for (int c = 0; c < nconf; ++c) {
+        const int n = atom_off[c + 1] - atom_off[c];
+        wg_of.insert(wg_of.end(), (size_t)std::min(64, std::max(1, (n + 511) / 512)), c);
+        wg_off.push_back((int)wg_of.size());
+    }
+    const size_t o_atoms = head.add(atom_off), o_wrap = head.add(wrapf), o_cell = head.add(cl),
+                 o_wgoff = head.add(wg_off), o_wgof = head.add(wg_of);
     DTRY(head.send(w.up_head, w.seg_head, s));
     const size_t pos_bytes = sizeof(double) * 3 * (size_t)ntot;
     DTRY(w.up_pos.ensure(pos_bytes + sizeof(int) * (size_t)ntot));
@@ -1813,30 +1829,24 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     g.cell = at<Cell>(w.seg_head, o_cell);
     DTRY(w.wrapped.ensure(sizeof(double) * 3 * (size_t)ntot));
     double *wr = w.wrapped.as<double>();
-    // workgroups per structure: about 512 atoms each, at most 64 (two round
-    // trips to the pinned positions a thread; 32,000 atoms: 22 us, 28 with
-    // eight round trips)
-    int nmax = 0;
-    for (int c = 0; c < nconf; ++c)
-        nmax = std::max(nmax, atom_off[c + 1] - atom_off[c]);
-    const int B = std::min(64, std::max(1, (nmax + 511) / 512));
-    const size_t npart = 6 * (size_t)nconf * B;
+    g.wg_off = at<int>(w.seg_head, o_wgoff);
+    g.wg_of = at<int>(w.seg_head, o_wgof);
+    const size_t npart = 6 * wg_of.size();
     DTRY(w.down.ensure(sizeof(double) * std::max<size_t>(npart, 8)));
     void *hdown = nullptr;  // pinned: the kernel writes the partials there
     DTRY(hipHostGetDevicePointer(&hdown, w.down.p, 0));
-    hipLaunchKernelGGL(wrap_minmax_kernel, dim3((unsigned)((size_t)nconf * B)), dim3(256), 0, s, g,
-                       dpos, dtypes_host, B, wr, static_cast<double *>(hdown),
-                       out.center_type.as<int>());
+    hipLaunchKernelGGL(wrap_minmax_kernel, dim3((unsigned)wg_of.size()), dim3(256), 0, s, g, dpos,
+                       dtypes_host, wr, static_cast<double *>(hdown), out.center_type.as<int>());
     DTRY(hipGetLastError());
     DTRY(hipStreamSynchronize(s));
     const double *part = w.down.as<double>();
     std::vector<double> mm(6 * (size_t)nconf);
     for (int c = 0; c < nconf; ++c)
         for (int d = 0; d < 3; ++d) {
-            double l = part[6 * (size_t)c * B + d], h = part[6 * (size_t)c * B + 3 + d];
-            for (int k = 1; k < B; ++k) {
-                const double pl = part[6 * ((size_t)c * B + k) + d];
-                const double ph = part[6 * ((size_t)c * B + k) + 3 + d];
+            double l = part[6 * (size_t)wg_off[c] + d], h = part[6 * (size_t)wg_off[c] + 3 + d];
+            for (int k = wg_off[c] + 1; k < wg_off[c + 1]; ++k) {
+                const double pl = part[6 * (size_t)k + d];
+                const double ph = part[6 * (size_t)k + 3 + d];
                 l = pl < l ? pl : l;
                 h = ph > h ? ph : h;
             }

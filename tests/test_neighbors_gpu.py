@@ -115,6 +115,35 @@ def test_one_pass_and_counted_builds_agree():
         c.close()
 
 
+def test_batch_of_very_different_sizes(nctx):
+    """Structures of 0 to 2,700 atoms in one batch (the wrap kernel gives each
+    as many workgroups as its own size asks for), atoms outside their cells:
+    every structure's lists are the oracle's bit for bit."""
+    rng = S.rng_for(420)
+    structs = []
+    for reps in [(2, 2, 2), None, (8, 8, 8), (1, 1, 1), (5, 5, 5), (6, 6, 15), None, (2, 3, 2)]:
+        s = S.displace(S.lattice("fcc" if reps else "bcc", reps or (1, 1, 1), 3.6), rng, 0.1)
+        if reps is None:  # no atoms
+            s = S.Structure(s.cell, np.zeros((0, 3)), np.zeros(0, np.int32), s.pbc)
+        s.pos = s.pos + 25.0 * (S.uniform(rng, 3 * s.n, -1.0, 1.0).reshape(-1, 3))
+        s.types = (S.uniform(rng, s.n) * 2).astype(np.int32)
+        structs.append(s)
+    structs[2].pbc = np.array([1, 0, 1], np.int32)
+    off = nctx.set_structures(structs, 5.0)
+    got = nctx.get_neighbors()
+    for s, a, b in zip(structs, off[:-1], off[1:]):
+        e0, e1 = got["offsets"][a], got["offsets"][b]
+        assert b - a == s.n
+        if s.n == 0:
+            assert e0 == e1
+            continue
+        # (both builders wrap the same unwrapped positions once)
+        nb = O.Neighbors.build(s.cell, s.pbc, s.pos, s.types, 5.0)
+        _compare(dict(offsets=got["offsets"][a:b + 1] - e0, idx=got["idx"][e0:e1] - a,
+                      types=got["types"][e0:e1], center_types=got["center_types"][a:b],
+                      vec=got["vec"][e0:e1], dist=got["dist"][e0:e1]), nb)
+
+
 def _rel(a, b):
     a, b = np.asarray(a, float), np.asarray(b, float)
     return np.abs(a - b).max() / max(np.abs(b).max(), 1e-300)
