@@ -1609,12 +1609,13 @@ void rank_lists(NeighborStore &out, NeighborScratch &w, int ntot, const int *cnt
 // One fully periodic structure of n <= kSmallAtoms atoms: four launches and
 // one synchronisation (3,072 atoms: 99 us a build, 119 the general way with its
 // eleven launches and two synchronisations; 1,000 atoms 66 us, of which 27 in
-// the preparation, bound by latency and the one CU).  *built stays false when the
-// structure does not fit the limits or a list its bin; it is then built the
-// general way, which also reports every error.
+// the preparation, bound by latency and the one CU).  A structure that does
+// not fit the limits (kNotTaken) or one of whose lists outgrows its bin
+// (kBinFull) is then built the general way, which also reports every error.
+enum class SmallResult { kNotTaken, kBinFull, kBuilt };
 int build_small(const double cell[9], const int pbc[3], int n, const double *pos,
                 const int *types, double cutoff, hipStream_t s, NeighborStore &out,
-                NeighborScratch &w, bool *built, std::string &err)
+                NeighborScratch &w, SmallResult *result, std::string &err)
 {
     SmallBuild a{};
     std::copy(cell, cell + 9, a.cell.m);
@@ -1729,11 +1730,13 @@ int build_small(const double cell[9], const int pbc[3], int n, const double *pos
     DTRY(hipGetLastError());
     DTRY(hipStreamSynchronize(s));
     const int *down = w.down.as<int>();
-    if (down[0] != 0)
+    if (down[0] != 0) {
+        *result = down[0] == 1 ? SmallResult::kBinFull : SmallResult::kNotTaken;
         return MTPX_OK;
+    }
     out.P = down[1];
     out.has_mirror = true;
-    *built = true;
+    *result = SmallResult::kBuilt;
     return MTPX_OK;
 }
 
@@ -1770,11 +1773,11 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     pbc += 3 * (size_t)c0;
     pos += 3 * (size_t)base;
     types += base;
+    SmallResult small = SmallResult::kNotTaken;
     if (nconf == 1 && ntot <= kSmallAtoms && pbc[0] && pbc[1] && pbc[2]) {
-        bool built = false;
-        if (int rc = build_small(cells, pbc, ntot, pos, types, cutoff, s, out, w, &built, err))
+        if (int rc = build_small(cells, pbc, ntot, pos, types, cutoff, s, out, w, &small, err))
             return rc;
-        if (built)
+        if (small == SmallResult::kBuilt)
             return MTPX_OK;
     }
     // host tables: offsets, cells
@@ -2025,8 +2028,9 @@ int build_chunk(int c0, int c1, const int *atom_offsets, const double *cells, co
     int *down = w.down.as<int>();
     // One pass into bins sized from the previous counted build: the entry
     // total comes back with the final synchronisation.  A list that outgrows
-    // its bin sends the chunk through the counted build below.
-    const long long cap = w.bin_cap;
+    // its bin sends the chunk through the counted build below, as one already
+    // did that outgrew the same bin of a small build.
+    const long long cap = small == SmallResult::kBinFull ? 0 : w.bin_cap;
     if (cap > 0 && (long long)ntot * cap <= kBinEntries) {
         cb.cap = (int)cap;
         DTRY(ensure_entries(out, w, (size_t)ntot * cap));

@@ -7,6 +7,7 @@ cutoff and, where a limit is passed, such that the general way takes over."""
 import numpy as np
 import pytest
 
+from mtpx import capi
 from mtpx import synth as S
 
 pytestmark = pytest.mark.gpu
@@ -63,18 +64,62 @@ def test_small_build_equals_the_batch_build(ctx, n, shape):
         assert np.array_equal(F, wantF)
 
 
-def test_bins_that_overflow_fall_back(ctx):
-    """A cluster in a large cell: its lists outgrow bins sized by the mean
-    density, and the next, sparser build uses the larger bins."""
+def _check(ctx, st, cutoff=CUTOFF):
+    """The lists of st alone on ctx against those of a batch in a context of
+    its own, which neither sizes nor fills ctx's bins."""
+    c = capi.Context(0)
+    try:
+        c.set_structures([st, _structure(7, "cubic", 3)], cutoff)
+        want = _lists(c)
+    finally:
+        c.close()
+    ctx.build_neighbors(st.cell, st.pbc, st.pos, st.types, cutoff)
+    got = _lists(ctx)
+    P = want["offsets"][st.n]
+    assert np.array_equal(got["offsets"], want["offsets"][:st.n + 1])
+    for k in ("idx", "types", "vec", "dist"):
+        assert np.array_equal(got[k], want[k][:P]), k
+    return int(np.diff(got["offsets"]).max())
+
+
+def _mean_list(st):
+    return st.n / abs(np.linalg.det(st.cell)) * 4 / 3 * np.pi * CUTOFF ** 3
+
+
+def test_bins_that_overflow_fall_back():
+    """A cluster in a large cell.  On a fresh context its lists outgrow the
+    bins sized by the mean density (one and a half times the mean list and 32)
+    and it is counted; the next builds use bins of the longest list and a
+    quarter, which a denser cluster outgrows again."""
     rng = S.rng_for(922)
-    pos = 4.0 * rng.random((300, 3)) + 8.0
-    dense = S.Structure(np.eye(3) * 20.0, pos, np.zeros(300, np.int32), np.ones(3, np.int32))
-    for st in (dense, _structure(500, "cubic", 5), dense):
-        ctx.set_structures([st, _structure(7, "cubic", 3)], CUTOFF)
-        want = _lists(ctx)
-        P = want["offsets"][len(st.types)]
-        ctx.build_neighbors(st.cell, st.pbc, st.pos, st.types, CUTOFF)
-        got = _lists(ctx)
-        assert len(got["idx"]) == P
-        for k in ("idx", "types", "vec", "dist"):
-            assert np.array_equal(got[k], want[k][:P]), k
+    cluster = lambda n: S.Structure(np.eye(3) * 20.0, 4.0 * rng.random((n, 3)) + 8.0,
+                                    np.zeros(n, np.int32), np.ones(3, np.int32))
+    dense, denser, sparse = cluster(300), cluster(500), _structure(500, "cubic", 5)
+    c = capi.Context(0)
+    try:
+        longest = _check(c, dense)
+        assert longest > 1.5 * _mean_list(dense) + 32
+        _check(c, sparse)
+        assert _check(c, denser) > longest + longest // 4 + 8
+        for st in (dense, denser, sparse):
+            _check(c, st)
+    finally:
+        c.close()
+
+
+def test_more_points_than_the_preparation_holds():
+    """Atoms crowded around the corner of the cell: each has seven images
+    within the cutoff of the bounding box, 20,800 points where the mean density
+    promises 5,000, so the one-workgroup preparation gives the build up."""
+    rng = S.rng_for(923)
+    n, a, rc = 2600, 16.0, 2.0
+    st = S.Structure(np.eye(3) * a, rng.uniform(-0.95 * rc, 0.95 * rc, (n, 3)),
+                     (S.uniform(rng, n) * 2).astype(np.int32), np.ones(3, np.int32))
+    assert n * (1 + 2 * rc / a) ** 3 < 18432 < 8 * n
+    c = capi.Context(0)
+    try:
+        for _ in range(2):
+            _check(c, st, rc)
+        _check(c, _structure(997, "cubic", 6))
+    finally:
+        c.close()
