@@ -91,28 +91,44 @@ def test_full_size_workload2_lists_bit_exact(nctx):
     assert 40 <= counts.mean() <= 55
 
 
-def test_one_pass_and_counted_builds_agree():
+def _build_sequence(s, cutoffs):
+    """Builds s at each cutoff in turn on a fresh context; every result is the
+    oracle's lists bit for bit."""
+    from mtpx import capi
+    pos = O.wrap(s.cell, s.pbc, s.pos)
+    ref = {rc: O.Neighbors.build(s.cell, s.pbc, pos, s.types, rc) for rc in set(cutoffs)}
+    longest = int(np.diff(ref[5.0].offsets).max())
+    assert int(np.diff(ref[7.0].offsets).max()) > longest + longest // 4 + 8
+    c = capi.Context(0)
+    try:
+        for rc in cutoffs:
+            c.build_neighbors(s.cell, s.pbc, pos, s.types, rc)
+            _compare(c.get_neighbors(), ref[rc])
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("pbc", [(1, 1, 1), (1, 1, 0)])
+def test_one_pass_and_counted_builds_agree(pbc):
     """The builder counts the lists on a context's first build and, on the
     next builds, writes them in one pass into bins sized from the longest
     list seen (plus a quarter and 8); a list that outgrows its bin sends the
     build back through the counting pass.  A fresh context walks every path:
     counted (first build), one pass (same cell), overflow then counted (a
     cutoff of 7 gives lists about 2.7 times longer), one pass at the longer
-    cutoff, one pass back at the shorter one.  Every result is the oracle's
-    lists bit for bit."""
-    from mtpx import capi
-    _, s = S.workload_inference(1)
-    pos = O.wrap(s.cell, s.pbc, s.pos)
-    ref = {rc: O.Neighbors.build(s.cell, s.pbc, pos, s.types, rc) for rc in (5.0, 7.0)}
-    longest = int(np.diff(ref[5.0].offsets).max())
-    assert int(np.diff(ref[7.0].offsets).max()) > longest + longest // 4 + 8
-    c = capi.Context(0)
-    try:
-        for rc in (5.0, 5.0, 7.0, 7.0, 5.0):
-            c.build_neighbors(s.cell, s.pbc, pos, s.types, rc)
-            _compare(c.get_neighbors(), ref[rc])
-    finally:
-        c.close()
+    cutoff, one pass back at the shorter one.  3,456 atoms: more than the
+    one-workgroup preparation of small periodic structures takes."""
+    rng = S.rng_for(421)
+    s = S.displace(S.lattice("fcc", (6, 12, 12), 3.56), rng, 0.1)
+    s.pbc = np.array(pbc, np.int32)
+    assert s.n == 3456
+    _build_sequence(s, (5.0, 5.0, 7.0, 7.0, 5.0))
+
+
+def test_builds_of_a_small_cell_agree():
+    """The same sequence on the periodic cell of 108 atoms, whose lists always
+    fit the bins that the one-workgroup preparation sizes from the density."""
+    _build_sequence(S.workload_inference(1)[1], (5.0, 5.0, 7.0, 7.0, 5.0))
 
 
 def test_batch_of_very_different_sizes(nctx):
