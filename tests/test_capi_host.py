@@ -246,6 +246,31 @@ def _check_lin_chunks(text):
     assert formed < consecutive
 
 
+@pytest.mark.parametrize("first,step,last", [(20000, 40, 24000), (5000, 100000, 2000000),
+                                             (160000, 32, 170000)])
+def test_pinned_buffers_grow_in_strides(tmp_path, first, step, last):
+    """Requests that grow a little from call to call pin memory a few times,
+    not on every call, and never hold more than half again what was asked for
+    (tests/pinned_growth.cpp; the smallest buffer has 4096 bytes)."""
+    import math
+    import os
+    import shutil
+    import subprocess
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc is not available")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path / "pinned_growth")
+    subprocess.run([hipcc, "-O1", "-std=c++17", "-w", "-I", os.path.join(root, "include"),
+                    "-I", os.path.join(root, "imr-mlp_amd", "csrc"),
+                    os.path.join(root, "tests", "pinned_growth.cpp"), "-o", exe], check=True)
+    out = subprocess.run([exe, str(first), str(step), str(last)], check=True, capture_output=True,
+                         text=True).stdout
+    allocations, held = (int(t) for t in out.split())
+    assert allocations <= 2 + math.ceil(math.log(last / first) / math.log(1.5))
+    assert held <= max(4096, 1.5 * last)
+
+
 @pytest.fixture(scope="module")
 def rule_dump(tmp_path_factory):
     """tests/rule_tables_dump.cpp built against the library's plan code."""
