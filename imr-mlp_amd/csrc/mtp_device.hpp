@@ -1002,8 +1002,11 @@ struct GlobalSteps {
 
 // The first cnt of four steps of a level.  A task's sum starts from zero and
 // is added to its target on the task's last entry (the sign bit of y): an
-// LDS add, so no lane waits for the target's old value, and the pieces of a
-// split task add to one target in program order.
+// LDS add, so no lane waits for the target's old value.  The pieces of a
+// split task add to one target step by step in program order; those that end
+// in the same step on different lanes (12 of the 52 reverse pieces of level
+// 10) meet in one instruction, whose lanes the LDS serves in a fixed order, so
+// the sums are repeatable bit for bit.
 __device__ __forceinline__ double step_factor(int y) { return (double)((int)((unsigned)y << 1) >> 18); }
 __device__ __forceinline__ void rule_group(const int2 (&e)[4], int cnt, unsigned base, double &acc,
                                            double &)

@@ -300,11 +300,15 @@ int mtpx_set_neighbors(mtpx_context *ctx, int n, const int *offsets, const int *
  * MTPGpuDirect::compute_batch (mtp_gpu_direct.h:892).  Outputs: total energy,
  * forces [n][3], stress [3][3] (extensive virial, eV, S_ab = -sum D_a r_b),
  * site energies [n].  Any output pointer may be NULL.  deterministic != 0
- * orders every reduction (no floating-point atomics): byte-repeatable.
+ * orders every reduction: byte-repeatable.  No sum then uses atomics on global
+ * memory; a wave adds to its own LDS work space in program order, and lanes of
+ * one instruction that meet in an address are served in the hardware's fixed
+ * order.
  * Lists built by mtpx_build_neighbors or mtpx_set_structures are always
  * assembled that way (each entry's reaction is gathered through the entry
- * of the other list that points back); lists from mtpx_set_neighbors use
- * floating-point atomics unless deterministic is set. */
+ * of the other list that points back); lists from mtpx_set_neighbors add the
+ * reactions with floating-point atomics on global memory unless deterministic
+ * is set. */
 int mtpx_efs(mtpx_context *ctx, int deterministic, double *energy, double *forces,
              double *stress, double *site_energies);
 /* PotMTP::getE (potentials/potential_mtp.cpp:2604-2621, over
@@ -377,7 +381,8 @@ int mtpx_set_add_efs(mtpx_context *ctx, int add_efs);
  * reuse_topology keeps the centres, offsets and neighbour indices of the
  * previous request (the counts must match) and refreshes types and
  * positions; when the kept centres change (a centre's species turns -1 or
- * back) the caller's offsets and neighbours are read and checked again.  deterministic orders every sum (no floating-point atomics).
+ * back) the caller's offsets and neighbours are read and checked again.
+ * deterministic orders every sum, as in mtpx_efs.
  * Independent of the resident lists of mtpx_build_neighbors /
  * mtpx_set_structures, which stay as they are. */
 typedef struct mtpx_site_request {
@@ -468,7 +473,8 @@ int mtpx_prepare_loss(mtpx_context *ctx, double metrics[7]);
  * dLdS_c : S_c), in the flat order [radial | species | moment].  dLdE
  * [nconf], dLdF [N][3], dLdS [nconf][9] (row-major 3x3); all three NULL use
  * the adjoints of mtpx_prepare_loss.  accumulate != 0 adds to gradient.
- * The sum is ordered: repeatable bit for bit. */
+ * The sum is ordered, as in mtpx_efs with deterministic: repeatable bit for
+ * bit. */
 int mtpx_accumulate_gradient(mtpx_context *ctx, const double *dLdE, const double *dLdF,
                              const double *dLdS, int accumulate, double *gradient);
 /* PotMTP::AddPenaltyGard, radial_mode 0 (potentials/potential_mtp.cpp:
