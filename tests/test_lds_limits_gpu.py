@@ -44,3 +44,20 @@ def test_gradient_of_many_species(ctx, template, Z, R):
     text = _model(template, Z, R)
     ctx.load_model_text(text)
     assert_loss_grad_close(ctx, loss_case(text, [_structure(Z, 2), _structure(Z, 3)], 932), 1e-9)
+
+
+@pytest.mark.parametrize("M", [3, 5])
+def test_force_table_longer_than_the_moments(ctx, M):
+    """M radial functions of degree 0 and no products: the force polynomials'
+    table (an even count per function) is longer than the moments, so the
+    staged adjoints lie behind the wave's blocks instead of over them."""
+    topo = dict(K=M, M=M, basic=[[mu, 0, 0, 0] for mu in range(M)], times=[], map=list(range(M)))
+    n = 4 * M * 8 + 2 + M
+    text = S.write_mtp(topo, 2, 8, 1.5, 5.0, 0.01, S.uniform(S.rng_for(933, M), n, -0.05, 0.05))
+    s = _structure(2, 4)
+    ref = oracle_case(text, s)
+    ctx.load_model_text(text)
+    upload_oracle_lists(ctx, ref["nb"])
+    assert_efs_close(ctx.efs(), ref, 1e-10)
+    assert_efs_close(ctx.efs(deterministic=True), ref, 1e-10)
+    assert_loss_grad_close(ctx, loss_case(text, [s, _structure(2, 5)], 934), 1e-9)
