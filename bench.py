@@ -553,8 +553,7 @@ def main():
         copy_probe(args.copy_probe)
         return
     if args.gpus != 1:
-        print("bench.py measures one GPU: this build has no multi-GPU path "
-              "(see DESIGN.md for how it would shard)", file=sys.stderr)
+        print("bench.py measures one GPU: the library has no multi-GPU path", file=sys.stderr)
         sys.exit(2)
 
     model_text, s = S.workload_inference(2)

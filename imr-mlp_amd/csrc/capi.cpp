@@ -467,9 +467,10 @@ int copy_out(mtpx_context *ctx, double *dst, const void *src, size_t count, bool
 // Up to this many doubles (2 MB) one launch packs the outputs into pinned
 // memory and the host copies them on, where a synchronous copy each cost a
 // round trip and the wait before them another (E/F/S call, 4,000 atoms 110 ->
-// 74 us, 32,000 atoms 310 -> 272).  Beyond it the host's part dominates
-// (256,000 atoms 4.91 against 4.99 ms), and pinning 8 MB for it costs the
-// first call 3.4 ms.
+// 74 us, 32,000 atoms 310 -> 272).  The limit is one on the pinned memory and
+// the time it takes to pin (8 MB cost the first call 3.4 ms), not a crossing:
+// packed, level-10 calls on lists from 66,000 to 180,000 atoms would still be
+// 4 to 6 % faster, 20 to 50 us.
 constexpr size_t kPackDoubles = 1 << 18;
 
 int finish_outputs(mtpx_context *ctx, std::initializer_list<OutPart> parts, const char *what)

@@ -27,8 +27,10 @@
 //   through the buffer, per-slot force sums and rules with predicated
 //   read-modify-writes 294 us and 6.0 ms; the matrix-core moments and Horner
 //   forces 246 us and 4.9 ms; rules in seven instructions a step 207 us and
-//   4.3 ms.  It is bound by the LDS pipe (rule gathers, transposes) and the
-//   vector unit in about equal parts.
+//   4.3 ms.  No unit is full: an atom of level 16 issues 530 LDS instructions
+//   (rule gathers, transposes, coefficients), by their costs about 45 % of the
+//   LDS pipe's cycles, the vector unit works in 40 % of its cycles, and the
+//   waves wait in 36 % of theirs.
 //   4. F_i += sum_j D_j, F_idx(j) -= D_j, S_ab -= D_ja r_jb.  Fast mode uses
 //      fp64 atomics for the neighbour reactions; deterministic mode stores D
 //      per pair for an ordered gather.  Each atom's energy and virial are
@@ -47,14 +49,12 @@ namespace mtpx {
 
 namespace {
 
-// Where the tables that not every model has LDS for lie.
-enum TablePlace {
-    kStepsLds,     // moment and step tables in LDS
-    kMomentsLds,   // moment tables in LDS, step tables in global memory
-    kTablesGlobal  // both in global memory (DevModel::mono_lds 0)
-};
+// Where the tables that not every model has LDS for lie (kTabs).
+constexpr int kStepsLds = 0;      // moment and step tables in LDS
+constexpr int kMomentsLds = 1;    // moment tables in LDS, step tables in global memory
+constexpr int kTablesGlobal = 2;  // both in global memory (DevModel::mono_lds 0)
 
-template <class P, TablePlace kTabs, int kMaxWaves, bool kHead>
+template <class P, int kTabs, int kMaxWaves, bool kHead>
 __global__ __launch_bounds__(kWave *kMaxWaves) void efs_kernel(DevModel m, DevNeighbors nb,
                                                                EfsOut out, int flags)
 {
@@ -427,7 +427,7 @@ void launch_variant(const DevModel &m, const DevNeighbors &nb, const EfsOut &out
     // MTP-M heads get kernels of their own: a linear model's kernel holds no
     // call of the out-of-line head (a call site costs registers and a stack)
     auto launch = [&](auto tabs) {
-        constexpr TablePlace kTabs = decltype(tabs)::value;
+        constexpr int kTabs = decltype(tabs)::value;
         if (m.head)
             hipLaunchKernelGGL((efs_kernel<P, kTabs, W, true>), grid, block, cfg.lds_bytes, s, m,
                                nb, out, det);
@@ -436,11 +436,11 @@ void launch_variant(const DevModel &m, const DevNeighbors &nb, const EfsOut &out
                                nb, out, det);
     };
     if (cfg.lds_tables)
-        launch(std::integral_constant<TablePlace, kStepsLds>{});
+        launch(std::integral_constant<int, kStepsLds>{});
     else if (m.mono_lds)
-        launch(std::integral_constant<TablePlace, kMomentsLds>{});
+        launch(std::integral_constant<int, kMomentsLds>{});
     else
-        launch(std::integral_constant<TablePlace, kTablesGlobal>{});
+        launch(std::integral_constant<int, kTablesGlobal>{});
 }
 
 int variant_max_waves(int v)

@@ -672,8 +672,8 @@ __device__ __forceinline__ int mono_entry(const DevModel &m, int ch, int g)
 }
 
 // One 8-byte LDS read; volatile keeps the compiler from pairing reads into
-// ds_read2_b64, which moves 16 bytes a lane in 8.3 cycles of the LDS pipe
-// (two ds_read_b64: 5.4).
+// ds_read2_b64: two operand columns (16 rows of kRedStride) take 16 cycles of
+// the LDS pipe paired and 4.8 as two ds_read_b64.
 __device__ __forceinline__ double lds_read(const double *p)
 {
     return *(const volatile __attribute__((address_space(3))) double *)p;
@@ -814,7 +814,7 @@ __device__ __forceinline__ unsigned lds_address(const double *p)
 }
 
 // Coefficients of one polynomial, streamed from LDS in blocks of eight
-// (16-byte broadcast reads: 4.5 cycles of the LDS pipe for two, against 8.3
+// (16-byte broadcast reads: 4.2 cycles of the LDS pipe for two, against 8.1
 // for the ds_read2_b64 the compiler forms from 8-byte reads), one block ahead
 // of its use.  The asm ties a block's reads to the running sums, so the
 // compiler cannot move all reads to the front and spill.
@@ -1069,8 +1069,8 @@ __device__ __forceinline__ void rule_group_dual(const int2 (&e)[4], int cnt, uns
 // past the level are read but not applied.  No task reads another task's
 // target within a level.
 //
-// The LDS pipe bounds the phase (two gathers of 6.6 cycles a step, against
-// 2.7 for a linear read) with the vector unit close behind: a step takes
+// The LDS pipe bounds the phase (two gathers of 6.5 cycles a step, against
+// 2.4 for a linear read) with the vector unit close behind: a step takes
 // seven instructions (two addresses, factor, product, sum, end test) where
 // separate shifts and masks, a predicated read-modify-write of the target
 // and partial sums combined afterwards took 17 and a wait per task.
