@@ -69,9 +69,15 @@ struct HBuf {
     {
         if (need <= bytes && p)
             return hipSuccess;
-        const size_t want = std::max({need, bytes + bytes / 2, size_t(4096)});
+        const size_t least = std::max(need, size_t(4096));
+        size_t want = std::max(least, bytes + bytes / 2);
         release();
         hipError_t e = hipHostMalloc(&p, want, 0);
+        if (e != hipSuccess && want > least) {  // no room for the reserve
+            (void)hipGetLastError();
+            want = least;
+            e = hipHostMalloc(&p, want, 0);
+        }
         if (e == hipSuccess)
             bytes = want;
         else

@@ -264,11 +264,16 @@ def test_pinned_buffers_grow_in_strides(tmp_path, first, step, last):
     subprocess.run([hipcc, "-O1", "-std=c++17", "-w", "-I", os.path.join(root, "include"),
                     "-I", os.path.join(root, "imr-mlp_amd", "csrc"),
                     os.path.join(root, "tests", "pinned_growth.cpp"), "-o", exe], check=True)
-    out = subprocess.run([exe, str(first), str(step), str(last)], check=True, capture_output=True,
-                         text=True).stdout
-    allocations, held = (int(t) for t in out.split())
+    def run(limit):
+        out = subprocess.run([exe, str(first), str(step), str(last), str(limit)], check=True,
+                             capture_output=True, text=True).stdout
+        return [int(t) for t in out.split()]
+
+    allocations, held = run(10 * last)
     assert allocations <= 2 + math.ceil(math.log(last / first) / math.log(1.5))
     assert held <= max(4096, 1.5 * last)
+    # with room for no more than the last request every request is still met
+    assert last - step < run(last)[1] <= last
 
 
 @pytest.fixture(scope="module")
